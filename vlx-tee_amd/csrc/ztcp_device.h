@@ -305,24 +305,150 @@ struct Sip {
     }
 };
 
-// Absorbs `total` consecutive 64-byte chunks delivered by fetch(uint4[4]),
-// with the loads of two chunks in flight ahead of the one being absorbed.
-template <class F>
-__device__ __forceinline__ void sip_stream64(Sip& s, uint32_t total, F&& fetch) {
-    uint4 x0[4], x1[4], x2[4];
-    if (total > 0u) fetch(x0);
-    if (total > 1u) fetch(x1);
-#pragma unroll 1
-    for (uint32_t c = 0; c < total; c += 3u) {
-        if (c + 2u < total) fetch(x2);
-        s.absorb64(x0);
-        if (c + 1u >= total) break;
-        if (c + 3u < total) fetch(x0);
-        s.absorb64(x1);
-        if (c + 2u >= total) break;
-        if (c + 4u < total) fetch(x1);
-        s.absorb64(x2);
+// ---------------------------------------------------------------------------
+// SipHash-2-4-128 of one page in two neighbouring lanes.
+// A SipRound is two halves, each of two independent add / rotate / xor steps:
+// lane A (even) takes the ones that update v1, lane B (odd) those of v3:
+//   half 1   A: v0 += v1, v1 = rotl(v1, 13) ^ v0    B: v2 += v3, v3 = rotl(v3, 16) ^ v2
+//   half 2   A: v2 += v1, v1 = rotl(v1, 17) ^ v2    B: v0 += v3, v3 = rotl(v3, 21) ^ v0
+// so v1 and v3 (y) stay in their lanes and v0 and v2 (t) change lanes at
+// every half.  The change costs nothing: the add reads the other lane's
+// halves through DPP (quad_perm [1, 0, 3, 2]).  Lane A's sum is the one that
+// SipRound rotates by 32 (v0 in half 1, v2 in half 2): two v_cndmask_b32
+// exchange its halves in lane A only.  A half is 8 instructions, a word 34
+// (two more for "v0 ^= m"; the next word's "v3 ^= m" is the third input of
+// the last xor), against 46 of one lane per page (Sip, above).  A lone wave
+// issues about one instruction per 4.1 clocks whatever it computes, so this
+// is the page's latency: 144 clocks per word against 191 (a probe of the
+// two chains alone, one wave per CU); two such waves on one SIMD take 210
+// clocks per word, on two SIMDs 144 each.
+// The message words must be zero in lane A.
+// Order inside a half: the carry is read two instructions after the add that
+// makes it, and a register is read through DPP at the earliest two
+// instructions after it was written, so no wait states are needed; the asm
+// starts with two, as the instruction before it may have written t.
+// ---------------------------------------------------------------------------
+#define ZTCP_SIP2_ADD(S)                                                                           \
+    "v_add_co_u32_dpp %[xl], vcc, %[tl], %[yl] quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"  \
+    "v_alignbit_b32 %[rl], %[yl], %[yh], %[" S "]\n\t"                                             \
+    "v_alignbit_b32 %[rh], %[yh], %[yl], %[" S "]\n\t"                                             \
+    "v_addc_co_u32_dpp %[xh], vcc, %[th], %[yh], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+#define ZTCP_SIP2_SEL                                    \
+    "v_cndmask_b32_e64 %[tl], %[xl], %[xh], %[am]\n\t"   \
+    "v_cndmask_b32_e64 %[th], %[xh], %[xl], %[am]\n\t"
+#define ZTCP_SIP2_HALF(S)                                                \
+    ZTCP_SIP2_ADD(S) "v_xor_b32_e32 %[yl], %[rl], %[xl]\n\t" ZTCP_SIP2_SEL \
+    "v_xor_b32_e32 %[yh], %[rh], %[xh]\n\t"
+#define ZTCP_SIP2_ROUND ZTCP_SIP2_HALF("s1") ZTCP_SIP2_HALF("s2")
+#define ZTCP_SIP2_INJ0(ML, MH)                \
+    "v_xor_b32_e32 %[tl], %[" ML "], %[tl]\n\t" \
+    "v_xor_b32_e32 %[th], %[" MH "], %[th]\n\t"
+// one word (whose "v3 ^= m" is applied), then the injection of the next one
+#define ZTCP_SIP2_WORD(ML, MH, NL, NH)                                                           \
+    ZTCP_SIP2_ROUND ZTCP_SIP2_HALF("s1") ZTCP_SIP2_ADD("s2")                                     \
+    "v_bitop3_b32 %[yl], %[rl], %[xl], %[" NL "] bitop3:0x96\n\t" ZTCP_SIP2_SEL                   \
+    ZTCP_SIP2_INJ0(ML, MH) "v_bitop3_b32 %[yh], %[rh], %[xh], %[" NH "] bitop3:0x96\n\t"
+// the last word: no next one
+#define ZTCP_SIP2_LAST(ML, MH) ZTCP_SIP2_ROUND ZTCP_SIP2_ROUND ZTCP_SIP2_INJ0(ML, MH)
+#define ZTCP_SIP2_STATE                                                                    \
+    [xl] "=&v"(xl), [xh] "=&v"(xh), [rl] "=&v"(rl), [rh] "=&v"(rh), [tl] "+v"(tl),         \
+        [th] "+v"(th), [yl] "+v"(yl), [yh] "+v"(yh)
+#define ZTCP_SIP2_CONST [s1] "v"(s1), [s2] "v"(s2), [am] "s"(0x5555555555555555ull)
+
+struct SipPair {
+    uint32_t tl, th;   // lane A: v2, lane B: v0
+    uint32_t yl, yh;   // lane A: v1, lane B: v3
+    uint32_t s1, s2;   // 32 - rotation of the lane's y in half 1 / half 2
+
+    __device__ __forceinline__ static bool lane_b() { return (threadIdx.x & 1u) != 0u; }
+
+    __device__ __forceinline__ void init(uint64_t mk0, uint64_t mk1) {
+        const bool b = lane_b();
+        const uint64_t t = b ? 0x736F6D6570736575ull ^ mk0 : 0x6C7967656E657261ull ^ mk0;
+        const uint64_t y = b ? 0x7465646279746573ull ^ mk1 : 0x646F72616E646F6Dull ^ mk1 ^ 0xEEull;
+        tl = (uint32_t)t; th = (uint32_t)(t >> 32);
+        yl = (uint32_t)y; yh = (uint32_t)(y >> 32);
+        s1 = b ? 32u - 16u : 32u - 13u;
+        s2 = b ? 32u - 21u : 32u - 17u;
     }
+    // Eight words, zero in lane A.
+    __device__ __forceinline__ void absorb64(const uint4 (&c)[4]) {
+        uint32_t xl, xh, rl, rh;
+        yl ^= c[0].x;
+        yh ^= c[0].y;
+        asm volatile("s_nop 1\n\t"
+                     ZTCP_SIP2_WORD("a0", "a1", "a2", "a3") ZTCP_SIP2_WORD("a2", "a3", "b0", "b1")
+                     ZTCP_SIP2_WORD("b0", "b1", "b2", "b3") ZTCP_SIP2_WORD("b2", "b3", "c0", "c1")
+                     ZTCP_SIP2_WORD("c0", "c1", "c2", "c3") ZTCP_SIP2_WORD("c2", "c3", "d0", "d1")
+                     ZTCP_SIP2_WORD("d0", "d1", "d2", "d3") ZTCP_SIP2_LAST("d2", "d3")
+                     : ZTCP_SIP2_STATE
+                     : ZTCP_SIP2_CONST, [a0] "v"(c[0].x), [a1] "v"(c[0].y), [a2] "v"(c[0].z), [a3] "v"(c[0].w),
+                       [b0] "v"(c[1].x), [b1] "v"(c[1].y), [b2] "v"(c[1].z), [b3] "v"(c[1].w),
+                       [c0] "v"(c[2].x), [c1] "v"(c[2].y), [c2] "v"(c[2].z), [c3] "v"(c[2].w),
+                       [d0] "v"(c[3].x), [d1] "v"(c[3].y), [d2] "v"(c[3].z), [d3] "v"(c[3].w)
+                     : "vcc");
+    }
+    // One word (any value in lane A: masked here).
+    __device__ __forceinline__ void absorb(uint64_t m) {
+        uint32_t xl, xh, rl, rh;
+        const uint32_t ml = lane_b() ? (uint32_t)m : 0u, mh = lane_b() ? (uint32_t)(m >> 32) : 0u;
+        yl ^= ml;
+        yh ^= mh;
+        asm volatile("s_nop 1\n\t" ZTCP_SIP2_LAST("m0", "m1")
+                     : ZTCP_SIP2_STATE
+                     : ZTCP_SIP2_CONST, [m0] "v"(ml), [m1] "v"(mh)
+                     : "vcc");
+    }
+    __device__ __forceinline__ void absorb(uint4 q) {  // two words
+        absorb((uint64_t)q.x | ((uint64_t)q.y << 32));
+        absorb((uint64_t)q.z | ((uint64_t)q.w << 32));
+    }
+    template <int N>
+    __device__ __forceinline__ void absorb_words(const uint64_t (&w)[N]) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) absorb(w[i]);
+    }
+    __device__ __forceinline__ void four_rounds() {
+        uint32_t xl, xh, rl, rh;
+        asm volatile("s_nop 1\n\t" ZTCP_SIP2_ROUND ZTCP_SIP2_ROUND ZTCP_SIP2_ROUND ZTCP_SIP2_ROUND
+                     : ZTCP_SIP2_STATE
+                     : ZTCP_SIP2_CONST
+                     : "vcc");
+    }
+    // v0 ^ v1 ^ v2 ^ v3, in both lanes.
+    __device__ __forceinline__ uint64_t fold() const {
+        const uint32_t a = tl ^ yl, b = th ^ yh;
+        const uint32_t oa = (uint32_t)__builtin_amdgcn_mov_dpp((int)a, 0xB1, 0xF, 0xF, true);  // quad_perm [1, 0, 3, 2]
+        const uint32_t ob = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, 0xB1, 0xF, 0xF, true);
+        return ((uint64_t)(b ^ ob) << 32) | (a ^ oa);
+    }
+    // As Sip::finish; both lanes get the tag.
+    __device__ __forceinline__ void finish(uint64_t last_word, uint64_t& lo, uint64_t& hi) {
+        absorb(last_word);
+        tl ^= lane_b() ? 0u : 0xEEu;  // v2 ^= 0xee
+        four_rounds();
+        lo = fold();
+        yl ^= lane_b() ? 0u : 0xDDu;  // v1 ^= 0xdd
+        four_rounds();
+        hi = fold();
+    }
+};
+
+// Absorbs `total` consecutive 64-byte chunks delivered by fetch(uint4[4]),
+// with the next chunk's loads in flight while one is absorbed.  One exit: the
+// compiler then keeps the chain's state in place over the loop.
+template <class S, class F>
+__device__ __forceinline__ void sip_stream64(S& s, uint32_t total, F&& fetch) {
+    uint4 x0[4], x1[4];
+    if (total > 0u) fetch(x0);
+#pragma unroll 1
+    for (uint32_t c = 2u; c <= total; c += 2u) {
+        fetch(x1);
+        s.absorb64(x0);
+        if (c < total) fetch(x0);
+        s.absorb64(x1);
+    }
+    if (total & 1u) s.absorb64(x0);
 }
 
 __device__ __forceinline__ uint64_t lo64(uint4 a) { return (uint64_t)a.x | ((uint64_t)a.y << 32); }

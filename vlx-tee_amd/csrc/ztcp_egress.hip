@@ -748,7 +748,7 @@ __global__ __launch_bounds__(64 * egress_waves<FAM>()) void egress_fused_kernel(
 // every page 192 at a time (load, quantize, keystream, XOR), write each to
 // the blob and to a copy of the page's whole payload in LDS, and stage its
 // scales; once every code row is made they encrypt the scale rows the same
-// way.  The MAC wave (0, one page per lane) absorbs the payload in order
+// way.  The MAC wave (0, two lanes per page) absorbs the payload in order
 // from LDS as the producers' passes complete, two rows of LDS reads ahead,
 // so it never reads global memory and waits only for the first pass.
 // ---------------------------------------------------------------------------
@@ -759,7 +759,9 @@ constexpr int kSmallTasks = 64 * (kSmallWaves - 1);  // tasks per producer pass
 constexpr int kSmFlagPass = 0;        // [3] passes completed by producer wave 1..3
 constexpr int kSmFlagScales = 3;      // producer waves done with the scale rows
 constexpr int kSmFlagExpired = 4;     // 1: a bounded wait of the workgroup expired
-constexpr int kSmFlags = 16;          // flag words
+constexpr int kSmZero = 16;           // [16] zero words: the message row of the MAC wave's A lanes
+constexpr int kSmFlags = 32;          // flag words, the zero row included
+static_assert(2 * kSmallMaxPpw <= 64, "two lanes of the MAC wave per page");
 constexpr int kSmPay = kSmFlags + kTimerLdsWords;  // the payload copy (64-byte aligned)
 
 // Payload block of the scale row of quantized unit g (staging order).
@@ -869,37 +871,43 @@ __device__ void small_produce(const EgressParams& p, int64_t page0, int ppw, int
     }
 }
 
-// The MAC wave: header, then payload rows 0..nrow-1 of page `lane` from LDS.
-// A code row is read once the pass holding its last page's task is complete
+// The MAC wave: header, then payload rows 0..nrow-1 of page `lane` / 2 from
+// LDS, two lanes per page (SipPair): the launch lasts one page's chain
+// (one page of 114,736 bytes: 1,214 us with one lane per page, 932 with two;
+// 256 pages of 12,336 bytes: 160 and 125 us).  A code row is read once the pass holding its last page's task is complete
 // in all three producer waves, a scale row once every wave has made its
-// scale rows.
+// scale rows.  A lanes read the zero row instead of a page's.
 template <int DT>
 __device__ void small_mac(const EgressParams& p, int64_t page0, int ppw, int32_t nrow, uint32_t* lds, uint64_t t0) {
-    const int lane = threadIdx.x & 63;
-    const bool active = lane < ppw;
-    const EgressPage pg = egress_page(p, page0 + (active ? lane : 0));
+    const int lane = threadIdx.x & 63, pl = lane >> 1;
+    const bool active = pl < ppw;
+    const bool writer = active && !SipPair::lane_b();  // stores the page's header and tag
+    const EgressPage pg = egress_page(p, page0 + (active ? pl : 0));
     uint32_t* flags = lds;
-    const uint32_t* mine = lds + kSmPay + (size_t)(active ? lane : 0) * nrow * kSmRowWords;
-    if (active) {  // header (cpp:1129-1140)
+    const uint32_t* mine =
+        SipPair::lane_b() ? lds + kSmPay + (size_t)(active ? pl : 0) * nrow * kSmRowWords : lds + kSmZero;
+    const int32_t step = SipPair::lane_b() ? kSmRowWords : 0;
+    if (writer) {  // header (cpp:1129-1140)
         stg16(pg.blob, 0, make_uint4((uint32_t)p.hdr0, (uint32_t)(p.hdr0 >> 32), (uint32_t)pg.hdr1,
                                      (uint32_t)(pg.hdr1 >> 32)));
         stg16(pg.blob, 1, make_uint4((uint32_t)pg.token, (uint32_t)(pg.token >> 32), (uint32_t)pg.seq,
                                      (uint32_t)(pg.seq >> 32)));
     }
-    Sip s;
+    SipPair s;
     s.init(p.mk0, p.mk1);
     const uint64_t hdr[4] = {p.hdr0, pg.hdr1, pg.token, pg.seq};
     s.absorb_words<4>(hdr);
     const Waiter wt = make_waiter(p.sink, flags + kSmFlagExpired, lds + kSmFlags, t0);
     const int32_t ncode = total_code_rows(p.lay);
-    int32_t r = 0;         // payload rows fetched
+    [[maybe_unused]] int32_t r = 0;  // payload rows fetched (phase timers)
     int32_t c = 0;         // code rows absorbed
     int32_t ready = 0;     // code rows complete for every page
     bool scales = false;   // scale rows complete
     auto fetch = [&](uint4 (&x)[4]) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const uint4*>(mine + r * kSmRowWords + 4 * q);
-        ++r;
+        for (int q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const uint4*>(mine + 4 * q);
+        mine += step;
+        if constexpr (kPhaseTimers) ++r;
     };
     __builtin_amdgcn_s_waitcnt(0);
     if constexpr (kPhaseTimers) tm_add(wt.tm, kTmMacRowsBegin, phase_clock() - t0);
@@ -944,7 +952,7 @@ __device__ void small_mac(const EgressParams& p, int64_t page0, int ppw, int32_t
     if constexpr (kPhaseTimers) tm_add(wt.tm, kTmMacRowsEnd, phase_clock() - t0);
     uint64_t lo, hi;
     s.finish((uint64_t)((kHeader + p.payload) & 0xFFu) << 56, lo, hi);
-    if (active)
+    if (writer)
         stg16(pg.blob + kHeader + p.payload, 0,
               make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)));
     if constexpr (kPhaseTimers) tm_add(wt.tm, kTmMacEnd, phase_clock() - t0);
@@ -972,8 +980,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void egress_small_kernel(EgressPa
     __syncthreads();
     tm_flush(lds + kSmFlags, p.timers, t0, rt0);
     if (__hip_atomic_load(lds + kSmFlagExpired, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0u &&
-        (int)threadIdx.x < ppw)
-        stg16(egress_page(p, page0 + threadIdx.x).blob, 0, make_uint4(0u, 0u, 0u, 0u));
+        (int)threadIdx.x < 2 * ppw && !SipPair::lane_b())
+        stg16(egress_page(p, page0 + (threadIdx.x >> 1)).blob, 0, make_uint4(0u, 0u, 0u, 0u));
 }
 
 }  // namespace

@@ -953,7 +953,7 @@ __global__ __launch_bounds__(kIngressThreads) void ingress_fused_kernel(IngressP
 // pipeline idle and the verify wave's chain waits for rows decoded one page
 // at a time.  Here three loader waves copy every payload row of every page
 // into LDS, lane = (row, page), 192 rows per pass, publishing their passes;
-// the verify wave (one page per lane) absorbs the rows from LDS as the passes
+// the verify wave (two lanes per page) absorbs the rows from LDS as the passes
 // complete, so its chain runs at the lone rate.  After their load passes the
 // same waves decode the pages with the workgroup's layout, lane = (unit,
 // page), with the unit decoder the row-pipeline kernel uses for pages of
@@ -970,19 +970,24 @@ constexpr int kSiFlagPass = 0;                 // [3] load passes completed by l
 constexpr int kSiFlagExpired = 4;              // 1: a bounded wait of the workgroup expired
 constexpr int kSiFlagStatus = 8;               // [4] verdicts
 constexpr int kSiFlagNaN = 12;                 // [4] 1: the page has an inf / NaN scale
-constexpr int kSiFlags = 16;
+constexpr int kSiZero = 16;                    // [16] zero words: the message row of the verify wave's A lanes
+constexpr int kSiFlags = 32;
+static_assert(2 * kSiMaxPpw <= 64, "two lanes of the verify wave per page");
 constexpr int kSiTimers = kSiFlags;                                     // phase timers (timer builds)
 constexpr int kSiHeaders = kSiTimers + kTimerLdsWords;                  // [4] 32-byte headers
 constexpr int kSiLayouts = kSiHeaders + kSiMaxPpw * 8;                  // [kNumLayouts] Layout
 constexpr int kSiPay = (kSiLayouts + kNumLayouts * kLayoutWords + 15) & ~15;  // payload copies, 64-byte aligned
 static_assert(kSiHeaders % 4 == 0, "header table must be 16-byte aligned");
 
-// Verdict of page `lane` (< ppw) from its payload copy in LDS.
+// Verdict of page `lane` / 2 from its payload copy in LDS, two lanes per page
+// (SipPair; both lanes return it; four pages of 114,736 bytes: 1,257 us with
+// one lane per page, 980 with two; 256 pages of 12,336 bytes: 160 and 128
+// us).  h0, h1: the header of that page.
 __device__ __forceinline__ int32_t small_verify(const IngressParams& p, int64_t page0, int ppw, int32_t nrow,
                                                 uint32_t* lds, const uint4 h0, const uint4 h1, uint64_t t0) {
-    const int lane = threadIdx.x & 63;
-    const bool active = lane < ppw;
-    const int64_t page = page0 + (active ? lane : 0);
+    const int pl = (int)(threadIdx.x & 63) >> 1;
+    const bool active = pl < ppw;
+    const int64_t page = page0 + (active ? pl : 0);
     const uint8_t* pay = ingress_blob(p, page) + kHeader;
     const uint32_t tail0 = (uint32_t)nrow * 64u;
     const int ntail = (int)((p.payload - tail0) / 16u);  // 0..3 chunks of 16 bytes
@@ -990,18 +995,19 @@ __device__ __forceinline__ int32_t small_verify(const IngressParams& p, int64_t 
 #pragma unroll
     for (int i = 0; i < 3; ++i) tl[i] = ldg16(pay + min(tail0 + 16u * (uint32_t)i, p.payload), 0);
     const uint4 tag = ldg16(pay + p.payload, 0);
-    Sip s;
+    SipPair s;
     s.init(p.mk0, p.mk1);
     const uint64_t hdr[4] = {lo64(h0), hi64(h0), lo64(h1), hi64(h1)};
     s.absorb_words<4>(hdr);
     uint32_t* flags = lds;
-    const uint32_t* mine = lds + kSiPay + (size_t)(active ? lane : 0) * nrow * kSiRowWords;
+    const uint32_t* mine =
+        SipPair::lane_b() ? lds + kSiPay + (size_t)(active ? pl : 0) * nrow * kSiRowWords : lds + kSiZero;
+    const int32_t step = SipPair::lane_b() ? kSiRowWords : 0;
     const Waiter wt = make_waiter(p.sink, flags + kSiFlagExpired, lds + kSiTimers, t0);
-    int32_t r = 0;  // rows fetched
     auto fetch = [&](uint4 (&x)[4]) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const uint4*>(mine + r * kSiRowWords + 4 * q);
-        ++r;
+        for (int q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const uint4*>(mine + 4 * q);
+        mine += step;
     };
     __builtin_amdgcn_s_waitcnt(0);
     if constexpr (kPhaseTimers) tm_add(wt.tm, kTmMacRowsBegin, phase_clock() - t0);
@@ -1117,8 +1123,9 @@ void ingress_small_kernel(IngressParams p) {
     const int li_wg = any_valid ? __builtin_amdgcn_readlane(li, (int)__builtin_ctzll(any_valid)) : -1;
     if (wave == 0) {
         __builtin_amdgcn_s_setprio(3);
-        const int32_t v = small_verify(p, page0, ppw, nrow, lds, h0, h1, t0);
-        if (active) flags[kSiFlagStatus + lane] = (uint32_t)v;
+        const int pv = (lane >> 1) < ppw ? lane >> 1 : 0;
+        const int32_t v = small_verify(p, page0, ppw, nrow, lds, hdrs[2 * pv], hdrs[2 * pv + 1], t0);
+        if ((lane >> 1) < ppw && !SipPair::lane_b()) flags[kSiFlagStatus + (lane >> 1)] = (uint32_t)v;
     } else {
         small_load_decode<DT>(p, page0, ppw, nrow, lds, li_wg, t0);
     }
