@@ -1,11 +1,13 @@
-"""The SipHash lanes of a workgroup, at the edges of every split.
+"""The lanes and page groups of a workgroup, at the edges of every split.
 
-The small-batch kernels hash each page in two lanes of the MAC wave; the
-page counts below put one to four pages in a workgroup, with the last
-workgroup full and partial.  Blobs and decoded pages must equal the oracle's,
-and a page with one flipped bit (the first, the last and one in the middle)
-must be the only one rejected: a word that reaches the wrong lane, or a lane
-left out, changes some page's tag.
+The small-batch kernels (one to four pages per workgroup) and the row-pipeline
+kernels of up to 32 pages hash each page in two lanes of the MAC wave, larger
+workgroups in one; the row pipeline makes its rows for groups of 16 pages.
+The page counts below put each of these in a workgroup, on both sides of every
+limit, with the last workgroup full and partial.  Blobs and decoded pages
+must equal the oracle's, and a page with one flipped bit (the first, the last
+and one in the middle) must be the only one rejected: a word that reaches the
+wrong lane, or a lane or page group left out, changes some page's tag.
 """
 import numpy as np
 import pytest
@@ -18,7 +20,8 @@ KEYS = dict(k0=0x452821E638D01377, k1=0xBE5466CF34E90C6C, mk0=0xC0AC29B7C97C50DD
 TEN, MOD, LAYER, HG, BASE = 0x5EED5EED, 0x0DDBA11, 3, 1, 9
 T, H, D, R = 2, 16, 32, 16
 # 256 CUs: one page per workgroup up to 256 pages, then two, three, four
-COUNTS = [1, 2, 255, 257, 512, 513, 769, 1023, 1024]
+# (small-batch kernels); 5, 16, 17, 32, 33, 48, 49 and 64 pages (row pipeline)
+COUNTS = [1, 2, 255, 257, 512, 513, 769, 1023, 1024, 1025, 4096, 4099, 8191, 8193, 12288, 12300, 16384, 16385]
 
 
 @pytest.mark.parametrize("preset,mode", [(2, 1), (1, 2)])

@@ -5,30 +5,35 @@
 // fused_encode_cold_pages_peak_into_cpu (cpp:1904-2004).
 //
 // Work decomposition (one workgroup = up to 64 pages, 16 waves, four per
-// SIMD, or 12 for the int4-per-32 and asym8 kinds; lane = page in every
-// wave):
+// SIMD, or 12 for the int4-per-32 and asym8 kinds):
 //   * A "row" is one 64-byte keystream block position of the payload, for all
 //     pages of the workgroup.  Every payload block is exactly one row: a code
 //     row (4 int8 / e4m3 / int4-per-32 groups, 8 int4 groups, 2 raw groups
 //     or 1 asym8 group) or a scale row (the 64 parameter bytes of one unit).
 //   * Eleven producer waves (on SIMDs 1-3; eight in the 12-wave kernels)
-//     take code rows in order from an LDS counter.  A code
-//     row quantizes its groups (loaded a row ahead; the int4 rows four lanes
+//     take tasks in order from an LDS counter: four consecutive code rows of
+//     a unit for one group of 16 pages, lane = (row, page).  A task
+//     quantizes its groups (loaded a task ahead; the int4 rows four lanes
 //     per page, transposed between the wave's 16-lane rows afterwards),
 //     stages the scales in LDS, computes the keystream, XORs, and writes the
 //     ciphertext into a ring of row slots in LDS at its place in payload
-//     order.
-//   * A storer wave (wave 1, SIMD 1) stores every code row from the ring to
-//     the blobs, in payload order, transposed (four lanes per page, 64
-//     contiguous bytes per page per store).  After a unit's last code row
-//     it also makes the unit's scale row: it encrypts the staged scales in
-//     their slot, and stores them the same way, freeing the slot, together
-//     with the next scale rows of the section, eight at a time.  Producers issue
-//     no stores: a wave's wait for its own loads also waits for every store
-//     it issued before them, which exposed the int4 rows' second loads; and
-//     the MAC wave's SIMD is kept free of stores.
-//   * Wave 0 runs SipHash for one page per lane, at raised priority on SIMD
-//     0.  It absorbs the header, then the payload rows in order from the
+//     order.  The task that stages the last scales of four units (a scale
+//     group) encrypts them in their staging slots.
+//     Four rows of 16 pages instead of one row of 64: a workgroup of a few
+//     pages leaves no lane idle (4,087 MLA pages, 16 a workgroup: 397 us a
+//     row at a time, 256 four rows at a time with the two-lane MAC wave;
+//     2,900 pages of K8V4_ASYM_G64, 12 a workgroup: 404 and 268), and
+//     the bytes of a page are asked for 512 to 1,024 at a time.
+//   * A storer wave (wave 1, SIMD 1) stores the code rows from the ring to
+//     the blobs, in payload order, four at a time (sixteen lanes per page,
+//     256 contiguous bytes per page), and the encrypted scale rows, four
+//     units at a time, from their staging slots, which it frees.  Producers
+//     issue no stores: a wave's wait for its own loads also waits for every
+//     store it issued before them, which exposed the int4 rows' second
+//     loads; and the MAC wave's SIMD is kept free of stores.
+//   * Wave 0 runs SipHash at raised priority on SIMD 0, two lanes per page
+//     in a workgroup of up to 32 pages, one lane per page in a larger one.  It
+//     absorbs the header, then the payload rows in order from the
 //     ring, so it never reads global memory.  Scale rows reach the ring
 //     through a feeder wave (wave 4, also on SIMD 0): a scale row is stored
 //     long before the MAC wave reaches it (after all of its section's code
@@ -36,11 +41,13 @@
 //     have completed.  Waves 8 and 12 exit at once: producers there slow the
 //     MAC chain down more than they add.
 //   * Hand-offs are monotonic LDS counters with workgroup-scope
-//     release/acquire: ring_flag[slot] = payload row index + 1 when written,
-//     mac_used = rows absorbed and stored = rows stored (a slot is free once
-//     both have passed it), stage_flag[slot] = unit + 1 when a scale row
-//     has read its staging slot, scale_flag[slot] = unit + 1 once the scale
-//     row's stores have completed.  Every wait is bounded; an
+//     release/acquire: ring_flag[page group][slot] = payload row index + 1
+//     when written, mac_used = rows absorbed and stored = rows stored (a slot
+//     is free once both have passed it), count[page group][slot] = tasks of a
+//     scale group that staged their scales, enc_flag[page group][slot] = unit
+//     + 1 once the group is encrypted, stage_flag[slot] = unit + 1 when the
+//     storer has read its staging slot, scale_flag[slot] = unit + 1 once the
+//     scale row's stores have completed.  Every wait is bounded; an
 //     expired wait sets a sticky diagnostic bit and the kernel still ends.
 //     Waits only point backwards in row order, so progress never depends on
 //     a later row.
@@ -64,23 +71,30 @@ template <int FAM>
 constexpr int egress_waves() { return FAM <= 1 ? 16 : 12; }  // family 2's quantizers need 168 VGPRs
 constexpr int kRing = 24;             // payload rows between their makers and the MAC wave
 constexpr int kStage = 13;            // units whose scales are staged at once
-constexpr int kScaleGroup = 8;        // scale rows stored together (at most kScaleGroup - 1 held)
+constexpr int kScaleGroup = 4;        // units whose scale rows are encrypted and stored together
 constexpr int kLdsStage = kRing * kRowWords;
 constexpr int kScaleSlots = 64;       // scale rows the feeder wave may still be waiting for
 constexpr int kLdsFlags = kLdsStage + kStage * kRowWords;
-constexpr int kFlagRing = 0;                          // [kRing] MAC row index + 1
-constexpr int kFlagStage = kFlagRing + kRing;         // [kStage] unit + 1: staging slot free
+constexpr int kFlagRing = 0;                          // [4][kRing] per page group: payload row index + 1
+constexpr int kFlagEnc = kFlagRing + 4 * kRing;       // [4][kStage] unit + 1: its scale group is encrypted
+constexpr int kFlagCount = kFlagEnc + 4 * kStage;     // [4][kStage] tasks of a scale group that staged their scales
+constexpr int kFlagStage = kFlagCount + 4 * kStage;   // [kStage] unit + 1: staging slot free
 constexpr int kFlagScale = kFlagStage + kStage;       // [kScaleSlots] unit + 1: scale row stored
 constexpr int kFlagMacUsed = kFlagScale + kScaleSlots;  // rows absorbed by the MAC wave
 constexpr int kFlagStored = kFlagMacUsed + 1;         // rows passed by the storer wave
-constexpr int kFlagTask = kFlagStored + 1;            // next code row to hand out
+constexpr int kFlagTask = kFlagStored + 1;            // next task to hand out
 constexpr int kFlagExpired = kFlagTask + 1;           // 1: a bounded wait of the workgroup expired
 constexpr int kNumFlags = (kFlagExpired + 2) & ~1;    // even: the blob table after it is 8-byte aligned
-constexpr int kLdsBlobs = kLdsFlags + kNumFlags;      // 64 blob pointers (8-byte aligned)
-constexpr int kLdsTimers = kLdsBlobs + 2 * 64;        // phase-timer counters (timer builds only)
-constexpr int kLdsWords = kLdsTimers + kTimerLdsWords;
+constexpr int kLdsBlobs = kLdsFlags + kNumFlags;      // [64] blob pointers (8-byte aligned)
+constexpr int kLdsHot = (kLdsBlobs + 2 * 64 + 3) & ~3;  // [64] K and V pointers
+constexpr int kLdsNonce = kLdsHot + 4 * 64;           // [64] nonce (3 words, a pad) and its ChaChaNonceCache
+constexpr int kNonceWords = 16;
+constexpr int kLdsTimers = kLdsNonce + kNonceWords * 64;  // phase-timer counters (timer builds only)
+constexpr int kLdsZero = (kLdsTimers + kTimerLdsWords + 3) & ~3;  // a zero quad: the message of the MAC wave's A lanes
+constexpr int kLdsWords = kLdsZero + 4;
 static_assert(kLdsWords * 4 <= 160 * 1024, "LDS budget of one CU");
-static_assert(kScaleGroup <= kStage, "held scale rows must leave a staging slot for the unit that completes their group");
+static_assert(kRing % 4 == 0 && kRing >= 2 * kTaskRows, "a group's ring flags are aligned; two tasks fit the ring");
+static_assert(kStage >= 3 * kScaleGroup, "the storer keeps one scale group while the producers stage the next two");
 static_assert(kLdsBlobs % 2 == 0 && kLdsTimers % 2 == 0, "blob table and timers must be 8-byte aligned");
 
 __device__ __forceinline__ int32_t total_rows(const Layout& lay) {
@@ -118,20 +132,71 @@ __device__ __forceinline__ void load_half(const EgressParams& p, const EgressPag
     }
 }
 
-// Half h of a code row with four lanes per page: load i (0..7) gives lane
-// 16 r + c quad 4 (i / 4) + r of page 16 (i % 4) + c, 64 contiguous bytes per
-// page per load; row_untranspose then gives every lane its own page's eight
-// quads.  Needs the half's four chunks contiguous (tq_row).
-__device__ __forceinline__ void load_half_t(const EgressParams& p, const EgressPage& pg, const Row& row, int h,
-                                            uint32_t (&w)[4][8]) {
-    const int ng = chunks_per_row(row.s.kind);
-    const GroupCursor cur = group_cursor(row.u * row.s.nblk * ng + row.j * ng + 4 * h, row.s.gpv, row.s.col, p.head_dim);
-    const uint32_t r16 = (threadIdx.x >> 4 & 3u) * 16u;
-    const uint8_t* pm[4];
-    column_ptrs(row.s.src ? pg.v : pg.k, pm);
+// ---------------------------------------------------------------------------
+// Tasks of the row pipeline: kTaskRows code rows of kTaskPages pages.
+// `row` is the task's first row, src the hot buffer (K or V) of this lane's
+// page; lane 16 r + c has row r.
+// ---------------------------------------------------------------------------
+
+// Hot loads of half h (chunks [4 h, 4 h + 4)) of this lane's own row.
+__device__ __forceinline__ void load_task_half(const EgressParams& p, const uint8_t* src, const Row& row, int h,
+                                               uint32_t (&w)[4][8]) {
+    const int nch = chunks_per_row(row.s.kind);
+    const uint32_t gpv = (uint32_t)row.s.gpv;
+    const uint32_t G0 = (uint32_t)((row.u * row.s.nblk + row.j) * nch + 4 * h);  // the first row's chunk
+    const uint32_t vec0 = G0 / gpv;
+    // this lane's chunk, counted from the start of the vector of the first
+    // row's: at most gpv - 1 + 3 * 8, so past 28 chunks per vector it wraps
+    // at most once, and below the reciprocal is exact
+    uint32_t g = G0 - vec0 * gpv + (threadIdx.x >> 4 & 3u) * (uint32_t)nch;
+    const uint32_t over = gpv > 28u ? (g >= gpv ? 1u : 0u) : (g * (65536u / gpv + 1u)) >> 16;
+    g -= over * gpv;
+    uint32_t off = (vec0 + over) * (uint32_t)p.head_dim * 2u + (uint32_t)row.s.col * 2u + g * 32u;
+    if ((gpv & 3u) == 0u) {  // four contiguous chunks
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (i < nch) load_group(src + off + 32 * i, w[i]);
+        return;
+    }
+    const uint32_t skip = (uint32_t)(p.head_dim - row.s.gpv * 16) * 2u;
+    GroupCursor cur{off, (int32_t)g};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (i < nch) {
+            load_group(src + cur.off, w[i]);
+            cur.step(row.s.gpv, skip);
+        }
+    }
+}
+
+// The same with four lanes per page: load i (0..7) gives lane 16 r + c quad
+// 4 (i / 4) + r of row i % 4 of page c, 64 contiguous bytes of 16 pages;
+// row_untranspose then gives every lane its own row's eight quads.  Needs the
+// half's four chunks contiguous (tq_row).
+__device__ __forceinline__ void load_task_half_t(const EgressParams& p, const uint8_t* src, const Row& row, int h,
+                                                 uint32_t (&w)[4][8]) {
+    const int32_t per_row = chunks_per_row(row.s.kind) / 4;  // pieces of four chunks
+    const int32_t gp4 = row.s.gpv / 4;                       // pieces per vector
+    const int32_t piece = (row.u * row.s.nblk + row.j) * per_row + h;
+    int32_t vec = piece / gp4, gi = piece - vec * gp4;
+    const uint8_t* base = src + (uint32_t)row.s.col * 2u + (threadIdx.x >> 4 & 3u) * 16u;
+    uint32_t off[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        off[i] = (uint32_t)vec * (uint32_t)p.head_dim * 2u + (uint32_t)gi * 128u;
+        gi += per_row;  // 1 or 2
+        if (gi >= gp4) {
+            gi -= gp4;
+            ++vec;
+        }
+        if (gi >= gp4) {  // one piece per vector
+            gi -= gp4;
+            ++vec;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const uint4 v = ldg16(pm[i & 3] + cur.off + (uint32_t)(i >> 2) * 64u + r16, 0);
+        const uint4 v = ldg16(base + off[i & 3], (i >> 2) * 4);
         w[i >> 1][(i & 1) * 4 + 0] = v.x;
         w[i >> 1][(i & 1) * 4 + 1] = v.y;
         w[i >> 1][(i & 1) * 4 + 2] = v.z;
@@ -145,43 +210,25 @@ __device__ __forceinline__ void row_untranspose(uint32_t (&w)[4][8]) {
 
 struct ProducerCtx {
     const EgressParams* p;
-    EgressPage pg;
-    uint32_t n0, n1, n2;
-    ChaChaNonceCache nc;
     uint32_t* lds;
     int lane;
-    // Transposed row stores: store k of a row writes quad (lane & 3) of page
-    // 16 k + (lane >> 2).  Past the last page of a partial workgroup the lane
-    // writes page 0's quad instead, the same bytes page 0's own lane writes,
-    // so every store is unconditional (a store under a branch makes the
-    // compiler wait for all outstanding stores before the next row's loads).
-    uint8_t* sb[4];   // blob of the page stored by store k
-    uint32_t sq[4];   // byte offset of that page's quad inside a row slot
+    int ng;       // page groups of the workgroup
     Waiter wt;
-
-    __device__ __forceinline__ void init_stores(int ppw) {
-        const uint64_t* blobs = reinterpret_cast<const uint64_t*>(lds + kLdsBlobs);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int pr = 16 * k + (lane >> 2);
-            const int pe = pr < ppw ? pr : 0;
-            sb[k] = reinterpret_cast<uint8_t*>(blobs[pe]);
-            sq[k] = quad_word(pe, lane & 3) * 4u;
-        }
+    // Hot buffer (K or V) of this lane's page in page group `group`.
+    __device__ __forceinline__ const uint8_t* hot(int group, int src) const {
+        const uint64_t* t = reinterpret_cast<const uint64_t*>(lds + kLdsHot) + 2 * (group * kTaskPages + (lane & 15));
+        return reinterpret_cast<const uint8_t*>(t[src]);
     }
 };
 
-// Stores one row slot to the blobs, each store instruction writing 64
-// contiguous bytes of 16 pages.  The four quads are read first, so the row
-// costs one LDS round trip.  The stores are issued after the next row's
-// loads, so the wave's wait for those loads does not include them (vector
-// memory operations complete in issue order).
-__device__ __forceinline__ void store_row(const uint32_t* slot, const ProducerCtx& c, uint32_t blob_off) {
-    uint4 x[4];
+// One ChaCha20 block of page `pg` of the workgroup, counter 1 + block, nonce
+// and first column round from the LDS table.
+__device__ __forceinline__ void nonce_cache(const uint32_t* tab, ChaChaNonceCache& nc) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) x[k] = lds_quad_at(slot, c.sq[k]);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) stg16(c.sb[k] + blob_off, c.lane & 3, x[k]);
+    for (int q = 0; q < 3; ++q) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(tab + 4 + 4 * q);
+        nc.c[4 * q] = v.x; nc.c[4 * q + 1] = v.y; nc.c[4 * q + 2] = v.z; nc.c[4 * q + 3] = v.w;
+    }
 }
 
 // Quantizes groups w[0..3] (int8: 4 code words each, int4: 2) into pt[] and
@@ -223,30 +270,30 @@ __device__ __forceinline__ uint32_t quant_half_int4g32(const uint32_t (&w)[4][8]
     return sa | (sbb << 16);
 }
 
-// The scale row of unit g (payload block `block`), made by the storer wave
-// once it has stored the unit's last code row: every code row of the unit
-// stages its scales before it releases its ring row, so all of them are in
-// the staging slot by then.  Encrypts the staged scales in place, stores the
-// block transposed and frees the staging slot; that the stores have
-// completed is published later (publish_scales).
-__device__ __forceinline__ void encrypt_scale_row(const ProducerCtx& c, int32_t g, uint32_t block) {
+// Encrypts the staged scale rows of a scale group (units u0 .. u0 + n - 1 of
+// their section, n <= kScaleGroup, the first one quantized unit g0) of one
+// page group in their staging slots: lane 16 r + c takes unit u0 + r of page
+// c (lanes past the last unit do the last one's again and write the same).
+// Run by the producer whose task staged the last scales of the group.
+__device__ __forceinline__ void encrypt_scales(const ProducerCtx& c, int group, int32_t n, int32_t g0, uint32_t block0) {
     const EgressParams& p = *c.p;
+    const int pg = group * kTaskPages + (c.lane & 15);
+    const int32_t i = min(c.lane >> 4, n - 1);
+    const uint32_t* tab = c.lds + kLdsNonce + pg * kNonceWords;
+    ChaChaNonceCache nc;
+    nonce_cache(tab, nc);
+    const u32x4 nn = *reinterpret_cast<const u32x4*>(tab);
     uint32_t ks[16];
-    chacha_block_cached(p.key, c.nc, 1u + block, c.n0, c.n1, c.n2, ks);
-    uint32_t* stage = c.lds + kLdsStage + (g % kStage) * kRowWords;
+    chacha_block_cached(p.key, nc, 1u + block0 + (uint32_t)i, nn.x, nn.y, nn.z, ks);
+    uint32_t* stage = c.lds + kLdsStage + ((g0 + i) % kStage) * kRowWords;
+    uint4 sw[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const uint4 s = lds_quad(stage, c.lane, q);
-        lds_put_quad(stage, c.lane, q,
-                     make_uint4(s.x ^ ks[4 * q], s.y ^ ks[4 * q + 1], s.z ^ ks[4 * q + 2], s.w ^ ks[4 * q + 3]));
-    }
-}
-// Stores unit g's encrypted scale row (payload block `block`) from its
-// staging slot and frees the slot.
-__device__ __forceinline__ void store_scale_row(const ProducerCtx& c, int32_t g, uint32_t block) {
-    uint32_t* flags = c.lds + kLdsFlags;
-    store_row(c.lds + kLdsStage + (g % kStage) * kRowWords, c, (uint32_t)kHeader + 64u * block);
-    publish(&flags[kFlagStage + g % kStage], (uint32_t)g + 1u);  // the release follows the slot reads
+    for (int q = 0; q < 4; ++q) sw[q] = lds_quad(stage, pg, q);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        lds_put_quad(stage, pg, q,
+                     make_uint4(sw[q].x ^ ks[4 * q], sw[q].y ^ ks[4 * q + 1], sw[q].z ^ ks[4 * q + 2],
+                                sw[q].w ^ ks[4 * q + 3]));
 }
 
 // Publishes that scale rows [from, to) are in the blobs, for the feeder.
@@ -288,12 +335,7 @@ __device__ __forceinline__ void quant_first(int32_t kind, const uint32_t (&w)[4]
     }
 }
 
-// The first half of a row's chunks: loads them, and once they have arrived
-// quantizes them and issues the loads of the second half (rows of eight
-// chunks), which then arrive during the row's first double rounds.  Run at
-// the end of the previous row, whose last rounds cover the first half's
-// loads.
-// Whether a row's hot loads are made four lanes per page: the rows that read
+// Whether a task's hot loads are made four lanes per page: the rows that read
 // 256 hot bytes per page (int4, int4 per 32) when each half is four
 // contiguous chunks (groups per vector a multiple of 4).  The rows of 128
 // hot bytes per page (int8, e4m3, asym8) measured slower that way.
@@ -303,41 +345,53 @@ __device__ __forceinline__ bool tq_row(const Row& row) {
            ((FAM == 0 && row.s.kind == kSecInt4) || (FAM == 2 && row.s.kind == kSecInt4G32));
 }
 template <int FAM>
-__device__ __forceinline__ void load_half_any(const EgressParams& p, const EgressPage& pg, const Row& row, int h,
+__device__ __forceinline__ void load_half_any(const EgressParams& p, const uint8_t* src, const Row& row, int h,
                                               uint32_t (&w)[4][8]) {
-    if (tq_row<FAM>(row)) load_half_t(p, pg, row, h, w);
-    else load_half(p, pg, row, h, w);
+    if (tq_row<FAM>(row)) load_task_half_t(p, src, row, h, w);
+    else load_task_half(p, src, row, h, w);
 }
 
+// The first half of a task's chunks, once they have arrived: quantizes them
+// and issues the loads of the second half (rows of eight chunks), which then
+// arrive during the task's first double rounds.  Run at the end of the
+// previous task, whose last rounds cover the first half's loads.
 template <int DT, int FAM>
-__device__ __forceinline__ void first_half(const EgressParams& p, const EgressPage& pg, const Row& row,
+__device__ __forceinline__ void first_half(const ProducerCtx& c, const Row& row, int group,
                                            uint32_t (&w)[4][8], uint32_t (&pt)[16], uint32_t (&sc)[4]) {
     if (tq_row<FAM>(row)) row_untranspose(w);
     quant_first<DT, FAM>(row.s.kind, w, pt, sc);
-    if (two_halves<FAM>(row.s.kind)) load_half_any<FAM>(p, pg, row, 1, w);
+    if (two_halves<FAM>(row.s.kind)) load_half_any<FAM>(*c.p, c.hot(group, row.s.src), row, 1, w);
 }
 
-// One code row.  pt / sc hold the row's first half quantized (first_half, at
-// the end of the previous row) and w the second half's chunks when the row
-// has two, loaded since; the second half is quantized after four double
-// rounds.  The next row's first four chunks are loaded into w then, and at
-// the end of this row first_half runs for the next row.  Every kind of row
-// issues the next row's loads at the same point, into the same registers,
+// One task.  pt / sc hold its rows' first half quantized (first_half, at
+// the end of the previous task) and w the second half's chunks when the rows
+// have two, loaded since; the second half is quantized after four double
+// rounds.  The next task's first four chunks are loaded into w then, and at
+// the end of this task first_half runs for the next one.  Every kind of row
+// issues the next task's loads at the same point, into the same registers,
 // so that no path has to move a register whose load is still in flight
 // (such a move would make the wave wait for it).
 template <int DT, int FAM>
-__device__ __forceinline__ void code_row(const ProducerCtx& c, const Row& row, const Row& nxt,
-                                         uint32_t (&w)[4][8], uint32_t (&pt)[16], uint32_t (&sc)[4]) {
+__device__ __forceinline__ void code_task(const ProducerCtx& c, const Row& row, int group, const Row& nxt, int ngroup,
+                                          uint32_t (&w)[4][8], uint32_t (&pt)[16], uint32_t (&sc)[4]) {
     const EgressParams& p = *c.p;
     uint32_t* flags = c.lds + kLdsFlags;
+    const uint32_t* used = &flags[kFlagMacUsed];
     const int32_t kind = row.s.kind;
+    const int r = c.lane >> 4, pg = group * kTaskPages + (c.lane & 15);
+    const uint32_t* tab = c.lds + kLdsNonce + pg * kNonceWords;
+    const uint32_t ctr = 1u + (uint32_t)(row.block + r);
     ChaChaState st;
-    st.start_cached(p.key, c.nc, 1u + (uint32_t)row.block);
+    {
+        ChaChaNonceCache nc;
+        nonce_cache(tab, nc);
+        st.start_cached(p.key, nc, ctr);
+    }
     st.double_rounds<4>();
     // the priority is refreshed after four and after seven double rounds;
     // pin_words keeps the rounds on their side of each refresh
     pin_words(st.x);
-    refresh_row_priority(&flags[kFlagMacUsed], row.mrow);
+    refresh_row_priority(used, row.mrow);
     // the second half's scale words go to variables of their own: stores
     // into sc at other indices than the first half's let the compiler merge
     // the two quantizer calls into one store at a runtime index, which puts
@@ -352,78 +406,95 @@ __device__ __forceinline__ void code_row(const ProducerCtx& c, const Row& row, c
     } else if (FAM == 2 && kind == kSecInt4G32) {
         s2 = quant_half_int4g32<DT>(w, pt + 8);
     }
-    if (nxt.valid) load_half_any<FAM>(p, c.pg, nxt, 0, w);
+    if (nxt.valid) load_half_any<FAM>(p, c.hot(ngroup, nxt.s.src), nxt, 0, w);
     st.double_rounds<3>();
     pin_words(st.x);
-    refresh_row_priority(&flags[kFlagMacUsed], row.mrow);
+    refresh_row_priority(used, row.mrow);
     st.double_rounds<2>();
     if (kind != kSecRaw) {
-        // the unit's staging slot is free once unit g - kStage's scale row is done
+        // the unit's staging slot is free once the storer has stored unit
+        // g - kStage's scale row
         uint32_t* stage = c.lds + kLdsStage + (row.g % kStage) * kRowWords;
         wait_ge<kDiagEgressWait, kTmStageWait>(&flags[kFlagStage + row.g % kStage], row.g - kStage + 1, c.wt);
-        // parameter words of this row: 2 (int8, e4m3, int4 per 32), 4 (int4)
-        // or 1 (asym8), at logical words j * sw .. of this lane's page.  One
+        // parameter words of this lane's row j: 2 (int8, e4m3, int4 per 32), 4
+        // (int4) or 1 (asym8), at logical words j * sw .. of its page.  One
         // branch per count: a loop bounded by a runtime count would index sc
         // at run time and put it in scratch memory.
-        const int sw = param_words_per_row(kind);
+        const int sw = param_words_per_row(kind), j = row.j + r;
         if (sw == 4) {  // int4: two words per half
-            stage[quad_word(c.lane, row.j) + 0] = sc[0];
-            stage[quad_word(c.lane, row.j) + 1] = sc[1];
-            stage[quad_word(c.lane, row.j) + 2] = s2;
-            stage[quad_word(c.lane, row.j) + 3] = s3;
+            *reinterpret_cast<uint4*>(stage + quad_word(pg, j)) = make_uint4(sc[0], sc[1], s2, s3);
         } else if (sw == 2) {  // int8, e4m3: both words from the first half; int4 per 32: one per half
-            const int wd = row.j * 2;
+            const int wd = j * 2;
             const bool split = FAM == 2 && kind == kSecInt4G32;
-            stage[quad_word(c.lane, wd >> 2) + (wd & 3)] = sc[0];
-            stage[quad_word(c.lane, wd >> 2) + (wd & 3) + 1] = split ? s2 : sc[1];
+            stage[quad_word(pg, wd >> 2) + (wd & 3)] = sc[0];
+            stage[quad_word(pg, wd >> 2) + (wd & 3) + 1] = split ? s2 : sc[1];
         } else {
-            stage[quad_word(c.lane, row.j >> 2) + (row.j & 3)] = sc[0];
+            stage[quad_word(pg, j >> 2) + (j & 3)] = sc[0];
         }
     }
     uint32_t ks[16];
-    st.finish(p.key, 1u + (uint32_t)row.block, c.n0, c.n1, c.n2, ks);
-    // the row's ciphertext is complete before the ring waits: left to
+    const u32x4 nn = *reinterpret_cast<const u32x4*>(tab);
+    st.finish(p.key, ctr, nn.x, nn.y, nn.z, ks);
+    // the rows' ciphertext is complete before the ring waits: left to
     // itself, the compiler sinks the last rounds below the waits (their
     // results are only used after them), so a wave that finds the ring full
     // would wait first and compute afterwards
 #pragma unroll
     for (int i = 0; i < 16; ++i) ks[i] ^= pt[i];
     pin_words(ks);
-    uint32_t* slot = c.lds + (row.mrow % kRing) * kRowWords;
-    wait_ge<kDiagEgressWait, kTmRingWait>(&flags[kFlagMacUsed], row.mrow - kRing + 1, c.wt);
-    wait_ge<kDiagEgressWait, kTmRingWait>(&flags[kFlagStored], row.mrow - kRing + 1, c.wt);
+    // four consecutive slots, the last of them the last to become free
+    int32_t slot = row.mrow % kRing + r;
+    slot -= slot >= kRing ? kRing : 0;
+    uint32_t* dst = c.lds + slot * kRowWords;
+    wait_both_ge<kDiagEgressWait, kTmRingWait>(used, &flags[kFlagStored], row.mrow + kTaskRows - kRing, c.wt);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-        lds_put_quad(slot, c.lane, q, make_uint4(ks[4 * q], ks[4 * q + 1], ks[4 * q + 2], ks[4 * q + 3]));
-    publish(&flags[kFlagRing + row.mrow % kRing], (uint32_t)row.mrow + 1u);  // the storer wave stores it
-    tm_trace(c.wt.trace, row.mrow, c.wt.t0);
-    if (nxt.valid) first_half<DT, FAM>(p, c.pg, nxt, w, pt, sc);
+        lds_put_quad(dst, pg, q, make_uint4(ks[4 * q], ks[4 * q + 1], ks[4 * q + 2], ks[4 * q + 3]));
+    // the MAC wave and the storer take them from here
+    if ((c.lane & 15) == 0) publish_lds(&flags[kFlagRing + group * kRing + slot], (uint32_t)(row.mrow + r) + 1u);
+    if constexpr (kPhaseTimers) {
+        if (group == 0)
+            for (int i = 0; i < kTaskRows; ++i) tm_trace(c.wt.trace, row.mrow + i, c.wt.t0);
+    }
+    if (kind != kSecRaw) {
+        // the task that stages the last scales of its scale group (for this
+        // page group) encrypts them; the storer stores them
+        const int32_t u0 = row.u & ~(kScaleGroup - 1), n = min(kScaleGroup, row.s.n_units - u0);
+        const int32_t g0 = row.g - (row.u - u0);
+        uint32_t old = 0;
+        if (c.lane == 0)
+            old = __hip_atomic_fetch_add(&flags[kFlagCount + group * kStage + g0 % kStage], 1u, __ATOMIC_ACQ_REL,
+                                         __HIP_MEMORY_SCOPE_WORKGROUP);
+        old = __builtin_amdgcn_readfirstlane(old);
+        if (old == (uint32_t)(n * (row.s.nblk / kTaskRows)) - 1u) {
+            flags[kFlagCount + group * kStage + g0 % kStage] = 0u;
+            encrypt_scales(c, group, n, g0, row.s.s_off / 64u + (uint32_t)u0);
+            publish_lds(&flags[kFlagEnc + group * kStage + g0 % kStage], (uint32_t)g0 + 1u);
+        }
+    }
+    if (nxt.valid) first_half<DT, FAM>(c, nxt, ngroup, w, pt, sc);
 }
 
 template <int DT, int FAM>
-__device__ void egress_produce(const EgressParams& p, int64_t page0, int ppw, uint32_t* lds) {
+__device__ void egress_produce(const EgressParams& p, int ppw, uint32_t* lds) {
     ProducerCtx c;
     c.p = &p;
     c.lane = threadIdx.x & 63;
-    c.pg = egress_page(p, page0 + (c.lane < ppw ? c.lane : 0));
-    c.n0 = (uint32_t)c.pg.seq;
-    c.n1 = (uint32_t)(c.pg.seq >> 32);
-    c.n2 = c.pg.nonce2;
-    c.nc.init(p.key, c.n0, c.n1, c.n2);
     c.lds = lds;
+    c.ng = page_groups(ppw);
     c.wt = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, phase_clock());
     c.wt.trace = trace_of(p.timers);
-    const int32_t total = total_code_rows(p.lay);
-    // The page descriptor and kernel argument loads above complete here,
-    // before the loop: a load still counted as in flight where the loop
-    // begins makes the compiler wait for every outstanding memory operation
-    // wherever the loop uses its result.
+    const int32_t total = total_code_rows(p.lay) / kTaskRows * c.ng;
+    // The kernel argument loads above complete here, before the loop: a load
+    // still counted as in flight where the loop begins makes the compiler
+    // wait for every outstanding memory operation wherever the loop uses its
+    // result.
     __builtin_amdgcn_s_waitcnt(0);
     if constexpr (kPhaseTimers) tm_min(c.wt.tm, kTmProdSetup, phase_clock() - c.wt.t0);
     uint32_t* flags = lds + kLdsFlags;
-    // code rows are handed out in order from an LDS counter, one row ahead of
-    // the one being made (so its groups can be prefetched): a slower wave
-    // simply takes fewer rows
+    // tasks are handed out in order from an LDS counter, one ahead of the
+    // one being made (so its groups can be prefetched): a slower wave simply
+    // takes fewer
     // (also reads how many rows the MAC wave has absorbed, for the priority)
     int32_t used = 0;
     auto grab = [&]() -> int32_t {
@@ -436,25 +507,29 @@ __device__ void egress_produce(const EgressParams& p, int64_t page0, int ppw, ui
     };
     uint32_t w[4][8];
     uint32_t pt[16], sc[4];
-    int32_t t = grab();
-    Row cur = row_info(p.lay, t);
+    int32_t t = grab(), quad, group;
+    split_task(t, c.ng, quad, group);
+    Row cur = row_info(p.lay, quad * kTaskRows);
     if (cur.valid) {
-        load_half_any<FAM>(p, c.pg, cur, 0, w);
-        first_half<DT, FAM>(p, c.pg, cur, w, pt, sc);
+        load_half_any<FAM>(p, c.hot(group, cur.s.src), cur, 0, w);
+        first_half<DT, FAM>(c, cur, group, w, pt, sc);
         if constexpr (kPhaseTimers) tm_min(c.wt.tm, kTmProdLoaded, phase_clock() - c.wt.t0);
     }
     [[maybe_unused]] int32_t made = 0;
 #pragma unroll 1
     while (t < total) {
         const int32_t tn = grab();
+        int32_t ngroup;
+        split_task(tn, c.ng, quad, ngroup);
         set_row_priority(cur.mrow - used);
-        const Row nxt = row_info(p.lay, tn);
-        code_row<DT, FAM>(c, cur, nxt, w, pt, sc);
+        const Row nxt = row_info(p.lay, quad * kTaskRows);
+        code_task<DT, FAM>(c, cur, group, nxt, ngroup, w, pt, sc);
         if constexpr (kPhaseTimers) {
             if (made++ == 0) tm_min(c.wt.tm, kTmProdFirstRow, phase_clock() - c.wt.t0);
         }
         t = tn;
         cur = nxt;
+        group = ngroup;
     }
     if constexpr (kPhaseTimers) {
         const uint64_t now = phase_clock() - c.wt.t0;
@@ -499,38 +574,41 @@ struct MacPlan {
     __device__ __forceinline__ int32_t ns(int32_t si) const { return si == 0 ? ns0 : (si == 1 ? ns1 : (si == 2 ? ns2 : 0)); }
 };
 
-template <int DT>
+// The MAC wave: page lane / 2, two lanes per page (PAIR), or page lane.
+template <bool PAIR>
 __device__ void egress_mac(const EgressParams& p, int64_t page0, int ppw, uint32_t* lds, uint64_t t0) {
-    const int lane = threadIdx.x & 63;
-    const bool active = lane < ppw;
-    const EgressPage pg = egress_page(p, page0 + (active ? lane : 0));
+    const int pl = MacQuads<PAIR>::page();
+    const bool active = pl < ppw;
+    const bool writer = active && MacQuads<PAIR>::reads();  // stores the page's header and tag
+    const EgressPage pg = egress_page(p, page0 + (active ? pl : 0));
     uint8_t* blob = pg.blob;
-    if (active) {  // header (cpp:1129-1140)
+    if (writer) {  // header (cpp:1129-1140)
         stg16(blob, 0, make_uint4((uint32_t)p.hdr0, (uint32_t)(p.hdr0 >> 32), (uint32_t)pg.hdr1,
                                   (uint32_t)(pg.hdr1 >> 32)));
         stg16(blob, 1, make_uint4((uint32_t)pg.token, (uint32_t)(pg.token >> 32), (uint32_t)pg.seq,
                                   (uint32_t)(pg.seq >> 32)));
     }
-    Sip s;
+    MacHash<PAIR> s;
     s.init(p.mk0, p.mk1);
     const uint64_t hdr[4] = {p.hdr0, pg.hdr1, pg.token, pg.seq};
-    s.absorb_words<4>(hdr);
-    PageQuads pq;
-    pq.init(lane);
-    MacPlan m;
-    m.init(p.lay);
+    s.template absorb_words<4>(hdr);
+    MacQuads<PAIR> mq;
+    mq.init((uint32_t)kLdsZero * 4u);
+    MacPlan mp;
+    mp.init(p.lay);
     // Rows arrive in MAC order in the ring (code rows from the producers,
     // scale rows from the feeder), so the next row is always the next slot.
     Waiter wt = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, t0);
     wt.trace = trace_of(p.timers);
-    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_waitcnt(0);  // also the header stores: a failed workgroup's headers are zeroed by another wave
     if constexpr (kPhaseTimers) tm_add(wt.tm, kTmMacRowsBegin, phase_clock() - t0);
-    mac_rows<kRing, kDiagEgressWait>(wt, lds, lds + kLdsFlags + kFlagRing, lds + kLdsFlags + kFlagMacUsed, pq, s,
-                                     m.total);
+    const int group = min(pl / kTaskPages, page_groups(ppw) - 1);
+    mac_rows<kRing, kDiagEgressWait, PAIR>(wt, lds, lds + kLdsFlags + kFlagRing + group * kRing,
+                                           lds + kLdsFlags + kFlagMacUsed, mq, s, mp.total);
     if constexpr (kPhaseTimers) tm_add(wt.tm, kTmMacRowsEnd, phase_clock() - t0);
     uint64_t lo, hi;
     s.finish((uint64_t)((kHeader + p.payload) & 0xFFu) << 56, lo, hi);
-    if (active)
+    if (writer)
         stg16(blob + kHeader + p.payload, 0,
               make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)));
     if constexpr (kPhaseTimers) tm_add(wt.tm, kTmMacEnd, phase_clock() - t0);
@@ -557,19 +635,19 @@ __device__ __forceinline__ void feed_load(const Waiter& wt, const uint32_t* lds,
     }
 }
 
-__device__ __forceinline__ void feed_put(const Waiter& wt, uint32_t* lds, const PageQuads& pq, int32_t rs,
+__device__ __forceinline__ void feed_put(const Waiter& wt, uint32_t* lds, const PageQuads& pq, int ng, int32_t rs,
                                          const uint4 (&x)[4]) {
     uint32_t* flags = lds + kLdsFlags;
-    wait_ge<kDiagEgressWait, kTmFeedWait>(&flags[kFlagMacUsed], rs - kRing + 1, wt);
-    wait_ge<kDiagEgressWait, kTmFeedWait>(&flags[kFlagStored], rs - kRing + 1, wt);
+    wait_both_ge<kDiagEgressWait, kTmFeedWait>(&flags[kFlagMacUsed], &flags[kFlagStored], rs - kRing + 1, wt);
     uint32_t* slot = lds + (rs % kRing) * kRowWords;
 #pragma unroll
     for (int q = 0; q < 4; ++q) lds_put_quad_at(slot, pq.off[q], x[q]);
-    publish(&flags[kFlagRing + rs % kRing], (uint32_t)rs + 1u);
+    const int g = (int)(threadIdx.x & 63);
+    if (g < ng) publish_lds(&flags[kFlagRing + g * kRing + rs % kRing], (uint32_t)rs + 1u);  // every page group's flag
     tm_trace(wt.trace, rs, wt.t0);
 }
 
-__device__ void egress_scale_feed(const EgressParams& p, uint32_t* lds) {
+__device__ void egress_scale_feed(const EgressParams& p, int ng, uint32_t* lds) {
     const int lane = threadIdx.x & 63;
     const uint8_t* blob = reinterpret_cast<const uint8_t*>(reinterpret_cast<const uint64_t*>(lds + kLdsBlobs)[lane]);
     PageQuads pq;
@@ -590,10 +668,10 @@ __device__ void egress_scale_feed(const EgressParams& p, uint32_t* lds) {
 #pragma unroll 1
         for (int32_t j = 0; j < n; j += 2) {
             if (j + 1 < n) feed_load(wt, lds, base ? base + 64u * (uint32_t)(j + 1) : nullptr, g0 + j + 1, b);
-            feed_put(wt, lds, pq, rs + j, a);
+            feed_put(wt, lds, pq, ng, rs + j, a);
             if (j + 1 >= n) break;
             if (j + 2 < n) feed_load(wt, lds, base ? base + 64u * (uint32_t)(j + 2) : nullptr, g0 + j + 2, a);
-            feed_put(wt, lds, pq, rs + j + 1, b);
+            feed_put(wt, lds, pq, ng, rs + j + 1, b);
         }
         g0 += n;
         r0 = rs + n;
@@ -601,49 +679,88 @@ __device__ void egress_scale_feed(const EgressParams& p, uint32_t* lds) {
     if constexpr (kPhaseTimers) tm_max(wt.tm, kTmFeedEnd, phase_clock() - wt.t0);
 }
 
-// Storer (one wave on SIMD 1): stores every code row from the ring to the
-// blobs, in payload order (the MAC order), transposed -- four lanes per page,
-// 64 contiguous bytes of 16 pages per store instruction -- and publishes
-// `stored` = rows passed; a ring slot is rewritten only once the MAC wave and
-// the storer have both passed it.  Once it has stored a unit's last code row
-// it also makes the unit's scale row (every code row stages its scales before
-// releasing its ring row), so the producers never wait for a unit to fill.
-// A section's scale rows are neighbours in the blob: the storer keeps each
-// encrypted one in its staging slot until it has made the next ones and
-// stores them kScaleGroup at a time (the section's last ones as they come),
-// so that the 128-byte lines they share are written at once instead of one
-// unit apart, when the first half is often evicted and written back alone.
-// Holding them creates no cycle of waits: the MAC wave reaches a section's
-// scale rows after all of its code rows, and a producer of unit g waits for
-// the slot of unit g - kStage, which is stored at the latest with unit
-// g - kStage + kScaleGroup - 1, a unit before g (kScaleGroup <= kStage).
-// That a scale row's stores have completed is published for the feeder
-// before the storer next waits for a row, or once four are outstanding: the
-// storer issues no loads, so those waits only cover its own stores.  Stores
-// are kept off the producers, whose waits for their own loads would
-// otherwise also wait for every store they issued before those loads, and
-// off the MAC wave's SIMD, where the data and address reads of scattered
-// stores take register-file cycles from the chain.
-__device__ void egress_store_rows(const EgressParams& p, int64_t page0, int ppw, uint32_t* lds) {
-    ProducerCtx c;
-    c.p = &p;
-    c.lane = threadIdx.x & 63;
-    c.pg = egress_page(p, page0 + (c.lane < ppw ? c.lane : 0));
-    c.n0 = (uint32_t)c.pg.seq;
-    c.n1 = (uint32_t)(c.pg.seq >> 32);
-    c.n2 = c.pg.nonce2;
-    c.nc.init(p.key, c.n0, c.n1, c.n2);
-    c.lds = lds;
-    c.wt = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, phase_clock());
-    c.init_stores(ppw);
+// Storer (one wave on SIMD 1): stores the code rows from the ring to the
+// blobs in payload order (the MAC order), the four rows of a task at a time
+// -- sixteen lanes per page, 256 contiguous bytes of four pages per store
+// instruction -- and publishes `stored` = rows passed; a ring slot is
+// rewritten only once the MAC wave and the storer have both passed it.  The
+// scale rows of a scale group (kScaleGroup units), neighbours in the blob,
+// are stored the same way from their staging slots, which that frees: one
+// scale group behind the code rows, so that the producer that encrypts them
+// has done so, and the last ones at the section's end.
+// The waits point backwards only: a scale group is waited for after all of
+// its code rows are stored, so each of its tasks is past its ring wait; the
+// producer of a unit waits for the slot of the unit kStage before it, which
+// lies at least two scale groups back (kStage >= 3 kScaleGroup).
+// That the scale rows' stores have completed is published for the feeder
+// before the storer next waits for a row, or once two groups are
+// outstanding: the storer issues no global loads, so those waits only cover
+// its own stores.  Stores are kept off the producers, whose waits for their
+// own loads would otherwise also wait for every store they issued before
+// those loads.
+struct RowStores {
+    const uint32_t* lds;
+    int ppw;
+    uint32_t pofs;   // this lane's place in the 256 bytes of a page
+    int page, row, quad;
+
+    __device__ __forceinline__ void init(const uint32_t* l, int pages) {
+        const int lane = threadIdx.x & 63;
+        lds = l;
+        ppw = pages;
+        page = lane >> 4;
+        row = lane >> 2 & 3;
+        quad = lane & 3;
+        pofs = (uint32_t)(lane & 15) * 16u;
+    }
+    // Rows in `slot` (this lane's row's, in words) of every page to blob
+    // offset off + row_off.  Past the last page of a partial workgroup a lane
+    // stores page 0's quad again: unconditional stores.
+    __device__ __forceinline__ void store(uint32_t slot, uint32_t off) const {
+        const uint64_t* blobs = reinterpret_cast<const uint64_t*>(lds + kLdsBlobs);
+#pragma unroll 1
+        for (int p0 = 0; p0 < ppw; p0 += 16) {
+            uint4 x[4];
+            uint8_t* b[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int pg = p0 + 4 * k + page, pe = pg < ppw ? pg : 0;
+                x[k] = lds_quad(lds + slot, pe, quad);
+                b[k] = reinterpret_cast<uint8_t*>(blobs[pe]);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) stg16(b[k] + off, 0, x[k]);
+        }
+    }
+};
+
+__device__ void egress_store_rows(const EgressParams& p, int ppw, uint32_t* lds) {
+    const int lane = threadIdx.x & 63, ng = page_groups(ppw);
+    const Waiter wt = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, phase_clock());
+    RowStores rs;
+    rs.init(lds, ppw);
     uint32_t* flags = lds + kLdsFlags;
     // a slot is reused only once stored: never let the producers sharing
     // this SIMD starve the storer
     __builtin_amdgcn_s_setprio(2);
     __builtin_amdgcn_s_waitcnt(0);
     int32_t r = 0, g0 = 0;      // payload row; quantized units before the section
-    int32_t made = 0, pub = 0;  // scale rows made / published as stored
-    int32_t held = 0;           // encrypted scale rows waiting in their slots for the rest of their group
+    int32_t made = 0, pub = 0;  // scale rows stored / published as stored
+    const int fg = min(lane >> 2 & 3, ng - 1);  // the page group and row this lane's flag stands for
+    auto store_scales = [&](int32_t u0, int32_t nu, uint32_t sblk) {
+        const int32_t n = min(kScaleGroup, nu - u0), first = g0 + u0;
+        wait_lanes_ge<kDiagEgressWait, kTmStorerWait>(&flags[kFlagEnc + fg * kStage + first % kStage], first + 1, wt);
+        const int32_t i = min(rs.row, n - 1);  // lanes past the last unit store its row again
+        rs.store((uint32_t)(kLdsStage + ((first + i) % kStage) * kRowWords),
+                 (uint32_t)kHeader + 64u * (sblk + (uint32_t)(u0 + i)) + 16u * (uint32_t)rs.quad);
+        // the release follows the slot reads
+        if (lane < n) publish(&flags[kFlagStage + (first + lane) % kStage], (uint32_t)(first + lane) + 1u);
+        made += n;
+        if (made - pub >= 2 * kScaleGroup) {
+            publish_scales(flags, pub, made);
+            pub = made;
+        }
+    };
 #pragma unroll
     for (int si = 0; si < 3; ++si) {
         if (si >= p.lay.n_sec) continue;
@@ -653,42 +770,40 @@ __device__ void egress_store_rows(const EgressParams& p, int64_t page0, int ppw,
         const uint32_t sblk = ZTCP_SEC_FIELD(p.lay, si, s_off) / 64u;
         const bool quant = kind != kSecRaw;
         const int32_t ncode = nu * nblk;
+        int32_t us = 0;  // units whose scale rows are stored
 #pragma unroll 1
-        for (int32_t cr = 0; cr < ncode; ++cr, ++r) {
-            const uint32_t* f = &flags[kFlagRing + r % kRing];
+        for (int32_t cr = 0; cr < ncode; cr += kTaskRows, r += kTaskRows) {
+            int32_t slot = r % kRing + (lane & 3);
+            slot -= slot >= kRing ? kRing : 0;
+            const uint32_t* f = &flags[kFlagRing + fg * kRing + slot];
+            const int32_t want = r + (lane & 3) + 1;
             if (pub < made &&
-                (int32_t)__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < r + 1) {
+                __builtin_amdgcn_ballot_w64((int32_t)__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <
+                                            want) != 0ull) {
                 publish_scales(flags, pub, made);
                 pub = made;
             }
-            wait_ge<kDiagEgressWait, kTmStorerWait>(f, r + 1, c.wt);
-            store_row(lds + (r % kRing) * kRowWords, c, (uint32_t)kHeader + 64u * (uint32_t)r);
-            publish(&flags[kFlagStored], (uint32_t)r + 1u);  // the release orders the slot reads before it
-            if (quant && (cr & (nblk - 1)) == nblk - 1) {
-                const int32_t u = cr / nblk;
-                encrypt_scale_row(c, g0 + u, sblk + (uint32_t)u);
-                if (held < kScaleGroup - 1 && u + 1 < nu) {
-                    ++held;
-                } else {
-#pragma unroll 1
-                    for (int32_t h = u - held; h <= u; ++h) store_scale_row(c, g0 + h, sblk + (uint32_t)h);
-                    made += held + 1;
-                    held = 0;
-                    if (made - pub >= 4) {
-                        publish_scales(flags, pub, made);
-                        pub = made;
-                    }
-                }
+            wait_lanes_ge<kDiagEgressWait, kTmStorerWait>(f, want, wt);
+            int32_t ds = r % kRing + rs.row;
+            ds -= ds >= kRing ? kRing : 0;
+            rs.store((uint32_t)(ds * kRowWords), (uint32_t)kHeader + 64u * (uint32_t)r + rs.pofs);
+            publish(&flags[kFlagStored], (uint32_t)(r + kTaskRows));  // the release orders the slot reads before it
+            const int32_t done = (cr + kTaskRows) / nblk;  // whole units stored
+            if (quant && done - us >= 2 * kScaleGroup) {
+                store_scales(us, nu, sblk);
+                us += kScaleGroup;
             }
         }
         if (quant) {  // the section's scale rows reach the ring through the feeder
 #pragma unroll 1
-            for (int32_t i = 0; i < nu; ++i, ++r) publish(&flags[kFlagStored], (uint32_t)r + 1u);
+            for (; us < nu; us += kScaleGroup) store_scales(us, nu, sblk);
+            r += nu;
+            publish(&flags[kFlagStored], (uint32_t)r);
             g0 += nu;
         }
     }
     publish_scales(flags, pub, made);
-    if constexpr (kPhaseTimers) tm_max(c.wt.tm, kTmStorerEnd, phase_clock() - c.wt.t0);
+    if constexpr (kPhaseTimers) tm_max(wt.tm, kTmStorerEnd, phase_clock() - wt.t0);
 }
 
 // FAM 0: the reference's section kinds (int8, int4, raw); FAM 1: also e4m3
@@ -702,12 +817,25 @@ __global__ __launch_bounds__(64 * egress_waves<FAM>()) void egress_fused_kernel(
     const int64_t page0 = (int64_t)blockIdx.x * p.ppw;
     const int ppw = (int)min((int64_t)p.ppw, p.batch - page0);
     for (int i = threadIdx.x; i < kNumFlags; i += blockDim.x) lds[kLdsFlags + i] = 0u;
+    if (threadIdx.x < 4) lds[kLdsZero + threadIdx.x] = 0u;
     tm_clear(lds + kLdsTimers);
     tm_trace_clear(p.timers);
     if (threadIdx.x < 64) {
         uint64_t* blobs = reinterpret_cast<uint64_t*>(lds + kLdsBlobs);
-        blobs[threadIdx.x] = (int)threadIdx.x < ppw ? reinterpret_cast<uint64_t>(egress_page(p, page0 + threadIdx.x).blob)
-                                                    : 0ull;  // null past the last page
+        // past the last page: page 0's tables, a null blob
+        const EgressPage pg = egress_page(p, page0 + ((int)threadIdx.x < ppw ? threadIdx.x : 0));
+        blobs[threadIdx.x] = (int)threadIdx.x < ppw ? reinterpret_cast<uint64_t>(pg.blob) : 0ull;
+        uint64_t* hot = reinterpret_cast<uint64_t*>(lds + kLdsHot);
+        hot[2 * threadIdx.x] = reinterpret_cast<uint64_t>(pg.k);
+        hot[2 * threadIdx.x + 1] = reinterpret_cast<uint64_t>(pg.v);
+        ChaChaNonceCache nc;
+        nc.init(p.key, (uint32_t)pg.seq, (uint32_t)(pg.seq >> 32), pg.nonce2);
+        uint32_t* tab = lds + kLdsNonce + threadIdx.x * kNonceWords;
+        tab[0] = (uint32_t)pg.seq;
+        tab[1] = (uint32_t)(pg.seq >> 32);
+        tab[2] = pg.nonce2;
+#pragma unroll
+        for (int i = 0; i < 12; ++i) tab[4 + i] = nc.c[i];
     }
     __syncthreads();
     [[maybe_unused]] const uint64_t t0 = phase_clock();
@@ -715,21 +843,22 @@ __global__ __launch_bounds__(64 * egress_waves<FAM>()) void egress_fused_kernel(
     const int wave = threadIdx.x >> 6;
     if (wave == 0) {
         __builtin_amdgcn_s_setprio(3);
-        egress_mac<DT>(p, page0, ppw, lds, t0);
+        if (p.ppw <= kPairPages) egress_mac<true>(p, page0, ppw, lds, t0);
+        else egress_mac<false>(p, page0, ppw, lds, t0);
     } else if (wave == 4) {
-        egress_scale_feed(p, lds);
+        egress_scale_feed(p, page_groups(ppw), lds);
     } else if ((wave & 3) == 0) {
         // the rest of the MAC wave's SIMD stays idle
     } else if (wave == 1) {
-        egress_store_rows(p, page0, ppw, lds);
+        egress_store_rows(p, ppw, lds);
     } else {
-        egress_produce<DT, FAM>(p, page0, ppw, lds);
+        egress_produce<DT, FAM>(p, ppw, lds);
     }
     // Fail closed: if any bounded wait of the workgroup expired, its rows may
     // have been read or overwritten out of turn, so no blob of the workgroup
-    // may verify.  The MAC wave's lanes, which stored the headers, zero the
-    // first 16 header bytes (magic 0: every ingress rejects the page with
-    // status 1).  Same lanes, same addresses: the stores stay in order.
+    // may verify.  The first 16 header bytes are zeroed (magic 0: every ingress
+    // rejects the page with status 1); the MAC wave's header stores completed
+    // before its first row.
     __syncthreads();
     tm_flush(lds + kLdsTimers, p.timers, t0, rt0);
     if (__hip_atomic_load(lds + kLdsFlags + kFlagExpired, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0u &&

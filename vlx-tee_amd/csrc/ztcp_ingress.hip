@@ -68,7 +68,8 @@ constexpr int kLdsLayouts = kLdsPtrs + 2 * 2 * 64;   // [kNumLayouts] Layout, on
 constexpr int kLayoutWords = (int)(sizeof(Layout) / 4);
 constexpr int kLdsHeaders = (kLdsLayouts + kNumLayouts * kLayoutWords + 3) & ~3;  // [64] 32-byte headers
 constexpr int kLdsTimers = kLdsHeaders + 64 * 8;       // phase-timer counters (timer builds only)
-constexpr int kLdsWords = kLdsTimers + kTimerLdsWords;
+constexpr int kLdsZero = (kLdsTimers + kTimerLdsWords + 3) & ~3;  // a zero quad: the message of the verify wave's A lanes
+constexpr int kLdsWords = kLdsZero + 4;
 static_assert(kLdsHeaders % 4 == 0, "header table must be 16-byte aligned");
 static_assert(sizeof(Layout) % 4 == 0, "Layout is copied word by word");
 static_assert(kLdsWords * 4 <= 160 * 1024, "LDS budget of one CU");
@@ -752,10 +753,12 @@ __device__ __forceinline__ int32_t page_verdict(const IngressParams& p, int64_t 
     return 0;
 }
 
-// Verdict of one page (cpp:2313-2355).  The payload's full 64-byte rows
-// come from the ring; its last (payload % 64) bytes and the tag are loaded
-// with the header.
-__device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t page, uint32_t* lds, int lane,
+// Verdict of this lane's page (MacQuads::page: with PAIR two lanes per page,
+// both return it), cpp:2313-2355.  The payload's full 64-byte rows come from
+// the ring; its last (payload % 64) bytes and the tag are loaded with the
+// header (h0, h1).
+template <bool PAIR>
+__device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t page, uint32_t* lds,
                                                const uint4 h0, const uint4 h1, uint64_t t0) {
     const uint8_t* blob = ingress_blob(p, page);
     const uint8_t* pay = blob + kHeader;
@@ -766,18 +769,18 @@ __device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t p
 #pragma unroll
     for (int i = 0; i < 3; ++i) tl[i] = ldg16(pay + min(tail0 + 16u * (uint32_t)i, p.payload), 0);
     const uint4 tag = ldg16(pay + p.payload, 0);
-    Sip s;
+    MacHash<PAIR> s;
     s.init(p.mk0, p.mk1);
     const uint64_t hdr[4] = {lo64(h0), hi64(h0), lo64(h1), hi64(h1)};
-    s.absorb_words<4>(hdr);
-    PageQuads pq;
-    pq.init(lane);
+    s.template absorb_words<4>(hdr);
+    MacQuads<PAIR> mq;
+    mq.init((uint32_t)kLdsZero * 4u);
     Waiter st = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, t0);
     st.trace = trace_of(p.timers);
     __builtin_amdgcn_s_waitcnt(0);
     if constexpr (kPhaseTimers) tm_add(st.tm, kTmMacRowsBegin, phase_clock() - t0);
-    mac_rows<kRing, kDiagIngressWait>(st, lds, lds + kLdsFlags + kFlagRing, lds + kLdsFlags + kFlagMacUsed, pq, s,
-                                      total);
+    mac_rows<kRing, kDiagIngressWait, PAIR>(st, lds, lds + kLdsFlags + kFlagRing, lds + kLdsFlags + kFlagMacUsed, mq, s,
+                                            total);
     if constexpr (kPhaseTimers) tm_add(st.tm, kTmMacRowsEnd, phase_clock() - t0);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -896,6 +899,7 @@ __global__ __launch_bounds__(kIngressThreads) void ingress_fused_kernel(IngressP
     if (threadIdx.x < kNumLayouts) layouts[threadIdx.x] = ingress_layout(p, (int)threadIdx.x);
     uint32_t* flags = lds + kLdsFlags;
     for (int i = threadIdx.x; i < kNumFlags; i += blockDim.x) flags[i] = 0u;
+    if (threadIdx.x < 4) lds[kLdsZero + threadIdx.x] = 0u;
     tm_clear(lds + kLdsTimers);
     tm_trace_clear(p.timers);
     if (threadIdx.x < 64) {
@@ -920,7 +924,13 @@ __global__ __launch_bounds__(kIngressThreads) void ingress_fused_kernel(IngressP
     const Layout& lay = layouts[has_lay ? li_wg : 0];
     if (wave == 0) {
         __builtin_amdgcn_s_setprio(3);
-        flags[kFlagStatus + lane] = (uint32_t)verify_page(p, page, lds, lane, h0, h1, t0);
+        if (p.ppw <= kPairPages) {
+            const int pl = MacQuads<true>::page(), pv = pl < ppw ? pl : 0;
+            const int32_t st = verify_page<true>(p, page0 + pv, lds, hdrs[2 * pv], hdrs[2 * pv + 1], t0);
+            if (MacQuads<true>::reads()) flags[kFlagStatus + pl] = (uint32_t)st;
+        } else {
+            flags[kFlagStatus + lane] = (uint32_t)verify_page<false>(p, page, lds, h0, h1, t0);
+        }
     } else if (wave == 4) {
         ingress_feed(p, lds, lay, has_lay, blob + kHeader, lane);
     } else if ((wave & 3) != 0 && has_lay) {  // waves 8 and 12 share SIMD 0 and idle

@@ -203,6 +203,22 @@ __device__ __forceinline__ Waiter make_waiter(const WaitSink& s, uint32_t* expir
     return Waiter{s.dev_diag, s.call_diag, expired_lds, s.spin_limit, s.call_tag, tm, t0, nullptr};
 }
 
+// Records an expired wait: the device's and the call's diagnostics, and the
+// workgroup's LDS word.
+template <uint32_t DIAG>
+__device__ __forceinline__ void expire(const Waiter& w) {
+    if ((threadIdx.x & 63) == 0) {
+        atomicOr(w.dev_diag, DIAG);
+        if (w.call_diag) {
+            // egress calls carry a tag (the host reads the slot back by tag);
+            // ingress calls or in their kernel's bit
+            if constexpr (DIAG == kDiagEgressWait) atomicMax(w.call_diag, w.call_tag);
+            else atomicOr(w.call_diag, DIAG);
+        }
+    }
+    __hip_atomic_store(w.expired, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // Waits until *flag >= want (monotonic counters; want <= 0 returns at once).
 // Bounded: after spin_limit polls the wait records DIAG (device and call
 // diagnostics, the workgroup's LDS word) and returns; the caller carries on,
@@ -219,20 +235,46 @@ __device__ __forceinline__ void wait_ge(const uint32_t* flag, int32_t want, cons
     for (uint32_t spin = 0;; ++spin) {
         if (__hip_atomic_load(w.expired, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0u) break;
         if (spin >= w.spin_limit) {
-            if ((threadIdx.x & 63) == 0) {
-                atomicOr(w.dev_diag, DIAG);
-                if (w.call_diag) {
-                    // egress calls carry a tag (the host reads the slot back
-                    // by tag); ingress calls or in their kernel's bit
-                    if constexpr (DIAG == kDiagEgressWait) atomicMax(w.call_diag, w.call_tag);
-                    else atomicOr(w.call_diag, DIAG);
-                }
-            }
-            __hip_atomic_store(w.expired, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            expire<DIAG>(w);
             break;
         }
         __builtin_amdgcn_s_sleep(1);
         if ((int32_t)__hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= want) break;
+    }
+    if constexpr (kPhaseTimers && TSLOT >= 0) tm_add(w.tm, TSLOT, phase_clock() - t_in);
+}
+
+// Waits until *f0 and *f1 are both >= want: the two counters are loaded
+// together, so a wait that is already satisfied costs one LDS latency.
+template <uint32_t DIAG, int TSLOT>
+__device__ __forceinline__ void wait_both_ge(const uint32_t* f0, const uint32_t* f1, int32_t want, const Waiter& w) {
+    const uint32_t a = __hip_atomic_load(f0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    const uint32_t b = __hip_atomic_load(f1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if ((int32_t)a >= want && (int32_t)b >= want) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        return;
+    }
+    wait_ge<DIAG, TSLOT>(f0, want, w);
+    wait_ge<DIAG, TSLOT>(f1, want, w);
+}
+
+// wait_ge with a flag (and bound) of its own in every lane: until all are set.
+template <uint32_t DIAG, int TSLOT = -1>
+__device__ __forceinline__ void wait_lanes_ge(const uint32_t* flag, int32_t want, const Waiter& w) {
+    auto ready = [&]() {
+        const bool late = (int32_t)__hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < want;
+        return __builtin_amdgcn_ballot_w64(late) == 0ull;
+    };
+    if (ready()) return;
+    [[maybe_unused]] const uint64_t t_in = (kPhaseTimers && TSLOT >= 0) ? phase_clock() : 0;
+    for (uint32_t spin = 0;; ++spin) {
+        if (__hip_atomic_load(w.expired, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0u) break;
+        if (spin >= w.spin_limit) {
+            expire<DIAG>(w);
+            break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        if (ready()) break;
     }
     if constexpr (kPhaseTimers && TSLOT >= 0) tm_add(w.tm, TSLOT, phase_clock() - t_in);
 }
@@ -316,8 +358,8 @@ __device__ __forceinline__ uint4 mac_flags4(const uint32_t* ring_flags, int32_t 
 }
 
 // Whether rows row0 .. row0 + 3 (those below total) are all in the ring.
-// Every lane read the same words: a vector compare and a ballot cost the
-// chain nothing measurable, where v_readfirstlane of a flag cost it about
+// Every lane read the flags of its own page's group: a vector compare and a
+// ballot cost the chain nothing measurable, where v_readfirstlane of a flag cost it about
 // 66 clocks.
 __device__ __forceinline__ bool mac_ready4(const uint4 f, int32_t row0, int32_t total) {
     const bool ok = ((int32_t)f.x > row0 || row0 >= total) && ((int32_t)f.y > row0 + 1 || row0 + 1 >= total) &&
@@ -325,9 +367,46 @@ __device__ __forceinline__ bool mac_ready4(const uint4 f, int32_t row0, int32_t 
     return __builtin_amdgcn_ballot_w64(!ok) == 0ull;
 }
 
-__device__ __forceinline__ void mac_row_data(const uint32_t* ring, const PageQuads& pq, int32_t slot, uint4 (&x)[4]) {
+// The MAC / verify wave hashes two lanes per page (SipPair) in a workgroup of
+// up to 32 pages, one lane per page (Sip) in a larger one.  Two lanes take 34
+// instructions per word against 46 and so shorten the chain, which is what a
+// launch of up to 32 pages per workgroup lasts; but 64 pages then need two
+// such waves, 68 instructions per word, and a large launch is bound by the
+// instructions all waves issue together (16,384 pages of K8V4: egress 436 us
+// with one wave and 451 with two, ingress 486 and 498; 4,087 MLA pages, 16 a
+// workgroup: egress 399 us with one lane per page, 361 with two).
+constexpr int kPairPages = 32;
+
+// Byte offsets of a MAC lane's four quads inside a row slot.  PAIR: lane 2 i + 1
+// (B) reads page i, the A lanes read the zero quad (`zero_off`, from the
+// ring's start) whatever the slot; else lane = page.
+template <bool PAIR>
+struct MacQuads {
+    uint32_t off[4];
+    uint32_t slot_mask;
+    __device__ __forceinline__ static int page() {
+        return (int)(threadIdx.x & 63) >> (PAIR ? 1 : 0);
+    }
+    __device__ __forceinline__ static bool reads() { return !PAIR || SipPair::lane_b(); }
+    __device__ __forceinline__ void init(uint32_t zero_off) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) x[q] = lds_quad_at(ring + slot * kRowWords, pq.off[q]);
+        for (int q = 0; q < 4; ++q) off[q] = reads() ? quad_word(page(), q) * 4u : zero_off;
+        slot_mask = reads() ? ~0u : 0u;
+    }
+    __device__ __forceinline__ uint32_t slot_off(int32_t slot) const {
+        const uint32_t so = (uint32_t)(slot * kRowWords * 4);
+        return PAIR ? so & slot_mask : so;
+    }
+};
+template <bool PAIR> struct MacHashOf { using type = Sip; };
+template <> struct MacHashOf<true> { using type = SipPair; };
+template <bool PAIR> using MacHash = typename MacHashOf<PAIR>::type;
+
+template <bool PAIR>
+__device__ __forceinline__ void mac_row_data(const uint32_t* ring, const MacQuads<PAIR>& mq, int32_t slot, uint4 (&x)[4]) {
+    const uint32_t so = mq.slot_off(slot);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[q] = lds_quad_at(ring, so + mq.off[q]);
 }
 
 // Absorbs payload rows [0, total) from a ring of RING slots, four rows per
@@ -341,9 +420,9 @@ __device__ __forceinline__ void mac_row_data(const uint32_t* ring, const PageQua
 // slots that are never absorbed.  The caller completes every load it has
 // issued before the call: a load still counted as in flight where the loop
 // begins would turn the loop's LDS waits into full waits.
-template <int RING, uint32_t DIAG>
+template <int RING, uint32_t DIAG, bool PAIR>
 __device__ __forceinline__ void mac_rows(const Waiter& wt, const uint32_t* ring, const uint32_t* ring_flags,
-                                         uint32_t* used, const PageQuads& pq, Sip& s, int32_t total) {
+                                         uint32_t* used, const MacQuads<PAIR>& pq, MacHash<PAIR>& s, int32_t total) {
     static_assert(RING % kMacGroup == 0 && kMacGroup == 4, "a group's flags are one aligned 16-byte read");
     uint4 b0[4], b1[4], b2[4], b3[4];
     int32_t gs = 0;  // ring slot of the group's first row
@@ -359,7 +438,7 @@ __device__ __forceinline__ void mac_rows(const Waiter& wt, const uint32_t* ring,
     // A row taken alone: waited for, read, absorbed and released at once.
     auto one_row = [&](int32_t row, int32_t slot, uint64_t& waited) {
         [[maybe_unused]] const uint64_t t_in = phase_clock();
-        wait_ge<DIAG>(ring_flags + slot, row + 1, wt);
+        wait_lanes_ge<DIAG>(ring_flags + slot, row + 1, wt);
         if constexpr (kPhaseTimers) waited += phase_clock() - t_in;
         mac_row_data(ring, pq, slot, b2);
         s.absorb64(b2);
@@ -428,13 +507,32 @@ __device__ __forceinline__ void mac_rows(const Waiter& wt, const uint32_t* ring,
 }
 
 // ---------------------------------------------------------------------------
-// Loads four lanes per page.  A load of 16 bytes per lane from 64 pages
-// touches 64 lines per instruction; four lanes per page read 64 contiguous
-// bytes of 16 pages (on all 256 workgroups at once: 4.8 TB/s against
-// 3.1 TB/s, a probe over 16,384 pages).  Lane 16 r + c takes quad r of page
-// 16 i + c in load i; the four 16-lane rows of four such loads are then
-// transposed (row_transpose) so that every lane holds its own page's quads.
+// Tasks.  A producer or decoder wave makes kTaskRows consecutive code rows of
+// a unit for kTaskPages pages of the workgroup at once: lane 16 r + c has row
+// r of page c of the task's page group.  Against one row of 64 pages the
+// same 64 keystream blocks touch runs of four times the bytes per page: all
+// workgroups walk their pages in step, so the bytes of a page that are asked
+// for together decide what HBM delivers (a probe over 16,384 pages of 32 KiB,
+// 256-byte rows: writes 2.87 TB/s a row at a time, 4.63 four rows at a time,
+// reads 5.22 and 5.40; 128-byte half rows: writes 4.76 and 6.92, reads 5.11
+// and 6.76), and a workgroup of 16 pages or fewer leaves no lane idle.
+// Loads of 16 bytes per lane from 64 places touch 64 lines per instruction;
+// the rows that read 256 hot bytes are loaded four lanes per page instead
+// (64 contiguous bytes of 16 pages): lane 16 r + c takes quad r of row i of
+// page c in load i, and the 16-lane rows of four such loads are then
+// transposed (row_transpose) so that every lane holds its own row's quads.
 // ---------------------------------------------------------------------------
+constexpr int kTaskRows = 4;
+constexpr int kTaskPages = 16;
+
+// Page groups of a workgroup.
+__device__ __forceinline__ int page_groups(int ppw) { return (ppw + kTaskPages - 1) / kTaskPages; }
+
+// Task t -> row quad and page group (the groups of a row quad one after the other).
+__device__ __forceinline__ void split_task(int32_t t, int ng, int32_t& quad, int32_t& group) {
+    quad = ng == 1 ? t : (ng == 2 ? t >> 1 : (ng == 4 ? t >> 2 : t / 3));
+    group = t - quad * ng;
+}
 
 typedef uint32_t ztcp_u32x2 __attribute__((ext_vector_type(2)));
 
@@ -462,27 +560,6 @@ __device__ __forceinline__ void row_transpose(uint32_t (&a)[8], uint32_t (&b)[8]
         swap_rows(a[d], a[4 + d]);
         swap_rows(b[d], b[4 + d]);
     }
-}
-
-// p of lanes c, 16 + c, 32 + c, 48 + c, for every lane of column c.
-__device__ __forceinline__ void column_ptrs(const void* p, const uint8_t* (&out)[4]) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    uint32_t lo[4], hi[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        lo[i] = (uint32_t)v;
-        hi[i] = (uint32_t)(v >> 32);
-    }
-    swap_halves(lo[0], lo[2]);
-    swap_halves(lo[1], lo[3]);
-    swap_rows(lo[0], lo[1]);
-    swap_rows(lo[2], lo[3]);
-    swap_halves(hi[0], hi[2]);
-    swap_halves(hi[1], hi[3]);
-    swap_rows(hi[0], hi[1]);
-    swap_rows(hi[2], hi[3]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = reinterpret_cast<const uint8_t*>(((uint64_t)hi[i] << 32) | lo[i]);
 }
 
 // Row geometry of one section (all values wave-uniform).
