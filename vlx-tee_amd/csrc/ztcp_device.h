@@ -144,15 +144,6 @@ struct ChaChaState {
     }
 };
 
-// Keystream block `ctr` of a page whose first column round is cached.
-__device__ __forceinline__ void chacha_block_cached(const ChaKey& key, const ChaChaNonceCache& nc, uint32_t ctr,
-                                                    uint32_t n0, uint32_t n1, uint32_t n2, uint32_t ks[16]) {
-    ChaChaState st;
-    st.start_cached(key, nc, ctr);
-    st.double_rounds<9>();
-    st.finish(key, ctr, n0, n1, n2, ks);
-}
-
 // ---------------------------------------------------------------------------
 // SipHash-2-4 with 128-bit output (cpp:401-471).
 // One page per lane; the chain is strictly sequential, so its cost is the

@@ -88,7 +88,6 @@ constexpr int kNumFlags = (kFlagExpired + 2) & ~1;    // even: the blob table af
 constexpr int kLdsBlobs = kLdsFlags + kNumFlags;      // [64] blob pointers (8-byte aligned)
 constexpr int kLdsHot = (kLdsBlobs + 2 * 64 + 3) & ~3;  // [64] K and V pointers
 constexpr int kLdsNonce = kLdsHot + 4 * 64;           // [64] nonce (3 words, a pad) and its ChaChaNonceCache
-constexpr int kNonceWords = 16;
 constexpr int kLdsTimers = kLdsNonce + kNonceWords * 64;  // phase-timer counters (timer builds only)
 constexpr int kLdsZero = (kLdsTimers + kTimerLdsWords + 3) & ~3;  // a zero quad: the message of the MAC wave's A lanes
 constexpr int kLdsWords = kLdsZero + 4;
@@ -96,18 +95,6 @@ static_assert(kLdsWords * 4 <= 160 * 1024, "LDS budget of one CU");
 static_assert(kRing % 4 == 0 && kRing >= 2 * kTaskRows, "a group's ring flags are aligned; two tasks fit the ring");
 static_assert(kStage >= 3 * kScaleGroup, "the storer keeps one scale group while the producers stage the next two");
 static_assert(kLdsBlobs % 2 == 0 && kLdsTimers % 2 == 0, "blob table and timers must be 8-byte aligned");
-
-__device__ __forceinline__ int32_t total_rows(const Layout& lay) {
-    int32_t t = 0;
-#pragma unroll
-    for (int si = 0; si < 3; ++si) {
-        if (si >= lay.n_sec) continue;
-        const int32_t kind = ZTCP_SEC_FIELD(lay, si, kind);
-        const int32_t rpu = code_rows_per_unit(kind) + (kind != kSecRaw ? 1 : 0);
-        t += ZTCP_SEC_FIELD(lay, si, n_units) * rpu;
-    }
-    return t;
-}
 
 __device__ __forceinline__ void load_group(const uint8_t* p, uint32_t w[8]) {
     const uint4 a = ldg16(p, 0), b = ldg16(p, 1);
@@ -144,12 +131,13 @@ __device__ __forceinline__ void load_task_half(const EgressParams& p, const uint
     const int nch = chunks_per_row(row.s.kind);
     const uint32_t gpv = (uint32_t)row.s.gpv;
     const uint32_t G0 = (uint32_t)((row.u * row.s.nblk + row.j) * nch + 4 * h);  // the first row's chunk
-    const uint32_t vec0 = G0 / gpv;
+    const uint32_t vec0 = div_gpv(row.s, G0);
     // this lane's chunk, counted from the start of the vector of the first
     // row's: at most gpv - 1 + 3 * 8, so past 28 chunks per vector it wraps
-    // at most once, and below the reciprocal is exact
+    // at most once, and below gmul is exact (a page holds less than 2^30
+    // elements)
     uint32_t g = G0 - vec0 * gpv + (threadIdx.x >> 4 & 3u) * (uint32_t)nch;
-    const uint32_t over = gpv > 28u ? (g >= gpv ? 1u : 0u) : (g * (65536u / gpv + 1u)) >> 16;
+    const uint32_t over = gpv > 28u ? (g >= gpv ? 1u : 0u) : (gpv == 1u ? g : __umulhi(g, row.s.gmul));
     g -= over * gpv;
     uint32_t off = (vec0 + over) * (uint32_t)p.head_dim * 2u + (uint32_t)row.s.col * 2u + g * 32u;
     if ((gpv & 3u) == 0u) {  // four contiguous chunks
@@ -176,9 +164,9 @@ __device__ __forceinline__ void load_task_half(const EgressParams& p, const uint
 __device__ __forceinline__ void load_task_half_t(const EgressParams& p, const uint8_t* src, const Row& row, int h,
                                                  uint32_t (&w)[4][8]) {
     const int32_t per_row = chunks_per_row(row.s.kind) / 4;  // pieces of four chunks
-    const int32_t gp4 = row.s.gpv / 4;                       // pieces per vector
+    const int32_t gp4 = row.s.gpv >> 2;                      // pieces per vector
     const int32_t piece = (row.u * row.s.nblk + row.j) * per_row + h;
-    int32_t vec = piece / gp4, gi = piece - vec * gp4;
+    int32_t vec = (int32_t)div_gpv(row.s, (uint32_t)piece * 4u), gi = piece - vec * gp4;
     const uint8_t* base = src + (uint32_t)row.s.col * 2u + (threadIdx.x >> 4 & 3u) * 16u;
     uint32_t off[4];
 #pragma unroll
@@ -220,16 +208,6 @@ struct ProducerCtx {
         return reinterpret_cast<const uint8_t*>(t[src]);
     }
 };
-
-// One ChaCha20 block of page `pg` of the workgroup, counter 1 + block, nonce
-// and first column round from the LDS table.
-__device__ __forceinline__ void nonce_cache(const uint32_t* tab, ChaChaNonceCache& nc) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(tab + 4 + 4 * q);
-        nc.c[4 * q] = v.x; nc.c[4 * q + 1] = v.y; nc.c[4 * q + 2] = v.z; nc.c[4 * q + 3] = v.w;
-    }
-}
 
 // Quantizes groups w[0..3] (int8: 4 code words each, int4: 2) into pt[] and
 // their fp16 scales into sc[] (two per word, low half first).
@@ -279,12 +257,8 @@ __device__ __forceinline__ void encrypt_scales(const ProducerCtx& c, int group, 
     const EgressParams& p = *c.p;
     const int pg = group * kTaskPages + (c.lane & 15);
     const int32_t i = min(c.lane >> 4, n - 1);
-    const uint32_t* tab = c.lds + kLdsNonce + pg * kNonceWords;
-    ChaChaNonceCache nc;
-    nonce_cache(tab, nc);
-    const u32x4 nn = *reinterpret_cast<const u32x4*>(tab);
     uint32_t ks[16];
-    chacha_block_cached(p.key, nc, 1u + block0 + (uint32_t)i, nn.x, nn.y, nn.z, ks);
+    table_block(p.key, c.lds + kLdsNonce + pg * kNonceWords, 1u + block0 + (uint32_t)i, ks);
     uint32_t* stage = c.lds + kLdsStage + ((g0 + i) % kStage) * kRowWords;
     uint4 sw[4];
 #pragma unroll
@@ -828,14 +802,7 @@ __global__ __launch_bounds__(64 * egress_waves<FAM>()) void egress_fused_kernel(
         uint64_t* hot = reinterpret_cast<uint64_t*>(lds + kLdsHot);
         hot[2 * threadIdx.x] = reinterpret_cast<uint64_t>(pg.k);
         hot[2 * threadIdx.x + 1] = reinterpret_cast<uint64_t>(pg.v);
-        ChaChaNonceCache nc;
-        nc.init(p.key, (uint32_t)pg.seq, (uint32_t)(pg.seq >> 32), pg.nonce2);
-        uint32_t* tab = lds + kLdsNonce + threadIdx.x * kNonceWords;
-        tab[0] = (uint32_t)pg.seq;
-        tab[1] = (uint32_t)(pg.seq >> 32);
-        tab[2] = pg.nonce2;
-#pragma unroll
-        for (int i = 0; i < 12; ++i) tab[4 + i] = nc.c[i];
+        put_nonce(lds + kLdsNonce + threadIdx.x * kNonceWords, p.key, (uint32_t)pg.seq, (uint32_t)(pg.seq >> 32), pg.nonce2);
     }
     __syncthreads();
     [[maybe_unused]] const uint64_t t0 = phase_clock();

@@ -3,23 +3,29 @@
 // HBM read of the blob and one HBM write of the hot page.  Replaces the
 // per-page decoder of fused_decode_cold_pages_peak_into_cpu (cpp:2309-2463).
 //
-// One workgroup handles up to 64 pages with 16 waves, four per SIMD (lane =
-// page in every wave):
+// One workgroup handles up to 64 pages with 16 waves, four per SIMD:
 //   * Every page is decoded according to its own header flags.  The
 //     workgroup's layout is that of its first page with valid flags; pages
 //     with that layout go through the row pipeline below, pages with another
 //     valid layout are decoded afterwards unit by unit, pages with invalid
 //     flags are not decoded (they fail with status 1).
-//   * Twelve decoder waves (on SIMDs 1-3) take rows in order from an LDS
-//     counter, each with its ciphertext block loaded one row ahead.  A
-//     unit's scale row is decrypted into an LDS staging slot four units ahead
-//     of its code rows.  A code row first puts its ciphertext into a ring of
-//     row slots in LDS, at its place in payload order, then decrypts, takes
-//     its scales from staging and dequantizes two groups at a time into a
-//     per-wave LDS tile, from which the wave stores them transposed: four
-//     lanes per page, so each store writes the two groups (64 bytes,
-//     contiguous within a head vector) of 16 pages.
-//   * Wave 0 verifies one page per lane at raised priority on SIMD 0:
+//   * Twelve decoder waves (on SIMDs 1-3) take tasks in order from an LDS
+//     counter, each with its ciphertext loaded a task ahead: four
+//     consecutive code rows of a unit for one group of 16 pages, lane = (row,
+//     page), or the scale rows of four units, which are decrypted into LDS
+//     staging slots half a scale group or more ahead of their code rows.  A
+//     code task first puts its ciphertext into a ring of row slots in LDS, at
+//     its place in payload order, then decrypts, takes its scales from
+//     staging and dequantizes two groups at a time into a per-wave LDS tile,
+//     from which the wave stores them transposed: four lanes per (row, page),
+//     so each store writes the two groups (64 bytes, contiguous within a head
+//     vector) of 16 pages.  Four rows of 16 pages instead of one row of 64: a
+//     workgroup of a few pages leaves no lane idle (1,777 MLA pages of int4
+//     per 32, 7 a workgroup: 355 us a row at a time, 239 four rows at a time
+//     with the two-lane verify wave), and a page's bytes are read 256 and
+//     written up to 1,024 at a time (16,384 pages of K8V4: 485 and 479 us).
+//   * Wave 0 verifies at raised priority on SIMD 0 (two lanes per page in a
+//     workgroup of up to 32 pages, one lane per page in a larger one):
 //     magic/version (status 1), AAD tenant/model/layer/token hash (status
 //     2), the SipHash-2-4-128 tag over header || ciphertext (status 3), then
 //     flags and payload size (status 1), in the reference's order
@@ -49,32 +55,34 @@ constexpr int kIngressThreads = 64 * kIngressWaves;
 constexpr int kDecoderWaves = 12;  // the waves on SIMDs 1-3
 constexpr int kRing = 16;          // payload rows between their makers and the verify wave
 constexpr int kStage = 8;          // units whose decrypted scales are staged at once
-constexpr int kLookahead = 4;      // a unit's scale row is handed out this many units early
+constexpr int kLookahead = 4;      // units whose scale rows are decrypted together, ahead of their code rows
 constexpr int kLdsStage = kRing * kRowWords;
-constexpr int kLdsTile = kLdsStage + kStage * kRowWords;       // per decoder wave: 2 groups per page
+constexpr int kLdsTile = kLdsStage + kStage * kRowWords;       // per decoder wave: 2 groups per row and page
 constexpr int kLdsFlags = kLdsTile + kDecoderWaves * kRowWords;
-constexpr int kFlagRing = 0;                         // [kRing] payload row index + 1
-constexpr int kFlagReady = kFlagRing + kRing;        // [kStage] unit + 1: scales decrypted
-constexpr int kFlagFree = kFlagReady + kStage;       // [kStage] unit + 1: scales consumed
-constexpr int kFlagCount = kFlagFree + kStage;       // [kStage] code rows that took their scales
-constexpr int kFlagMacUsed = kFlagCount + kStage;    // payload rows absorbed by the verify wave
-constexpr int kFlagTask = kFlagMacUsed + 1;          // next row to hand out
+constexpr int kFlagRing = 0;                         // [4][kRing] per page group: payload row index + 1
+constexpr int kFlagReady = kFlagRing + 4 * kRing;    // [4][kStage] unit + 1: scales decrypted
+constexpr int kFlagFree = kFlagReady + 4 * kStage;   // [4][kStage] unit + 1: scales consumed
+constexpr int kFlagCount = kFlagFree + 4 * kStage;   // [4][kStage] tasks of a unit that took their scales
+constexpr int kFlagMacUsed = kFlagCount + 4 * kStage;  // payload rows absorbed by the verify wave
+constexpr int kFlagTask = kFlagMacUsed + 1;          // next task to hand out
 constexpr int kFlagStatus = kFlagTask + 1;           // [64] verdicts
 constexpr int kFlagNaN = kFlagStatus + 64;           // [64] 1: the page has an inf / NaN scale
 constexpr int kFlagExpired = kFlagNaN + 64;          // 1: a bounded wait of the workgroup expired
 constexpr int kNumFlags = (kFlagExpired + 2) & ~1;   // even: the pointer table after it is 8-byte aligned
-constexpr int kLdsPtrs = kLdsFlags + kNumFlags;      // [2][64] output pointers (K, V)
-constexpr int kLdsLayouts = kLdsPtrs + 2 * 2 * 64;   // [kNumLayouts] Layout, one per header flags value
+constexpr int kLdsPtrs = kLdsFlags + kNumFlags;      // [2][64] output pointers (K, V), [64] blob pointers
+constexpr int kLdsLayouts = kLdsPtrs + 3 * 2 * 64;   // [kNumLayouts] Layout, one per header flags value
 constexpr int kLayoutWords = (int)(sizeof(Layout) / 4);
 constexpr int kLdsHeaders = (kLdsLayouts + kNumLayouts * kLayoutWords + 3) & ~3;  // [64] 32-byte headers
-constexpr int kLdsTimers = kLdsHeaders + 64 * 8;       // phase-timer counters (timer builds only)
+constexpr int kLdsNonce = kLdsHeaders + 64 * 8;      // [64] nonce table
+constexpr int kLdsTimers = kLdsNonce + 64 * kNonceWords;  // phase-timer counters (timer builds only)
 constexpr int kLdsZero = (kLdsTimers + kTimerLdsWords + 3) & ~3;  // a zero quad: the message of the verify wave's A lanes
 constexpr int kLdsWords = kLdsZero + 4;
 static_assert(kLdsHeaders % 4 == 0, "header table must be 16-byte aligned");
 static_assert(sizeof(Layout) % 4 == 0, "Layout is copied word by word");
 static_assert(kLdsWords * 4 <= 160 * 1024, "LDS budget of one CU");
 static_assert(kLdsPtrs % 2 == 0, "pointer table must be 8-byte aligned");
-static_assert(kStage >= kLookahead + 1, "a scale row only waits for units whose code rows come before it");
+static_assert(kRing % 4 == 0 && kRing >= 2 * kTaskRows, "a group's ring flags are aligned; two tasks fit the ring");
+static_assert(kStage >= 2 * kLookahead, "scales are decrypted while the units before them are decoded");
 
 __device__ __forceinline__ void load_block(const uint8_t* p, uint32_t w[16]) {
 #pragma unroll
@@ -267,146 +275,108 @@ __device__ __forceinline__ void decode_unit(const IngressParams& p, const Layout
 // Row pipeline.
 // ---------------------------------------------------------------------------
 
-// Row t of the decode order.  Per section of U units: the scale rows of units
-// 0 .. L-1, then the units' code rows, two units at a time with the scale
-// rows of units u + L and u + 1 + L (L = kLookahead) between them (task_info
-// below), so a unit's scales are decrypted while the units before it are
-// being decoded.
+// Task t of a workgroup: an item of the layout's decode order, for one page
+// group of it (split_task).  An item is four consecutive code rows of a unit,
+// or the scale rows of a scale group (kLookahead = 4 units).  Per quantized
+// section of G scale groups: S(0), S(1), C(0), then for q = 1 .. G - 2 the
+// code items C(q) with S(q + 1) halfway, then C(G - 1): the slots of S(q + 1)
+// are those of C(q - 1), whose tasks have all been handed out half a group
+// before.  The four scale rows of a group are neighbours in the blob, 256
+// bytes that one task reads at once.
 struct Task {
     int32_t valid;
-    int32_t scale;    // 1: scale row of unit u
-    int32_t u, j;     // unit in section, code block in unit
+    int32_t scale;    // 1: scale rows of units u .. u + n - 1
+    int32_t n;        // rows (code: kTaskRows)
+    int32_t u, j;     // unit in section, first code row in unit
     int32_t g;        // unit index among the page's quantized units (staging order)
-    int32_t cidx;     // code row index (payload order of the code rows)
-    int32_t mrow;     // payload row of a code row (its place in the ring)
-    int32_t block;    // payload block index (keystream counter - 1)
+    int32_t mrow;     // payload row of the first code row (its place in the ring)
+    int32_t block;    // payload block index of the first row (keystream counter - 1)
+    int32_t group;    // page group
     SecRows s;
 };
 
-template <int FAM>
-__device__ __forceinline__ int32_t div_nblk(int32_t x, int32_t kind) {  // nblk = 8, 4, 16
-    if constexpr (FAM == 1) {
-        const int32_t nblk = code_rows_per_unit(kind);
-        return nblk == 8 ? x / 8 : (nblk == 4 ? x / 4 : x / 16);
-    }
-    return kind == kSecInt8 ? x / 8 : (kind == kSecInt4 ? x / 4 : x / 16);
-}
-template <int FAM>
-__device__ __forceinline__ int32_t div_rpu2(int32_t x, int32_t kind) {  // 2 (nblk + 1) = 18, 10, 34
-    if constexpr (FAM == 1) {
-        const int32_t nblk = code_rows_per_unit(kind);
-        return nblk == 8 ? x / 18 : (nblk == 4 ? x / 10 : x / 34);
-    }
-    return kind == kSecInt8 ? x / 18 : x / 10;
+// Item i of a quantized section of `nsg` scale groups, qpu code items per
+// unit: returns the code item's index, or ~q for S(q).
+__device__ __forceinline__ int32_t section_item(int32_t i, int32_t nsg, int32_t qpu) {
+    const int32_t pre = min(2, nsg), per = kLookahead * qpu;  // code items of a whole scale group
+    if (i < pre) return ~i;
+    i -= pre;
+    if (i < per || nsg <= 2) return i;
+    i -= per;
+    const int32_t span = per + 1;
+    const int32_t b = qpu == 1 ? i / (kLookahead + 1) : (qpu == 2 ? i / (2 * kLookahead + 1) : i / (4 * kLookahead + 1));
+    if (b >= nsg - 2) return per * (nsg - 1) + i - (nsg - 2) * span;
+    const int32_t off = i - b * span;
+    if (off == per / 2) return ~(b + 2);
+    return per * (b + 1) + off - (off > per / 2 ? 1 : 0);
 }
 
-// Task t of the workgroup layout.  A quantized section hands out the scale
-// rows of its first kLookahead units, then its units' code rows two units
-// at a time with the scale rows of the two units kLookahead further on
-// between them: code rows of u, scale rows of u + L and u + 1 + L, code
-// rows of u + 1.  Neighbouring scale rows share 128-byte lines in the blob,
-// and decoders that take them one after the other read those lines at once.
-template <int FAM>
-__device__ __forceinline__ Task task_info(const Layout& lay, int32_t t) {
+__device__ __forceinline__ Task task_info(const Layout& lay, int32_t t, int ng) {
     Task k{};
-    int32_t tb = 0, cb = 0, qb = 0;
+    int32_t item;
+    split_task(t, ng, item, k.group);
+    int32_t ib = 0, cb = 0, qb = 0;
 #pragma unroll
     for (int si = 0; si < 3; ++si) {
         if (si >= lay.n_sec || k.valid) continue;
         const SecRows s = sec_rows(lay, si, cb, qb);
         const bool quant = s.kind != kSecRaw;
-        const int32_t n = s.n_units * s.nblk + (quant ? s.n_units : 0);
-        if (t >= tb && t < tb + n) {
-            int32_t x = t - tb;
+        const int32_t qpu = s.nblk / kTaskRows;  // 1, 2 or 4 code items per unit
+        const int32_t nsg = quant ? (s.n_units + kLookahead - 1) / kLookahead : 0;
+        const int32_t n = s.n_units * qpu + nsg;
+        if (item >= ib && item < ib + n) {
+            const int32_t x = quant ? section_item(item - ib, nsg, qpu) : item - ib;
             k.valid = 1;
-            if (!quant) {
-                k.u = div_nblk<FAM>(x, s.kind);
-                k.j = x - k.u * s.nblk;
-            } else {
-                const int32_t pre = min(kLookahead, s.n_units);
-                const int32_t full = max(s.n_units - kLookahead, 0);  // units followed by a scale row
-                if (x < pre) {
-                    k.scale = 1;
-                    k.u = x;
-                } else if ((x -= pre) < full * s.rpu) {
-                    const int32_t span = 2 * s.rpu, pairs = full >> 1;
-                    int32_t u0, off;
-                    if (x < pairs * span) {
-                        const int32_t p2 = div_rpu2<FAM>(x, s.kind);
-                        u0 = 2 * p2;
-                        off = x - p2 * span;
-                    } else {  // an odd last unit: its code rows, then one scale row
-                        u0 = full - 1;
-                        off = x - pairs * span;
-                    }
-                    if (off < s.nblk) {
-                        k.u = u0;
-                        k.j = off;
-                    } else if (off <= s.nblk + 1) {
-                        k.scale = 1;
-                        k.u = u0 + kLookahead + (off - s.nblk);
-                    } else {
-                        k.u = u0 + 1;
-                        k.j = off - s.nblk - 2;
-                    }
-                } else {
-                    x -= full * s.rpu;
-                    const int32_t u = div_nblk<FAM>(x, s.kind);
-                    k.u = full + u;
-                    k.j = x - u * s.nblk;
-                }
-            }
+            k.scale = x < 0 ? 1 : 0;
+            const int32_t u = qpu == 1 ? x : (qpu == 2 ? x >> 1 : x >> 2);
+            k.u = x < 0 ? ~x * kLookahead : u;
+            k.j = x < 0 ? 0 : (x - u * qpu) * kTaskRows;
+            k.n = x < 0 ? min(kLookahead, s.n_units - k.u) : kTaskRows;
             k.g = s.qunit_begin + k.u;
-            k.cidx = cb + k.u * s.nblk + k.j;
-            k.mrow = k.cidx + qb;  // a section's codes follow the scale rows of the sections before it
-            k.block = k.scale ? (int32_t)(s.s_off / 64u) + k.u : (int32_t)(s.q_off / 64u) + k.u * s.nblk + k.j;
+            k.mrow = cb + k.u * s.nblk + k.j + qb;  // a section's codes follow the scale rows of the sections before it
+            k.block = x < 0 ? (int32_t)(s.s_off / 64u) + k.u : (int32_t)(s.q_off / 64u) + k.u * s.nblk + k.j;
             k.s = s;
         }
-        tb += n;
+        ib += n;
         cb += s.n_units * s.nblk;
         if (quant) qb += s.n_units;
     }
     return k;
 }
 
-__device__ __forceinline__ int32_t total_tasks(const Layout& lay) {
+__device__ __forceinline__ int32_t total_items(const Layout& lay) {
     int32_t t = 0;
 #pragma unroll
     for (int si = 0; si < 3; ++si) {
         if (si >= lay.n_sec) continue;
-        const int32_t kind = ZTCP_SEC_FIELD(lay, si, kind);
-        t += ZTCP_SEC_FIELD(lay, si, n_units) * (code_rows_per_unit(kind) + (kind != kSecRaw ? 1 : 0));
+        const int32_t kind = ZTCP_SEC_FIELD(lay, si, kind), nu = ZTCP_SEC_FIELD(lay, si, n_units);
+        t += nu * (code_rows_per_unit(kind) / kTaskRows) + (kind != kSecRaw ? (nu + kLookahead - 1) / kLookahead : 0);
     }
     return t;
 }
 
-// The payload row that sets a task's urgency: a code task's own row; a
-// scale task is as urgent as the first code row of its unit.
-__device__ __forceinline__ int32_t task_lead_row(const Task& k) {
-    return k.scale ? (int32_t)(k.s.q_off / 64u) + k.u * k.s.nblk : k.mrow;
-}
-
 struct DecoderCtx {
     const IngressParams* p;
-    const uint8_t* pay;     // this lane's page payload
-    uint32_t n0, n1, n2;    // this lane's page nonce (from its header)
-    ChaChaNonceCache nc;
     uint32_t* lds;
-    uint32_t* tile;         // this wave's dequantized tile
-    PageQuads pq;           // this lane's quads in a row slot
+    uint32_t* tile;         // this wave's dequantized tile: entry 16 r + c is row r of page c of the task
+    PageQuads tq;           // this lane's quads in the tile
     Waiter wt;
     int lane;
-    // Transposed tile stores: store k (0..3) writes quad (lane & 3) of page
-    // 16 k + (lane >> 2), whose output pointer is entry 16 k + (lane >> 2)
-    // of the pointer table.  Past the last page of a partial workgroup the
-    // table holds page 0's pointers, and the tile holds page 0's data (those
-    // lanes decode page 0), so every store is unconditional: a store under a
-    // branch makes the compiler wait for all outstanding stores before the
-    // next row's loads.  The quad swizzle of page 16 k + i equals that of
-    // page i, so store k's tile offset is tq0 + 1024 k bytes.
+    int ng;                 // page groups of the workgroup
+    // Transposed tile stores: store r (0..3) writes quad (lane & 3) of row r
+    // of page lane >> 2 of the task's page group, whose output pointer comes
+    // from the pointer table.  Past the last page of a partial workgroup the
+    // tables hold page 0's entries, so those lanes decode and store page 0's
+    // bytes and every store is unconditional: a store under a branch makes
+    // the compiler wait for all outstanding stores before the next row's
+    // loads.  The quad swizzle of entry 16 r + i equals that of entry i, so
+    // store r's tile offset is tq0 + 1024 r bytes.
     uint32_t tq0;
 
     __device__ __forceinline__ void init_stores() { tq0 = quad_word(lane >> 2, lane & 3) * 4u; }
+    // Ciphertext of this lane's row of a task (a scale group's lanes past its
+    // last row read that row again).
+    __device__ __forceinline__ void load(const Task& k, uint32_t (&ct)[16]) const;
 
     // 16 on odd lanes, else 0: the second quad of the 32 bytes that a lane
     // pair stores.  Bits 4-5 of tq0 are (lane & 3) ^ ((lane >> 3) & 3) and
@@ -424,189 +394,151 @@ struct DecoderCtx {
     }
 };
 
+// Page `lane & 15` of page group `group`, of the workgroup.
+__device__ __forceinline__ int group_page(int lane, int group) { return group * kTaskPages + (lane & 15); }
+
+__device__ __forceinline__ void DecoderCtx::load(const Task& k, uint32_t (&ct)[16]) const {
+    const uint64_t* blobs = reinterpret_cast<const uint64_t*>(lds + kLdsPtrs) + 2 * 64;
+    const uint8_t* blob = reinterpret_cast<const uint8_t*>(blobs[group_page(lane, k.group)]);
+    load_block(blob + kHeader + 64u * (uint32_t)(k.block + min(lane >> 4, k.n - 1)), ct);
+}
+
+// Chunks 2 pc, 2 pc + 1 (32 elements, 16 packed hot words) of a decrypted code
+// row pt with the row's parameter words sc.
 template <int DT, int KIND>
-__device__ __forceinline__ void code_task(const DecoderCtx& c, const Task& k, uint32_t (&ct)[16],
-                                          const Task& nxt) {
-    constexpr int GPB = KIND == kSecInt8 ? 4 : (KIND == kSecInt4 ? 8 : 2);
-    constexpr int SW = GPB / 2;  // scale words of this row
+__device__ __forceinline__ void dequant_pair(const uint32_t* pt, const uint32_t* sc, int pc, uint32_t o[16]) {
+    if constexpr (KIND == kSecRaw) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[i] = pt[i];
+    } else if constexpr (KIND == kSecInt8 || KIND == kSecInt4) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int gi = 2 * pc + h;
+            const uint32_t sbits = (gi & 1) ? (sc[gi >> 1] >> 16) : (sc[gi >> 1] & 0xFFFFu);
+            if constexpr (KIND == kSecInt8) dequant_group_int8<DT>(pt + 4 * gi, sbits, o + 8 * h);
+            else dequant_group_int4<DT>(pt + 2 * gi, sbits, o + 8 * h);
+        }
+    } else {
+        dequant_pair_ext<DT, KIND>(pt, sc, pc, o);
+    }
+}
+
+// Four code rows of a unit, for one page group.
+template <int DT, int KIND>
+__device__ __forceinline__ void code_task(const DecoderCtx& c, const Task& k, uint32_t (&ct)[16], const Task& nxt) {
+    constexpr int CH = KIND == kSecRaw ? 2 : ((KIND == kSecInt4 || KIND == kSecInt4G32) ? 8 : 4);  // chunks per row
+    constexpr int SW = KIND == kSecRaw ? 0 : (KIND == kSecInt4 ? 4 : (KIND == kSecAsym8 ? 1 : 2));  // parameter words per row
     const IngressParams& p = *c.p;
     uint32_t* flags = c.lds + kLdsFlags;
-    // ciphertext to the verify wave, at its place in payload order
-    uint32_t* slot = c.lds + (k.mrow % kRing) * kRowWords;
-    wait_ge<kDiagIngressWait, kTmRingWait>(&flags[kFlagMacUsed], k.mrow - kRing + 1, c.wt);
+    const int r = c.lane >> 4, pg = group_page(c.lane, k.group);
+    // ciphertext to the verify wave, at its place in payload order: four
+    // consecutive slots, the last of them the last to become free
+    int32_t slot = k.mrow % kRing + r;
+    slot -= slot >= kRing ? kRing : 0;
+    uint32_t* dst = c.lds + slot * kRowWords;
+    wait_ge<kDiagIngressWait, kTmRingWait>(&flags[kFlagMacUsed], k.mrow + kTaskRows - kRing, c.wt);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-        lds_put_quad_at(slot, c.pq.off[q], make_uint4(ct[4 * q], ct[4 * q + 1], ct[4 * q + 2], ct[4 * q + 3]));
-    publish(&flags[kFlagRing + k.mrow % kRing], (uint32_t)k.mrow + 1u);
-    tm_trace(c.wt.trace, k.mrow, c.wt.t0);
-    // this row is out: the rest of the task runs at the urgency of the next
-    if (nxt.valid) refresh_row_priority(&flags[kFlagMacUsed], task_lead_row(nxt));
+        lds_put_quad(dst, pg, q, make_uint4(ct[4 * q], ct[4 * q + 1], ct[4 * q + 2], ct[4 * q + 3]));
+    if ((c.lane & 15) == 0) publish_lds(&flags[kFlagRing + k.group * kRing + slot], (uint32_t)(k.mrow + r) + 1u);
+    if constexpr (kPhaseTimers) {
+        if (k.group == 0)
+            for (int i = 0; i < kTaskRows; ++i) tm_trace(c.wt.trace, k.mrow + i, c.wt.t0);
+    }
+    // these rows are out: the rest of the task runs at the urgency of the next
+    if (nxt.valid) refresh_row_priority(&flags[kFlagMacUsed], nxt.mrow);
     uint32_t pt[16];
     {
         uint32_t ks[16];
-        chacha_block_cached(p.key, c.nc, 1u + (uint32_t)k.block, c.n0, c.n1, c.n2, ks);
+        table_block(p.key, c.lds + kLdsNonce + pg * kNonceWords, 1u + (uint32_t)(k.block + r), ks);
 #pragma unroll
         for (int i = 0; i < 16; ++i) pt[i] = ct[i] ^ ks[i];
     }
-    if (nxt.valid) load_block(c.pay + 64u * (uint32_t)nxt.block, ct);
-    uint32_t sc[SW];
-    if constexpr (KIND != kSecRaw) {
-        const int slot_s = k.g % kStage;
-        wait_ge<kDiagIngressWait, kTmStageWait>(&flags[kFlagReady + slot_s], k.g + 1, c.wt);
+    if (nxt.valid) c.load(nxt, ct);
+    uint32_t sc[SW > 0 ? SW : 1];
+    if constexpr (SW > 0) {
+        const int slot_s = k.g % kStage, fl = k.group * kStage + slot_s, j = k.j + r;
+        wait_ge<kDiagIngressWait, kTmStageWait>(&flags[kFlagReady + fl], k.g + 1, c.wt);
         const uint32_t* stage = c.lds + kLdsStage + slot_s * kRowWords;
-        if constexpr (KIND == kSecInt8) {  // words 2j, 2j + 1 of the page's scale row
-            const uint32_t* w = stage + quad_word(c.lane, k.j >> 1) + 2 * (k.j & 1);
+        if constexpr (SW == 4) {  // words 4j .. 4j + 3 of the page's scale row
+            const uint4 v = lds_quad(stage, pg, j);
+            sc[0] = v.x; sc[1] = v.y; sc[2] = v.z; sc[3] = v.w;
+        } else if constexpr (SW == 2) {  // words 2j, 2j + 1
+            const uint32_t* w = stage + quad_word(pg, j >> 1) + 2 * (j & 1);
             sc[0] = w[0];
             sc[1] = w[1];
-        } else {  // words 4j .. 4j + 3
-            const uint4 v = lds_quad(stage, c.lane, k.j);
-            sc[0] = v.x; sc[1] = v.y; sc[2] = v.z; sc[3] = v.w;
+        } else {  // word j
+            sc[0] = stage[quad_word(pg, j >> 2) + (j & 3)];
         }
-        // the last code row of the unit to take its scales frees the slot
+        // the last task of the unit to take its scales frees the slot
         uint32_t old = 0;
         if (c.lane == 0)
-            old = __hip_atomic_fetch_add(&flags[kFlagCount + slot_s], 1u, __ATOMIC_ACQ_REL,
-                                         __HIP_MEMORY_SCOPE_WORKGROUP);
+            old = __hip_atomic_fetch_add(&flags[kFlagCount + fl], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
         old = __builtin_amdgcn_readfirstlane(old);
-        if (old == (uint32_t)k.s.nblk - 1u) {
-            flags[kFlagCount + slot_s] = 0u;
-            publish(&flags[kFlagFree + slot_s], (uint32_t)k.g + 1u);
+        if (old == (uint32_t)(k.s.nblk / kTaskRows) - 1u) {
+            flags[kFlagCount + fl] = 0u;
+            publish(&flags[kFlagFree + fl], (uint32_t)k.g + 1u);
         }
     }
-    // output offsets of the row's groups, walked in (vec, group) order
-    GroupCursor cur = group_cursor(k.u * 32 + k.j * GPB, k.s.gpv, k.s.col, p.head_dim);
-    const uint32_t skip = (uint32_t)(p.head_dim - k.s.gpv * 16) * 2u;
-    const bool to_v = k.s.src != 0;
-#pragma unroll
-    for (int pc = 0; pc < GPB / 2; ++pc) {
-        uint32_t o[16];
-        if constexpr (KIND == kSecRaw) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o[i] = pt[i];
-        } else {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int gi = 2 * pc + h;
-                const uint32_t sbits = (gi & 1) ? (sc[gi >> 1] >> 16) : (sc[gi >> 1] & 0xFFFFu);
-                if constexpr (KIND == kSecInt8) dequant_group_int8<DT>(pt + 4 * gi, sbits, o + 8 * h);
-                else dequant_group_int4<DT>(pt + 2 * gi, sbits, o + 8 * h);
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            lds_put_quad_at(c.tile, c.pq.off[q], make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]));
-        const uint32_t off_a = cur.off;
-        cur.step(k.s.gpv, skip);
-        const uint32_t off_b = cur.off;
-        cur.step(k.s.gpv, skip);
-        // lanes 4i, 4i + 1 store the first group's two quads, 4i + 2, 4i + 3 the second's
-        const uint32_t off = ((c.lane & 2) ? off_b : off_a) + c.odd16();
-        const uint64_t* ptab = reinterpret_cast<const uint64_t*>(c.lds + kLdsPtrs) + (to_v ? 64 : 0) + (c.lane >> 2);
-        uint4 x[4];
-        uint8_t* out[4];
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-            x[s4] = lds_quad_at(c.tile, c.tq0 + 1024u * (uint32_t)s4);
-            out[s4] = reinterpret_cast<uint8_t*>(ptab[16 * s4]);
-        }
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) stg16(out[s4] + off, 0, x[s4]);
-    }
-}
-
-// code_task for the extension kinds (family 1): the same steps with the
-// kind's row geometry (ExtRows) and dequantizer.
-template <int DT, int KIND>
-__device__ __forceinline__ void code_task_ext(const DecoderCtx& c, const Task& k, uint32_t (&ct)[16],
-                                              const Task& nxt) {
-    using G = ExtRows<KIND>;
-    const IngressParams& p = *c.p;
-    uint32_t* flags = c.lds + kLdsFlags;
-    uint32_t* slot = c.lds + (k.mrow % kRing) * kRowWords;
-    wait_ge<kDiagIngressWait, kTmRingWait>(&flags[kFlagMacUsed], k.mrow - kRing + 1, c.wt);
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        lds_put_quad_at(slot, c.pq.off[q], make_uint4(ct[4 * q], ct[4 * q + 1], ct[4 * q + 2], ct[4 * q + 3]));
-    publish(&flags[kFlagRing + k.mrow % kRing], (uint32_t)k.mrow + 1u);
-    tm_trace(c.wt.trace, k.mrow, c.wt.t0);
-    // this row is out: the rest of the task runs at the urgency of the next
-    if (nxt.valid) refresh_row_priority(&flags[kFlagMacUsed], task_lead_row(nxt));
-    uint32_t pt[16];
+    // output offset of every row's first chunk, then the rows' chunks walked
+    // in (vec, chunk) order (wave-uniform)
+    GroupCursor cur[kTaskRows];
     {
-        uint32_t ks[16];
-        chacha_block_cached(p.key, c.nc, 1u + (uint32_t)k.block, c.n0, c.n1, c.n2, ks);
+        const uint32_t G0 = (uint32_t)((k.u * k.s.nblk + k.j) * CH);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) pt[i] = ct[i] ^ ks[i];
+        for (int i = 0; i < kTaskRows; ++i) {
+            const uint32_t G = G0 + (uint32_t)(i * CH), vec = div_gpv(k.s, G), g = G - vec * (uint32_t)k.s.gpv;
+            cur[i] = GroupCursor{vec * (uint32_t)p.head_dim * 2u + ((uint32_t)k.s.col + g * 16u) * 2u, (int32_t)g};
+        }
     }
-    if (nxt.valid) load_block(c.pay + 64u * (uint32_t)nxt.block, ct);
-    uint32_t sc[2];
-    const int slot_s = k.g % kStage;
-    wait_ge<kDiagIngressWait, kTmStageWait>(&flags[kFlagReady + slot_s], k.g + 1, c.wt);
-    const uint32_t* stage = c.lds + kLdsStage + slot_s * kRowWords;
-    if constexpr (G::kParamWords == 2) {  // words 2j, 2j + 1 of the page's parameter row
-        const uint32_t* w = stage + quad_word(c.lane, k.j >> 1) + 2 * (k.j & 1);
-        sc[0] = w[0];
-        sc[1] = w[1];
-    } else {  // word j
-        sc[0] = stage[quad_word(c.lane, k.j >> 2) + (k.j & 3)];
-        sc[1] = 0u;
-    }
-    uint32_t old = 0;
-    if (c.lane == 0)
-        old = __hip_atomic_fetch_add(&flags[kFlagCount + slot_s], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-    old = __builtin_amdgcn_readfirstlane(old);
-    if (old == (uint32_t)k.s.nblk - 1u) {
-        flags[kFlagCount + slot_s] = 0u;
-        publish(&flags[kFlagFree + slot_s], (uint32_t)k.g + 1u);
-    }
-    GroupCursor cur = group_cursor((k.u * G::kRowsPerUnit + k.j) * G::kChunks, k.s.gpv, k.s.col, p.head_dim);
     const uint32_t skip = (uint32_t)(p.head_dim - k.s.gpv * 16) * 2u;
-    const bool to_v = k.s.src != 0;
+    const uint64_t* ptab = reinterpret_cast<const uint64_t*>(c.lds + kLdsPtrs) + (k.s.src != 0 ? 64 : 0);
+    uint8_t* out = reinterpret_cast<uint8_t*>(ptab[k.group * kTaskPages + (c.lane >> 2)]);
 #pragma unroll
-    for (int pc = 0; pc < G::kChunks / 2; ++pc) {
+    for (int pc = 0; pc < CH / 2; ++pc) {
         uint32_t o[16];
-        dequant_pair_ext<DT, KIND>(pt, sc, pc, o);
+        dequant_pair<DT, KIND>(pt, sc, pc, o);
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            lds_put_quad_at(c.tile, c.pq.off[q], make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]));
-        const uint32_t off_a = cur.off;
-        cur.step(k.s.gpv, skip);
-        const uint32_t off_b = cur.off;
-        cur.step(k.s.gpv, skip);
-        const uint32_t off = ((c.lane & 2) ? off_b : off_a) + c.odd16();
-        const uint64_t* ptab = reinterpret_cast<const uint64_t*>(c.lds + kLdsPtrs) + (to_v ? 64 : 0) + (c.lane >> 2);
+            lds_put_quad_at(c.tile, c.tq.off[q], make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]));
         uint4 x[4];
-        uint8_t* out[4];
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-            x[s4] = lds_quad_at(c.tile, c.tq0 + 1024u * (uint32_t)s4);
-            out[s4] = reinterpret_cast<uint8_t*>(ptab[16 * s4]);
+        for (int i = 0; i < kTaskRows; ++i) x[i] = lds_quad_at(c.tile, c.tq0 + 1024u * (uint32_t)i);
+        uint8_t* const dst0 = out + c.odd16();
+#pragma unroll
+        for (int i = 0; i < kTaskRows; ++i) {
+            const uint32_t off_a = cur[i].off;
+            cur[i].step(k.s.gpv, skip);
+            const uint32_t off_b = cur[i].off;
+            cur[i].step(k.s.gpv, skip);
+            // lanes 4i, 4i + 1 store the first chunk's two quads, 4i + 2, 4i + 3 the second's
+            stg16(dst0 + ((c.lane & 2) ? off_b : off_a), 0, x[i]);
         }
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) stg16(out[s4] + off, 0, x[s4]);
     }
 }
 
-__device__ __forceinline__ void scale_task(const DecoderCtx& c, const Task& k, uint32_t (&ct)[16],
-                                           const Task& nxt) {
+// The scale rows of a scale group, for one page group: lane 16 r + c decrypts
+// unit u + r of page c.
+__device__ __forceinline__ void scale_task(const DecoderCtx& c, const Task& k, uint32_t (&ct)[16], const Task& nxt) {
     const IngressParams& p = *c.p;
     uint32_t* flags = c.lds + kLdsFlags;
+    const int i = min(c.lane >> 4, k.n - 1), pg = group_page(c.lane, k.group);
     uint32_t sc[16];
     {
         uint32_t ks[16];
-        chacha_block_cached(p.key, c.nc, 1u + (uint32_t)k.block, c.n0, c.n1, c.n2, ks);
+        table_block(p.key, c.lds + kLdsNonce + pg * kNonceWords, 1u + (uint32_t)(k.block + i), ks);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sc[i] = ct[i] ^ ks[i];
+        for (int w = 0; w < 16; ++w) sc[w] = ct[w] ^ ks[w];
     }
-    if (nxt.valid) load_block(c.pay + 64u * (uint32_t)nxt.block, ct);
-    if (params_nonfinite(sc)) flags[kFlagNaN + c.lane] = 1u;
-    const int slot_s = k.g % kStage;
-    wait_ge<kDiagIngressWait, kTmFreeWait>(&flags[kFlagFree + slot_s], k.g - kStage + 1, c.wt);
-    uint32_t* stage = c.lds + kLdsStage + slot_s * kRowWords;
+    if (nxt.valid) c.load(nxt, ct);
+    if (params_nonfinite(sc)) flags[kFlagNaN + pg] = 1u;
+    const int32_t g = k.g + i, fl = k.group * kStage + g % kStage;
+    wait_lanes_ge<kDiagIngressWait, kTmFreeWait>(&flags[kFlagFree + fl], g - kStage + 1, c.wt);
+    uint32_t* stage = c.lds + kLdsStage + (g % kStage) * kRowWords;
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-        lds_put_quad_at(stage, c.pq.off[q], make_uint4(sc[4 * q], sc[4 * q + 1], sc[4 * q + 2], sc[4 * q + 3]));
-    publish(&flags[kFlagReady + slot_s], (uint32_t)k.g + 1u);
+        lds_put_quad(stage, pg, q, make_uint4(sc[4 * q], sc[4 * q + 1], sc[4 * q + 2], sc[4 * q + 3]));
+    publish(&flags[kFlagReady + fl], (uint32_t)g + 1u);
 }
 
 template <int DT, int FAM>
@@ -622,12 +554,12 @@ __device__ __forceinline__ void decode_rows(const DecoderCtx& c, const Layout& l
         used = (int32_t)__builtin_amdgcn_readfirstlane(u);
         return (int32_t)__builtin_amdgcn_readfirstlane(t);
     };
-    const int32_t total = total_tasks(lay);
+    const int32_t total = total_items(lay) * c.ng;
     int32_t t = grab();
-    Task k = task_info<FAM>(lay, t);
+    Task k = task_info(lay, t, c.ng);
     uint32_t ct[16];
     if constexpr (kPhaseTimers) tm_min(c.wt.tm, kTmProdSetup, phase_clock() - c.wt.t0);
-    if (k.valid) load_block(c.pay + 64u * (uint32_t)k.block, ct);
+    if (k.valid) c.load(k, ct);
     // The layout, descriptor and pointer-table reads complete here, before
     // the loop: a load still counted as in flight where the loop begins makes
     // the compiler wait for every outstanding memory operation wherever the
@@ -641,8 +573,8 @@ __device__ __forceinline__ void decode_rows(const DecoderCtx& c, const Layout& l
         if constexpr (kPhaseTimers) {
             if (made++ == 1) tm_min(c.wt.tm, kTmProdFirstRow, phase_clock() - c.wt.t0);
         }
-        set_row_priority(task_lead_row(k) - used);
-        const Task nxt = task_info<FAM>(lay, tn);
+        set_row_priority(k.mrow - used);  // a scale task: its first code row's urgency
+        const Task nxt = task_info(lay, tn, c.ng);
         if (k.scale)
             scale_task(c, k, ct, nxt);
         else if (k.s.kind == kSecInt8)
@@ -653,11 +585,11 @@ __device__ __forceinline__ void decode_rows(const DecoderCtx& c, const Layout& l
             code_task<DT, kSecRaw>(c, k, ct, nxt);
         else if constexpr (FAM == 1) {
             if (k.s.kind == kSecE4m3)
-                code_task_ext<DT, kSecE4m3>(c, k, ct, nxt);
+                code_task<DT, kSecE4m3>(c, k, ct, nxt);
             else if (k.s.kind == kSecInt4G32)
-                code_task_ext<DT, kSecInt4G32>(c, k, ct, nxt);
+                code_task<DT, kSecInt4G32>(c, k, ct, nxt);
             else
-                code_task_ext<DT, kSecAsym8>(c, k, ct, nxt);
+                code_task<DT, kSecAsym8>(c, k, ct, nxt);
         }
         t = tn;
         k = nxt;
@@ -676,18 +608,19 @@ __device__ __forceinline__ void decode_rows(const DecoderCtx& c, const Layout& l
 // from the blob into the ring, in payload order, two rows in flight.  It
 // depends only on the verify wave freeing slots, so the rows before any row
 // it waits for are always in the ring already.
-__device__ __forceinline__ void feed_put(const Waiter& wt, uint32_t* lds, const PageQuads& pq, int32_t r,
+__device__ __forceinline__ void feed_put(const Waiter& wt, uint32_t* lds, const PageQuads& pq, int ng, int32_t r,
                                          const uint4 (&x)[4]) {
     uint32_t* flags = lds + kLdsFlags;
     wait_ge<kDiagIngressWait, kTmFeedWait>(&flags[kFlagMacUsed], r - kRing + 1, wt);
     uint32_t* slot = lds + (r % kRing) * kRowWords;
 #pragma unroll
     for (int q = 0; q < 4; ++q) lds_put_quad_at(slot, pq.off[q], x[q]);
-    publish(&flags[kFlagRing + r % kRing], (uint32_t)r + 1u);
+    const int g = (int)(threadIdx.x & 63);
+    if (g < ng) publish_lds(&flags[kFlagRing + g * kRing + r % kRing], (uint32_t)r + 1u);  // every page group's flag
     tm_trace(wt.trace, r, wt.t0);
 }
 
-__device__ void ingress_feed(const IngressParams& p, uint32_t* lds, const Layout& lay, bool has_lay,
+__device__ void ingress_feed(const IngressParams& p, int ng, uint32_t* lds, const Layout& lay, bool has_lay,
                              const uint8_t* pay, int lane) {
     PageQuads pq;
     pq.init(lane);
@@ -728,11 +661,11 @@ __device__ void ingress_feed(const IngressParams& p, uint32_t* lds, const Layout
     load(rb, b);
 #pragma unroll 1
     for (;;) {
-        feed_put(wt, lds, pq, ra, a);
+        feed_put(wt, lds, pq, ng, ra, a);
         if (rb >= total) break;
         ra = next_fed(rb + 1);
         load(ra, a);
-        feed_put(wt, lds, pq, rb, b);
+        feed_put(wt, lds, pq, ng, rb, b);
         if (ra >= total) break;
         rb = next_fed(ra + 1);
         load(rb, b);
@@ -758,7 +691,7 @@ __device__ __forceinline__ int32_t page_verdict(const IngressParams& p, int64_t 
 // the ring; its last (payload % 64) bytes and the tag are loaded with the
 // header (h0, h1).
 template <bool PAIR>
-__device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t page, uint32_t* lds,
+__device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t page, int ng, uint32_t* lds,
                                                const uint4 h0, const uint4 h1, uint64_t t0) {
     const uint8_t* blob = ingress_blob(p, page);
     const uint8_t* pay = blob + kHeader;
@@ -779,8 +712,9 @@ __device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t p
     st.trace = trace_of(p.timers);
     __builtin_amdgcn_s_waitcnt(0);
     if constexpr (kPhaseTimers) tm_add(st.tm, kTmMacRowsBegin, phase_clock() - t0);
-    mac_rows<kRing, kDiagIngressWait, PAIR>(st, lds, lds + kLdsFlags + kFlagRing, lds + kLdsFlags + kFlagMacUsed, mq, s,
-                                            total);
+    const int group = min(MacQuads<PAIR>::page() / kTaskPages, ng - 1);
+    mac_rows<kRing, kDiagIngressWait, PAIR>(st, lds, lds + kLdsFlags + kFlagRing + group * kRing,
+                                            lds + kLdsFlags + kFlagMacUsed, mq, s, total);
     if constexpr (kPhaseTimers) tm_add(st.tm, kTmMacRowsEnd, phase_clock() - t0);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -911,6 +845,11 @@ __global__ __launch_bounds__(kIngressThreads) void ingress_fused_kernel(IngressP
         uint8_t* v = ingress_v(p, page);
         ptrs[threadIdx.x] = reinterpret_cast<uint64_t>(k);
         ptrs[64 + threadIdx.x] = reinterpret_cast<uint64_t>(v ? v : k);
+        ptrs[2 * 64 + threadIdx.x] = reinterpret_cast<uint64_t>(blob);
+        // nonce from the page's own header (cpp:2357-2365)
+        const uint4 h0 = hdrs[2 * threadIdx.x], h1 = hdrs[2 * threadIdx.x + 1];
+        put_nonce(lds + kLdsNonce + threadIdx.x * kNonceWords, p.key, h1.z, h1.w,
+                  ((h0.w & 0xFFFFu) << 16) | (h0.w >> 16));
     }
     __syncthreads();
     [[maybe_unused]] const uint64_t t0 = phase_clock();
@@ -926,25 +865,21 @@ __global__ __launch_bounds__(kIngressThreads) void ingress_fused_kernel(IngressP
         __builtin_amdgcn_s_setprio(3);
         if (p.ppw <= kPairPages) {
             const int pl = MacQuads<true>::page(), pv = pl < ppw ? pl : 0;
-            const int32_t st = verify_page<true>(p, page0 + pv, lds, hdrs[2 * pv], hdrs[2 * pv + 1], t0);
+            const int32_t st = verify_page<true>(p, page0 + pv, page_groups(ppw), lds, hdrs[2 * pv], hdrs[2 * pv + 1], t0);
             if (MacQuads<true>::reads()) flags[kFlagStatus + pl] = (uint32_t)st;
         } else {
-            flags[kFlagStatus + lane] = (uint32_t)verify_page<false>(p, page, lds, h0, h1, t0);
+            flags[kFlagStatus + lane] = (uint32_t)verify_page<false>(p, page, page_groups(ppw), lds, h0, h1, t0);
         }
     } else if (wave == 4) {
-        ingress_feed(p, lds, lay, has_lay, blob + kHeader, lane);
+        ingress_feed(p, page_groups(ppw), lds, lay, has_lay, blob + kHeader, lane);
     } else if ((wave & 3) != 0 && has_lay) {  // waves 8 and 12 share SIMD 0 and idle
         DecoderCtx c;
         c.p = &p;
-        c.pay = blob + kHeader;
-        c.n0 = h1.z;  // nonce from the page's own header (cpp:2357-2365)
-        c.n1 = h1.w;
-        c.n2 = ((h0.w & 0xFFFFu) << 16) | (h0.w >> 16);
-        c.nc.init(p.key, c.n0, c.n1, c.n2);
         c.lds = lds;
         c.tile = lds + kLdsTile + (wave - 1 - (wave >> 2)) * kRowWords;
         c.lane = lane;
-        c.pq.init(lane);
+        c.ng = page_groups(ppw);
+        c.tq.init(lane);
         c.wt = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, t0);
         c.wt.trace = trace_of(p.timers);
         c.init_stores();

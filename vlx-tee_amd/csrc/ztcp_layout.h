@@ -58,6 +58,7 @@ struct Section {
     uint32_t q_off;      // payload offset of the codes (or raw bytes)
     uint32_t s_off;      // payload offset of the parameters (quantized sections)
     uint32_t bytes;      // section bytes (codes + parameters)
+    uint32_t gmul;       // floor(2^32 / gpv) + 1: divides a chunk index by gpv (div_gpv); 0: not exact
 };
 
 struct Layout {
@@ -110,6 +111,11 @@ ZTCP_HD inline Section make_section(int32_t kind, int32_t src, int32_t col, int3
     const uint32_t code = (uint32_t)s.n_groups * (uint32_t)code_bytes_per_group(kind);
     s.s_off = off + code;
     s.bytes = code + (uint32_t)param_bytes_per_group(kind) * (uint32_t)s.n_groups;
+    // the quotient is exact while index * gpv < 2^32 (the error of the
+    // multiplier is at most gpv); a kernel may look a few vectors past the end
+    const uint64_t chunks = (uint64_t)(vecs + 64) * (uint64_t)(s.gpv > 0 ? s.gpv : 1);
+    s.gmul = (s.gpv > 1 && chunks * (uint64_t)s.gpv < ((uint64_t)1 << 32)) ? (uint32_t)(0xFFFFFFFFu / (uint32_t)s.gpv) + 1u
+                                                                          : 0u;
     return s;
 }
 
@@ -119,7 +125,8 @@ ZTCP_HD inline Section pick(bool c, const Section& x, const Section& y) {
     return Section{c ? x.kind : y.kind,         c ? x.src : y.src,         c ? x.col : y.col,
                    c ? x.gpv : y.gpv,           c ? x.n_groups : y.n_groups,
                    c ? x.unit_begin : y.unit_begin, c ? x.n_units : y.n_units,
-                   c ? x.q_off : y.q_off,       c ? x.s_off : y.s_off,     c ? x.bytes : y.bytes};
+                   c ? x.q_off : y.q_off,       c ? x.s_off : y.s_off,     c ? x.bytes : y.bytes,
+                   c ? x.gmul : y.gmul};
 }
 
 // Number of header-flag layouts: presets 1..6 x RoPE modes 0..3, index
@@ -168,7 +175,7 @@ ZTCP_HD inline bool build_layout(int64_t preset, int64_t rope_mode, int64_t vecs
     const Section c = make_section(kc, 1, 0, pc ? (int32_t)head_dim : 0, vecs, off_c, units_c);
     const uint32_t end = off_c + (pc ? c.bytes : 0u);
     const int32_t units = units_c + (pc ? c.n_units : 0);
-    const Section e{kSecInt8, 0, 0, 0, 0, units, 0, end, end, 0};  // unused slot
+    const Section e{kSecInt8, 0, 0, 0, 0, units, 0, end, end, 0, 0};  // unused slot
     const Section c_or_e = pick(pc, c, e);
     const Section b_or_c = pick(pb, b, c_or_e);
     L.sec[0] = pick(pa, a, b_or_c);

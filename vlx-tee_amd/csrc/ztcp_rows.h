@@ -525,6 +525,38 @@ __device__ __forceinline__ void mac_rows(const Waiter& wt, const uint32_t* ring,
 constexpr int kTaskRows = 4;
 constexpr int kTaskPages = 16;
 
+// Nonce table: per page of the workgroup the nonce (3 words, a pad) and its
+// ChaChaNonceCache.
+constexpr int kNonceWords = 16;
+__device__ __forceinline__ void put_nonce(uint32_t* tab, const ChaKey& key, uint32_t n0, uint32_t n1, uint32_t n2) {
+    ChaChaNonceCache nc;
+    nc.init(key, n0, n1, n2);
+    tab[0] = n0;
+    tab[1] = n1;
+    tab[2] = n2;
+#pragma unroll
+    for (int i = 0; i < 12; ++i) tab[4 + i] = nc.c[i];
+}
+__device__ __forceinline__ void nonce_cache(const uint32_t* tab, ChaChaNonceCache& nc) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(tab + 4 + 4 * q);
+        nc.c[4 * q] = v.x; nc.c[4 * q + 1] = v.y; nc.c[4 * q + 2] = v.z; nc.c[4 * q + 3] = v.w;
+    }
+}
+// Keystream block `ctr` of the page with nonce table entry `tab`.
+__device__ __forceinline__ void table_block(const ChaKey& key, const uint32_t* tab, uint32_t ctr, uint32_t ks[16]) {
+    ChaChaState st;
+    {
+        ChaChaNonceCache nc;
+        nonce_cache(tab, nc);
+        st.start_cached(key, nc, ctr);
+    }
+    st.double_rounds<9>();
+    const u32x4 nn = *reinterpret_cast<const u32x4*>(tab);
+    st.finish(key, ctr, nn.x, nn.y, nn.z, ks);
+}
+
 // Page groups of a workgroup.
 __device__ __forceinline__ int page_groups(int ppw) { return (ppw + kTaskPages - 1) / kTaskPages; }
 
@@ -569,7 +601,14 @@ struct SecRows {
     int32_t qunit_begin;  // units of quantized sections before this one (staging order)
     int32_t gpv, col, src;
     uint32_t q_off, s_off;
+    uint32_t gmul;
 };
+
+// Chunk index -> vector (index / gpv).
+__device__ __forceinline__ uint32_t div_gpv(const SecRows& s, uint32_t g) {
+    if (s.gpv == 1) return g;
+    return s.gmul ? __umulhi(g, s.gmul) : g / (uint32_t)s.gpv;
+}
 
 __device__ __forceinline__ SecRows sec_rows(const Layout& lay, int si, int32_t code_begin, int32_t qunit_begin) {
     SecRows s;
@@ -584,6 +623,7 @@ __device__ __forceinline__ SecRows sec_rows(const Layout& lay, int si, int32_t c
     s.src = ZTCP_SEC_FIELD(lay, si, src);
     s.q_off = ZTCP_SEC_FIELD(lay, si, q_off);
     s.s_off = ZTCP_SEC_FIELD(lay, si, s_off);
+    s.gmul = ZTCP_SEC_FIELD(lay, si, gmul);
     return s;
 }
 
