@@ -14,8 +14,9 @@
 //            decrypts the group's code and scale bytes and dequantizes; then
 //            failing pages are zeroed (per page, or all-or-nothing).
 // Byte-granular loads and stores keep every access in bounds for any
-// alignment.  This path is correct for every geometry the reference accepts;
-// the fused kernels are the fast path.
+// alignment.  This path is correct for every geometry the reference accepts.
+// Pages whose payload fits the LDS take the kernels of ztcp_ragged.hip
+// instead (for ingress two copies of it), so these run for larger ones.
 #include "ztcp_params.h"
 
 namespace ztcp {
@@ -369,6 +370,7 @@ static uint32_t grid_for(int64_t items, int block, int64_t cap = 65536) {
 }
 
 hipError_t launch_egress_generic(const EgressParams& p, int dtype, hipStream_t s) {
+    if (launch_egress_ragged(p, dtype, s)) return hipGetLastError();
     const int64_t nblk = ((int64_t)p.payload + 63) / 64;
     if (nblk > 0) {
         const uint32_t g = grid_for(p.batch * nblk, 256);
@@ -384,15 +386,17 @@ hipError_t launch_egress_generic(const EgressParams& p, int dtype, hipStream_t s
 // `status` must hold p.batch entries (the caller's array or library scratch).
 hipError_t launch_ingress_generic_impl(const IngressParams& p, int dtype, int32_t* status,
                                        hipStream_t s) {
-    hipLaunchKernelGGL(ingress_generic_verify_kernel, dim3(grid_for(p.batch, 64)), dim3(64), 0, s, p,
-                       status);
-    const int64_t gpp = (int64_t)p.n_units;  // groups per page (see host)
-    if (dtype == kHotBf16)
-        hipLaunchKernelGGL(ingress_generic_decode_kernel<kHotBf16>, dim3(grid_for(p.batch * gpp, 256)),
-                           dim3(256), 0, s, p, gpp);
-    else
-        hipLaunchKernelGGL(ingress_generic_decode_kernel<kHotFp16>, dim3(grid_for(p.batch * gpp, 256)),
-                           dim3(256), 0, s, p, gpp);
+    if (!launch_ingress_ragged(p, dtype, status, s)) {
+        hipLaunchKernelGGL(ingress_generic_verify_kernel, dim3(grid_for(p.batch, 64)), dim3(64), 0, s, p,
+                           status);
+        const int64_t gpp = (int64_t)p.n_units;  // groups per page (see host)
+        if (dtype == kHotBf16)
+            hipLaunchKernelGGL(ingress_generic_decode_kernel<kHotBf16>, dim3(grid_for(p.batch * gpp, 256)),
+                               dim3(256), 0, s, p, gpp);
+        else
+            hipLaunchKernelGGL(ingress_generic_decode_kernel<kHotFp16>, dim3(grid_for(p.batch * gpp, 256)),
+                               dim3(256), 0, s, p, gpp);
+    }
     hipLaunchKernelGGL(ingress_generic_zero_kernel, dim3(grid_for(p.page_bytes * p.batch, 256, 8192)),
                        dim3(256), 0, s, p, status, p.per_page ? 0 : 1);
     return hipGetLastError();

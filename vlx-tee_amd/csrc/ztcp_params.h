@@ -187,6 +187,9 @@ __device__ __forceinline__ GroupCursor group_cursor(int32_t G0, int32_t gpv, int
 hipError_t launch_egress_fused(const EgressParams& p, int dtype, hipStream_t s);
 hipError_t launch_ingress_fused(const IngressParams& p, int dtype, hipStream_t s);
 hipError_t launch_egress_generic(const EgressParams& p, int dtype, hipStream_t s);
+// False when a page does not fit the LDS (nothing was launched).
+bool launch_egress_ragged(const EgressParams& p, int dtype, hipStream_t s);
+bool launch_ingress_ragged(const IngressParams& p, int dtype, int32_t* status, hipStream_t s);
 hipError_t launch_egress_zero_blobs(const EgressParams& p, hipStream_t s);
 hipError_t launch_ingress_generic_impl(const IngressParams& p, int dtype, int32_t* status,
                                        hipStream_t s);
