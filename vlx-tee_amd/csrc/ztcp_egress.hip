@@ -89,8 +89,7 @@ constexpr int kLdsBlobs = kLdsFlags + kNumFlags;      // [64] blob pointers (8-b
 constexpr int kLdsHot = (kLdsBlobs + 2 * 64 + 3) & ~3;  // [64] K and V pointers
 constexpr int kLdsNonce = kLdsHot + 4 * 64;           // [64] nonce (3 words, a pad) and its ChaChaNonceCache
 constexpr int kLdsTimers = kLdsNonce + kNonceWords * 64;  // phase-timer counters (timer builds only)
-constexpr int kLdsZero = (kLdsTimers + kTimerLdsWords + 3) & ~3;  // a zero quad: the message of the MAC wave's A lanes
-constexpr int kLdsWords = kLdsZero + 4;
+constexpr int kLdsWords = kLdsTimers + kTimerLdsWords;
 static_assert(kLdsWords * 4 <= 160 * 1024, "LDS budget of one CU");
 static_assert(kRing % 4 == 0 && kRing >= 2 * kTaskRows, "a group's ring flags are aligned; two tasks fit the ring");
 static_assert(kStage >= 3 * kScaleGroup, "the storer keeps one scale group while the producers stage the next two");
@@ -567,7 +566,7 @@ __device__ void egress_mac(const EgressParams& p, int64_t page0, int ppw, uint32
     const uint64_t hdr[4] = {p.hdr0, pg.hdr1, pg.token, pg.seq};
     s.template absorb_words<4>(hdr);
     MacQuads<PAIR> mq;
-    mq.init((uint32_t)kLdsZero * 4u);
+    mq.init();
     MacPlan mp;
     mp.init(p.lay);
     // Rows arrive in MAC order in the ring (code rows from the producers,
@@ -791,7 +790,7 @@ __global__ __launch_bounds__(64 * egress_waves<FAM>()) void egress_fused_kernel(
     const int64_t page0 = (int64_t)blockIdx.x * p.ppw;
     const int ppw = (int)min((int64_t)p.ppw, p.batch - page0);
     for (int i = threadIdx.x; i < kNumFlags; i += blockDim.x) lds[kLdsFlags + i] = 0u;
-    if (threadIdx.x < 4) lds[kLdsZero + threadIdx.x] = 0u;
+    if (p.ppw <= kPairPages) clear_zero_page(lds, kRing);
     tm_clear(lds + kLdsTimers);
     tm_trace_clear(p.timers);
     if (threadIdx.x < 64) {

@@ -75,8 +75,7 @@ constexpr int kLayoutWords = (int)(sizeof(Layout) / 4);
 constexpr int kLdsHeaders = (kLdsLayouts + kNumLayouts * kLayoutWords + 3) & ~3;  // [64] 32-byte headers
 constexpr int kLdsNonce = kLdsHeaders + 64 * 8;      // [64] nonce table
 constexpr int kLdsTimers = kLdsNonce + 64 * kNonceWords;  // phase-timer counters (timer builds only)
-constexpr int kLdsZero = (kLdsTimers + kTimerLdsWords + 3) & ~3;  // a zero quad: the message of the verify wave's A lanes
-constexpr int kLdsWords = kLdsZero + 4;
+constexpr int kLdsWords = kLdsTimers + kTimerLdsWords;
 static_assert(kLdsHeaders % 4 == 0, "header table must be 16-byte aligned");
 static_assert(sizeof(Layout) % 4 == 0, "Layout is copied word by word");
 static_assert(kLdsWords * 4 <= 160 * 1024, "LDS budget of one CU");
@@ -613,9 +612,11 @@ __device__ __forceinline__ void feed_put(const Waiter& wt, uint32_t* lds, const 
     uint32_t* flags = lds + kLdsFlags;
     wait_ge<kDiagIngressWait, kTmFeedWait>(&flags[kFlagMacUsed], r - kRing + 1, wt);
     uint32_t* slot = lds + (r % kRing) * kRowWords;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) lds_put_quad_at(slot, pq.off[q], x[q]);
     const int g = (int)(threadIdx.x & 63);
+    if (g < ng * kTaskPages) {  // never the zero page of the verify wave's A lanes
+#pragma unroll
+        for (int q = 0; q < 4; ++q) lds_put_quad_at(slot, pq.off[q], x[q]);
+    }
     if (g < ng) publish_lds(&flags[kFlagRing + g * kRing + r % kRing], (uint32_t)r + 1u);  // every page group's flag
     tm_trace(wt.trace, r, wt.t0);
 }
@@ -688,8 +689,8 @@ __device__ __forceinline__ int32_t page_verdict(const IngressParams& p, int64_t 
 
 // Verdict of this lane's page (MacQuads::page: with PAIR two lanes per page,
 // both return it), cpp:2313-2355.  The payload's full 64-byte rows come from
-// the ring; its last (payload % 64) bytes and the tag are loaded with the
-// header (h0, h1).
+// the ring; its tag is loaded with the header (h0, h1), its last (payload %
+// 64) bytes after them.
 template <bool PAIR>
 __device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t page, int ng, uint32_t* lds,
                                                const uint4 h0, const uint4 h1, uint64_t t0) {
@@ -698,16 +699,13 @@ __device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t p
     const int32_t total = (int32_t)(p.payload / 64u);
     const uint32_t tail0 = (uint32_t)total * 64u;
     const int ntail = (int)((p.payload - tail0) / 16u);  // 0..3 chunks of 16 bytes
-    uint4 tl[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) tl[i] = ldg16(pay + min(tail0 + 16u * (uint32_t)i, p.payload), 0);
     const uint4 tag = ldg16(pay + p.payload, 0);
     MacHash<PAIR> s;
     s.init(p.mk0, p.mk1);
     const uint64_t hdr[4] = {lo64(h0), hi64(h0), lo64(h1), hi64(h1)};
     s.template absorb_words<4>(hdr);
     MacQuads<PAIR> mq;
-    mq.init((uint32_t)kLdsZero * 4u);
+    mq.init();
     Waiter st = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, t0);
     st.trace = trace_of(p.timers);
     __builtin_amdgcn_s_waitcnt(0);
@@ -716,9 +714,8 @@ __device__ __forceinline__ int32_t verify_page(const IngressParams& p, int64_t p
     mac_rows<kRing, kDiagIngressWait, PAIR>(st, lds, lds + kLdsFlags + kFlagRing + group * kRing,
                                             lds + kLdsFlags + kFlagMacUsed, mq, s, total);
     if constexpr (kPhaseTimers) tm_add(st.tm, kTmMacRowsEnd, phase_clock() - t0);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-        if (i < ntail) s.absorb(tl[i]);
+    // loaded only here: held over the rows, they would not fit the registers
+    for (int i = 0; i < ntail; ++i) s.absorb(ldg16(pay + tail0, i));
     uint64_t lo, hi;
     s.finish((uint64_t)((kHeader + p.payload) & 0xFFu) << 56, lo, hi);
     const uint32_t diff = (tag.x ^ (uint32_t)lo) | (tag.y ^ (uint32_t)(lo >> 32)) |
@@ -833,7 +830,7 @@ __global__ __launch_bounds__(kIngressThreads) void ingress_fused_kernel(IngressP
     if (threadIdx.x < kNumLayouts) layouts[threadIdx.x] = ingress_layout(p, (int)threadIdx.x);
     uint32_t* flags = lds + kLdsFlags;
     for (int i = threadIdx.x; i < kNumFlags; i += blockDim.x) flags[i] = 0u;
-    if (threadIdx.x < 4) lds[kLdsZero + threadIdx.x] = 0u;
+    if (p.ppw <= kPairPages) clear_zero_page(lds, kRing);
     tm_clear(lds + kLdsTimers);
     tm_trace_clear(p.timers);
     if (threadIdx.x < 64) {

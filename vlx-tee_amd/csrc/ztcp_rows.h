@@ -357,14 +357,15 @@ __device__ __forceinline__ uint4 mac_flags4(const uint32_t* ring_flags, int32_t 
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// Whether rows row0 .. row0 + 3 (those below total) are all in the ring.
-// Every lane read the flags of its own page's group: a vector compare and a
-// ballot cost the chain nothing measurable, where v_readfirstlane of a flag cost it about
-// 66 clocks.
-__device__ __forceinline__ bool mac_ready4(const uint4 f, int32_t row0, int32_t total) {
-    const bool ok = ((int32_t)f.x > row0 || row0 >= total) && ((int32_t)f.y > row0 + 1 || row0 + 1 >= total) &&
-                    ((int32_t)f.z > row0 + 2 || row0 + 2 >= total) && ((int32_t)f.w > row0 + 3 || row0 + 3 >= total);
-    return __builtin_amdgcn_ballot_w64(!ok) == 0ull;
+// Whether rows row0 .. row0 + 3 are all in the ring: a slot's flag is the
+// number of the row after it from the time the row is complete until the MAC
+// wave has passed it.  Every lane read the flags of its own page's group: a
+// vector compare and a ballot cost the chain nothing measurable, where
+// v_readfirstlane of a flag cost it about 66 clocks.
+__device__ __forceinline__ bool mac_ready4(const uint4 f, int32_t row0) {
+    const uint32_t r = (uint32_t)row0;
+    const uint32_t late = (f.x ^ (r + 1u)) | (f.y ^ (r + 2u)) | (f.z ^ (r + 3u)) | (f.w ^ (r + 4u));
+    return __builtin_amdgcn_ballot_w64(late != 0u) == 0ull;
 }
 
 // The MAC / verify wave hashes two lanes per page (SipPair) in a workgroup of
@@ -378,36 +379,49 @@ __device__ __forceinline__ bool mac_ready4(const uint4 f, int32_t row0, int32_t 
 constexpr int kPairPages = 32;
 
 // Byte offsets of a MAC lane's four quads inside a row slot.  PAIR: lane 2 i + 1
-// (B) reads page i, the A lanes read the zero quad (`zero_off`, from the
-// ring's start) whatever the slot; else lane = page.
+// (B) reads page i, the A lanes page kZeroPage, whose 64 bytes of every slot
+// are zero (clear_zero_page; a workgroup of up to 32 pages has no such page);
+// else lane = page.
+constexpr int kZeroPage = 63;
 template <bool PAIR>
 struct MacQuads {
     uint32_t off[4];
-    uint32_t slot_mask;
     __device__ __forceinline__ static int page() {
         return (int)(threadIdx.x & 63) >> (PAIR ? 1 : 0);
     }
     __device__ __forceinline__ static bool reads() { return !PAIR || SipPair::lane_b(); }
-    __device__ __forceinline__ void init(uint32_t zero_off) {
+    __device__ __forceinline__ void init() {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) off[q] = reads() ? quad_word(page(), q) * 4u : zero_off;
-        slot_mask = reads() ? ~0u : 0u;
-    }
-    __device__ __forceinline__ uint32_t slot_off(int32_t slot) const {
-        const uint32_t so = (uint32_t)(slot * kRowWords * 4);
-        return PAIR ? so & slot_mask : so;
+        for (int q = 0; q < 4; ++q) off[q] = quad_word(reads() ? page() : kZeroPage, q) * 4u;
     }
 };
+// Every thread of the workgroup, before its first barrier.
+__device__ __forceinline__ void clear_zero_page(uint32_t* ring, int ring_len) {
+    for (int i = threadIdx.x; i < ring_len * 16; i += blockDim.x)
+        ring[(i >> 4) * kRowWords + kZeroPage * 16 + (i & 15)] = 0u;
+}
 template <bool PAIR> struct MacHashOf { using type = Sip; };
 template <> struct MacHashOf<true> { using type = SipPair; };
 template <bool PAIR> using MacHash = typename MacHashOf<PAIR>::type;
 
-template <bool PAIR>
-__device__ __forceinline__ void mac_row_data(const uint32_t* ring, const MacQuads<PAIR>& mq, int32_t slot, uint4 (&x)[4]) {
-    const uint32_t so = mq.slot_off(slot);
+// Row i (0..3) of the group whose slots start at `gs`: the four slots are
+// neighbours, so the group's 16 reads share four addresses (`base`) and
+// differ in the instruction's offset.
+struct MacBase {
+    const char* q[4];
+    template <bool PAIR>
+    __device__ __forceinline__ void set(const uint32_t* ring, const MacQuads<PAIR>& mq, int32_t gs) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) x[q] = lds_quad_at(ring, so + mq.off[q]);
-}
+        for (int i = 0; i < 4; ++i) q[i] = reinterpret_cast<const char*>(ring) + (mq.off[i] + (uint32_t)(gs * kRowWords * 4));
+    }
+    __device__ __forceinline__ void read(int i, uint4 (&x)[4]) const {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(q[k] + i * kRowWords * 4);
+            x[k] = make_uint4(v.x, v.y, v.z, v.w);
+        }
+    }
+};
 
 // Absorbs payload rows [0, total) from a ring of RING slots, four rows per
 // group.  The group's flags are read, then the data of its first two rows,
@@ -427,8 +441,10 @@ __device__ __forceinline__ void mac_rows(const Waiter& wt, const uint32_t* ring,
     uint4 b0[4], b1[4], b2[4], b3[4];
     int32_t gs = 0;  // ring slot of the group's first row
     uint4 fl = mac_flags4(ring_flags, 0);
-    mac_row_data(ring, pq, 0, b0);
-    mac_row_data(ring, pq, 1, b1);
+    MacBase base;
+    base.set(ring, pq, 0);
+    base.read(0, b0);
+    base.read(1, b1);
     [[maybe_unused]] auto traced = [&](int32_t row) {
         if constexpr (kPhaseTimers) {
             if (row == 0) tm_add(wt.tm, kTmMacFirstRow, phase_clock() - wt.t0);
@@ -437,10 +453,12 @@ __device__ __forceinline__ void mac_rows(const Waiter& wt, const uint32_t* ring,
     };
     // A row taken alone: waited for, read, absorbed and released at once.
     auto one_row = [&](int32_t row, int32_t slot, uint64_t& waited) {
+        MacBase one;
+        one.set(ring, pq, slot);
         [[maybe_unused]] const uint64_t t_in = phase_clock();
         wait_lanes_ge<DIAG>(ring_flags + slot, row + 1, wt);
         if constexpr (kPhaseTimers) waited += phase_clock() - t_in;
-        mac_row_data(ring, pq, slot, b2);
+        one.read(0, b2);
         s.absorb64(b2);
         traced(row);
         publish(used, (uint32_t)(row + 1));
@@ -457,22 +475,25 @@ __device__ __forceinline__ void mac_rows(const Waiter& wt, const uint32_t* ring,
     while (r < full) {
 #pragma unroll 1
         for (; r < full; r += kMacGroup) {
-            if (__builtin_expect(!mac_ready4(fl, r, total), 0)) break;
+            if (__builtin_expect(!mac_ready4(fl, r), 0)) break;
             const int32_t ns = gs + kMacGroup == RING ? 0 : gs + kMacGroup;
-            mac_row_data(ring, pq, gs + 2, b2);
+            base.read(2, b2);
             s.absorb64(b0);
             traced(r);
-            mac_row_data(ring, pq, gs + 3, b3);
+            base.read(3, b3);
             s.absorb64(b1);
             traced(r + 1);
             fl = mac_flags4(ring_flags, ns);
-            mac_row_data(ring, pq, ns, b0);
+            base.set(ring, pq, ns);
+            base.read(0, b0);
             s.absorb64(b2);
             traced(r + 2);
-            mac_row_data(ring, pq, ns + 1, b1);
+            base.read(1, b1);
             s.absorb64(b3);
             traced(r + 3);
-            publish(used, (uint32_t)(r + kMacGroup));
+            // the group's reads were issued before this store, and LDS
+            // operations of a wave are performed in order
+            publish_lds(used, (uint32_t)(r + kMacGroup));
             gs = ns;
         }
         if (r >= full) break;
@@ -493,8 +514,9 @@ __device__ __forceinline__ void mac_rows(const Waiter& wt, const uint32_t* ring,
                 tm_trace_put(wt.trace, 2 * kTraceRows + r, (uint32_t)waited);
         }
         fl = mac_flags4(ring_flags, ns);
-        mac_row_data(ring, pq, ns, b0);
-        mac_row_data(ring, pq, ns + 1, b1);
+        base.set(ring, pq, ns);
+        base.read(0, b0);
+        base.read(1, b1);
         gs = ns;
         r += kMacGroup;
     }
