@@ -133,12 +133,13 @@ __device__ __forceinline__ void load_task_half(const EgressParams& p, const uint
     const uint32_t vec0 = div_gpv(row.s, G0);
     // this lane's chunk, counted from the start of the vector of the first
     // row's: at most gpv - 1 + 3 * 8, so past 28 chunks per vector it wraps
-    // at most once, and below gmul is exact (a page holds less than 2^30
-    // elements)
+    // at most once, and below a 16-bit reciprocal is exact.  24-bit
+    // multiplies where the operands allow: a 32-bit one takes four issues.
     uint32_t g = G0 - vec0 * gpv + (threadIdx.x >> 4 & 3u) * (uint32_t)nch;
-    const uint32_t over = gpv > 28u ? (g >= gpv ? 1u : 0u) : (gpv == 1u ? g : __umulhi(g, row.s.gmul));
-    g -= over * gpv;
-    uint32_t off = (vec0 + over) * (uint32_t)p.head_dim * 2u + (uint32_t)row.s.col * 2u + g * 32u;
+    const uint32_t m16 = (row.s.gmul >> 16) + 1u;
+    const uint32_t over = gpv > 28u ? (g >= gpv ? 1u : 0u) : (gpv == 1u ? g : __umul24(g, m16) >> 16);
+    g -= gpv > 28u ? (over ? gpv : 0u) : __umul24(over, gpv);
+    uint32_t off = (vec0 * (uint32_t)p.head_dim + (uint32_t)row.s.col) * 2u + over * ((uint32_t)p.head_dim * 2u) + g * 32u;
     if ((gpv & 3u) == 0u) {  // four contiguous chunks
 #pragma unroll
         for (int i = 0; i < 4; ++i)
