@@ -7,6 +7,7 @@
 // 64-byte keystream blocks and every pointer is 16-byte aligned, otherwise
 // the generic kernels (ztcp_generic.hip).
 #include <atomic>
+#include <cstring>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -30,7 +31,7 @@ constexpr int kCallSlots = 64;
 struct DeviceCtx {
     DeviceState* state = nullptr;      // sticky diagnostics (ztcp_device_diag)
     CallState* calls = nullptr;        // [kCallSlots], device
-    CallState* host_calls = nullptr;   // [kCallSlots], pinned: verdict read-back
+    CallState* host_calls = nullptr;   // [kCallSlots], pinned: where kernels leave a call's verdict for the host
     hipEvent_t done[kCallSlots] = {};
     bool busy[kCallSlots] = {};        // taken by a call
     bool pending[kCallSlots] = {};     // released by an asynchronous call: free once done[k] completes
@@ -64,6 +65,7 @@ int device_ctx(DeviceCtx** out) {
                   hipMalloc(&c->calls, sizeof(CallState) * kCallSlots) == hipSuccess &&
                   hipHostMalloc(&c->host_calls, sizeof(CallState) * kCallSlots, hipHostMallocDefault) == hipSuccess &&
                   hipDeviceGetAttribute(&c->cu_count, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess;
+        if (ok) std::memset(c->host_calls, 0, sizeof(CallState) * kCallSlots);  // no egress tag
         // A slot's event only tells the host that the device is done with the
         // slot's CallState, which only later device work touches: a device-scope
         // release suffices, and spares each asynchronous call the system-scope
@@ -286,20 +288,20 @@ int egress_common(const void* k, const void* v, const int64_t* tok, uint8_t* blo
     int slot = 0;
     rc = acquire_call(ctx, &slot);
     if (rc) return rc;
-    CallState* call = ctx->calls + slot;
     uint32_t tag;
     {
         std::lock_guard<std::mutex> lock(g_mu);
         tag = ctx->egress_tag = ctx->egress_tag == 0xFFFFFFFFu ? 16u : ctx->egress_tag + 1u;
     }
-    p.sink = wait_sink(ctx, call);
+    // The word is in pinned host memory: only an expiry writes it, and a
+    // synchronous call reads it once the stream is done, without a copy
+    // (one page of 114,736 bytes: 932 us with the copy, 910 without).
+    p.sink = wait_sink(ctx, ctx->host_calls + slot);
     p.sink.call_tag = tag;
     p.timers = timer_record(0, (batch + p.ppw - 1) / p.ppw);
     hipError_t e = launch_egress_fused(p, g->hot_dtype, stream);
-    if (e == hipSuccess && !async) e = hipMemcpyAsync(ctx->host_calls + slot, call, sizeof(CallState),
-                                                      hipMemcpyDeviceToHost, stream);
     if (e == hipSuccess && !async) e = hipStreamSynchronize(stream);
-    const bool expired = e == hipSuccess && !async && ctx->host_calls[slot].diag == tag;
+    const bool expired = e == hipSuccess && !async && *(volatile uint32_t*)&ctx->host_calls[slot].diag == tag;
     if (expired) {  // fail closed: every blob of the call is zeroed before the call returns
         e = launch_egress_zero_blobs(p, stream);
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
@@ -395,11 +397,13 @@ int ingress_prepare(const uint8_t* blobs, int64_t blob_bytes, const int64_t* tok
 // finalize, and for a synchronous call the verdict's read-back into
 // `result`.  `status` is the per-page status array of the generic path when
 // the caller gave none (nullptr: a stream-ordered allocation of its own).
+// `result`: pinned memory that a kernel writes (`pinned`), or any host memory.
 hipError_t ingress_enqueue(IngressCall& c, CallState* call, int32_t* status, const WaitSink& sink,
-                           CallState* result, hipStream_t stream) {
+                           CallState* result, bool pinned, hipStream_t stream) {
     IngressParams& p = c.p;
     p.call = call;
     p.sink = sink;
+    p.host_call = pinned && !c.async ? result : nullptr;
     if (p.page_status) status = p.page_status;
     bool own_status = false;
     hipError_t e = launch_reset_call(call, stream);
@@ -410,10 +414,13 @@ hipError_t ingress_enqueue(IngressCall& c, CallState* call, int32_t* status, con
     if (e == hipSuccess) {
         if (c.fast) p.timers = timer_record(1, (p.batch + p.ppw - 1) / p.ppw);
         e = c.fast ? launch_ingress_fused(p, c.dtype, stream) : launch_ingress_generic_impl(p, c.dtype, status, stream);
+        // the finalize kernel also leaves the verdict in p.host_call
         if (e == hipSuccess && c.fast && !p.per_page) e = launch_ingress_finalize(p, stream);
+        else if (e == hipSuccess && p.host_call) e = launch_publish_call(call, p.host_call, stream);
     }
     if (own_status && hipFreeAsync(status, stream) != hipSuccess && e == hipSuccess) e = hipErrorUnknown;
-    if (e == hipSuccess && !c.async) e = hipMemcpyAsync(result, call, sizeof(CallState), hipMemcpyDeviceToHost, stream);
+    if (e == hipSuccess && !c.async && !p.host_call)
+        e = hipMemcpyAsync(result, call, sizeof(CallState), hipMemcpyDeviceToHost, stream);
     if (e == hipSuccess && !c.async) e = hipStreamSynchronize(stream);
     return e;
 }
@@ -439,7 +446,7 @@ int ingress_common(const uint8_t* blobs, int64_t blob_bytes, const int64_t* tok,
     rc = acquire_call(ctx, &slot);
     if (rc) return rc;
     CallState* call = ctx->calls + slot;
-    const hipError_t e = ingress_enqueue(c, call, nullptr, wait_sink(ctx, call), ctx->host_calls + slot, stream);
+    const hipError_t e = ingress_enqueue(c, call, nullptr, wait_sink(ctx, call), ctx->host_calls + slot, true, stream);
     // read the verdict while the slot (and its read-back area) is still ours
     const CallState r = (e == hipSuccess && !c.async) ? ctx->host_calls[slot] : CallState{~0ull, 0u, 0u};
     // a failed launch leaves the slot to an event, as the kernels before it
@@ -603,7 +610,7 @@ int ztcp_ingress_peak_into_noalloc(const uint8_t* cold_blobs, int64_t blob_bytes
     int32_t* status = reinterpret_cast<int32_t*>(d->scratch + kScratchStatusOff);
     CallState result{~0ull, 0u, 0u};  // pageable: the read-back allocates nothing
     const WaitSink sink{&sticky->diag, &call->diag, g_spin_limit.load(std::memory_order_relaxed)};
-    const hipError_t e = ingress_enqueue(c, call, status, sink, &result, (hipStream_t)stream);
+    const hipError_t e = ingress_enqueue(c, call, status, sink, &result, false, (hipStream_t)stream);
     if (e != hipSuccess) return ZTCP_EHIP;
     return c.async ? ZTCP_OK : verdict(result);
 }

@@ -397,7 +397,7 @@ hipError_t launch_ingress_generic_impl(const IngressParams& p, int dtype, int32_
             hipLaunchKernelGGL(ingress_generic_decode_kernel<kHotFp16>, dim3(grid_for(p.batch * gpp, 256)),
                                dim3(256), 0, s, p, gpp);
     }
-    hipLaunchKernelGGL(ingress_generic_zero_kernel, dim3(grid_for(p.page_bytes * p.batch, 256, 8192)),
+    hipLaunchKernelGGL(ingress_generic_zero_kernel, dim3(grid_for(p.page_bytes * p.batch, 256, p.per_page ? 8192 : 1024)),
                        dim3(256), 0, s, p, status, p.per_page ? 0 : 1);
     return hipGetLastError();
 }

@@ -1080,9 +1080,20 @@ void ingress_small_kernel(IngressParams p) {
 
 }  // namespace
 
+// Leaves a call's verdict in pinned host memory: a store at the end of the
+// call instead of a copy behind it (1,200 ragged pages of 2,988 bytes: 104 us
+// with the copy, 98 without).
+__device__ __forceinline__ void publish_call(const CallState* call, CallState* host) {
+    __hip_atomic_store(&host->fail, call->fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&host->diag, call->diag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ void publish_call_kernel(const CallState* call, CallState* host) { publish_call(call, host); }
+
 // All-or-nothing epilogue (cpp:2481-2486): if any page failed, zero both
-// outputs entirely.  Every block reads the failure word once.
+// outputs entirely.  Every block reads the failure word once; the first
+// thread leaves the verdict for the host.
 __global__ void ingress_finalize_kernel(IngressParams p) {
+    if (p.host_call && blockIdx.x == 0 && threadIdx.x == 0) publish_call(p.call, p.host_call);
     if (p.call->fail == ~0ull) return;
     const int64_t n16 = p.page_bytes / 16;
     const int64_t total = n16 * p.batch;
@@ -1131,9 +1142,14 @@ hipError_t launch_ingress_fused(const IngressParams& p, int dtype, hipStream_t s
 hipError_t launch_ingress_finalize(const IngressParams& p, hipStream_t s) {
     const int64_t total = (p.page_bytes / 16) * p.batch;
     int64_t blocks = (total + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
+    if (blocks > 1024) blocks = 1024;  // almost always they find nothing to do (4,096 of them: 4.9 us)
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(ingress_finalize_kernel, dim3((uint32_t)blocks), dim3(256), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_publish_call(const CallState* call, CallState* host, hipStream_t s) {
+    hipLaunchKernelGGL(publish_call_kernel, dim3(1), dim3(1), 0, s, call, host);
     return hipGetLastError();
 }
 

@@ -36,14 +36,15 @@ struct CallState {
 
 // What a bounded wait reports to when it expires.  Ingress or-s its kDiag*
 // bit into the call's diag word (reset by the call's first kernel); egress
-// raises it to the call's tag instead (atomic max of a per-device call
-// counter, never below 16), so the host learns of an expiry in this call
-// without a reset kernel: the word equals the tag only if this call wrote it.
+// stores the call's tag instead (a per-device call counter, never below 16),
+// into pinned host memory, so the host learns of an expiry in this call
+// without a reset kernel or a copy: the word equals the tag only if this
+// call wrote it.
 struct WaitSink {
     uint32_t* dev_diag;        // DeviceState::diag (sticky, per device)
-    uint32_t* call_diag;       // CallState::diag, or nullptr
+    uint32_t* call_diag;       // CallState::diag (egress: in pinned host memory), or nullptr
     uint32_t spin_limit;       // polls before giving up
-    uint32_t call_tag;         // 0: or the kDiag* bit into call_diag; else max it with this tag
+    uint32_t call_tag;         // 0: or the kDiag* bit into call_diag; else store this tag there
 };
 
 struct EgressParams {
@@ -92,6 +93,7 @@ struct IngressParams {
     int32_t per_page;              // zero failing pages in-kernel
     int32_t ppw;
     CallState* call;               // this call's failure word and diagnostics
+    CallState* host_call;          // pinned host copy of it, written by the call's last kernel; may be null
     WaitSink sink;
     unsigned long long* timers;    // phase-timer records, one per workgroup (timer builds; else nullptr)
 };
@@ -195,6 +197,7 @@ hipError_t launch_ingress_generic_impl(const IngressParams& p, int dtype, int32_
                                        hipStream_t s);
 hipError_t launch_ingress_finalize(const IngressParams& p, hipStream_t s);
 hipError_t launch_reset_call(CallState* call, hipStream_t s);
+hipError_t launch_publish_call(const CallState* call, CallState* host, hipStream_t s);
 hipError_t launch_chacha_xor(const uint8_t* src, uint8_t* dst, size_t len, ChaKey key,
                              uint32_t ctr, uint32_t n0, uint32_t n1, uint32_t n2, hipStream_t s);
 hipError_t launch_selftest(unsigned int* bad, hipStream_t s);

@@ -212,7 +212,8 @@ __device__ __forceinline__ void expire(const Waiter& w) {
         if (w.call_diag) {
             // egress calls carry a tag (the host reads the slot back by tag);
             // ingress calls or in their kernel's bit
-            if constexpr (DIAG == kDiagEgressWait) atomicMax(w.call_diag, w.call_tag);
+            if constexpr (DIAG == kDiagEgressWait)
+                __hip_atomic_store(w.call_diag, w.call_tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             else atomicOr(w.call_diag, DIAG);
         }
     }
