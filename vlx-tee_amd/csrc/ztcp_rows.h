@@ -310,11 +310,15 @@ __device__ __forceinline__ void publish_lds(uint32_t* flag, uint32_t value) {
 // handed out in order while the MAC wave consumes them in order, so a row
 // held by a starved wave stalls the chain.  A worker therefore raises its
 // priority by how soon the MAC wave absorbs the row it is making: `lead` =
-// payload row - rows absorbed (wave-uniform).
+// payload row - rows absorbed (wave-uniform; a task's first row).  The bounds
+// suit tasks of four rows: 16,384-page ingress of int8 sections takes
+// 535.1 us with 6 / 12 / 20, 539.6 with 4 / 10 / 18, 549.5 with 3 / 8 / 12
+// and 535.5 with 8 / 14 / 20 (k8v4: 478.0, 479.9, 483.5, 478.4); egress does
+// not feel them.
 __device__ __forceinline__ void set_row_priority(int32_t lead) {
-    if (lead <= 4) __builtin_amdgcn_s_setprio(3);
-    else if (lead <= 10) __builtin_amdgcn_s_setprio(2);
-    else if (lead <= 18) __builtin_amdgcn_s_setprio(1);
+    if (lead <= 6) __builtin_amdgcn_s_setprio(3);
+    else if (lead <= 12) __builtin_amdgcn_s_setprio(2);
+    else if (lead <= 20) __builtin_amdgcn_s_setprio(1);
     else __builtin_amdgcn_s_setprio(0);
 }
 
