@@ -25,9 +25,9 @@
 //     2,900 pages of K8V4_ASYM_G64, 12 a workgroup: 404 and 268), and
 //     the bytes of a page are asked for 512 to 1,024 at a time.
 //   * A storer wave (wave 1, SIMD 1) stores the code rows from the ring to
-//     the blobs, in payload order, four at a time (sixteen lanes per page,
-//     256 contiguous bytes per page), and the encrypted scale rows, four
-//     units at a time, from their staging slots, which it frees.  Producers
+//     the blobs, in payload order, a row at a time (four lanes per page, 64
+//     contiguous bytes of 16 pages per store), and the encrypted scale rows,
+//     four units at a time, from their staging slots, which it frees.  Producers
 //     issue no stores: a wave's wait for its own loads also waits for every
 //     store it issued before them, which exposed the int4 rows' second
 //     loads; and the MAC wave's SIMD is kept free of stores.
@@ -660,11 +660,15 @@ __device__ void egress_scale_feed(const EgressParams& p, int ng, uint32_t* lds) 
 }
 
 // Storer (one wave on SIMD 1): stores the code rows from the ring to the
-// blobs in payload order (the MAC order), the four rows of a task at a time
-// -- sixteen lanes per page, 256 contiguous bytes of four pages per store
+// blobs in payload order (the MAC order), the four rows of a task one after
+// the other -- four lanes per page, 64 contiguous bytes of 16 pages per store
 // instruction -- and publishes `stored` = rows passed; a ring slot is
-// rewritten only once the MAC wave and the storer have both passed it.  The
-// scale rows of a scale group (kScaleGroup units), neighbours in the blob,
+// rewritten only once the MAC wave and the storer have both passed it.
+// (Sixteen lanes per page, 256 bytes of four pages per store, leaves as many
+// lines written in part, reads the ring with four-way bank conflicts, and
+// costs 16,384 MLA pages of int4 467 us against 452, K8V4 444 against 439;
+// blob addresses made per store instead of kept, 12,000 vector instructions
+// a workgroup more.)  The scale rows of a scale group (kScaleGroup units)
 // are stored the same way from their staging slots, which that frees: one
 // scale group behind the code rows, so that the producer that encrypts them
 // has done so, and the last ones at the section's end.
@@ -679,38 +683,30 @@ __device__ void egress_scale_feed(const EgressParams& p, int ng, uint32_t* lds) 
 // own loads would otherwise also wait for every store they issued before
 // those loads.
 struct RowStores {
-    const uint32_t* lds;
-    int ppw;
-    uint32_t pofs;   // this lane's place in the 256 bytes of a page
-    int page, row, quad;
+    uint8_t* blob[4];   // store k: the blob of page 16 k + (lane >> 2) (past the last page page 0's, whose
+                        // bytes those pages' slots hold), at this lane's 16 of a row's 64 bytes
+    uint32_t off;       // byte offset of that quad in a row slot; 16 pages on: + 1,024
+    int ng;
 
-    __device__ __forceinline__ void init(const uint32_t* l, int pages) {
-        const int lane = threadIdx.x & 63;
-        lds = l;
-        ppw = pages;
-        page = lane >> 4;
-        row = lane >> 2 & 3;
-        quad = lane & 3;
-        pofs = (uint32_t)(lane & 15) * 16u;
-    }
-    // Rows in `slot` (this lane's row's, in words) of every page to blob
-    // offset off + row_off.  Past the last page of a partial workgroup a lane
-    // stores page 0's quad again: unconditional stores.
-    __device__ __forceinline__ void store(uint32_t slot, uint32_t off) const {
+    __device__ __forceinline__ void init(const uint32_t* lds, int pages) {
+        const int lane = threadIdx.x & 63, page = lane >> 2, quad = lane & 3;
         const uint64_t* blobs = reinterpret_cast<const uint64_t*>(lds + kLdsBlobs);
-#pragma unroll 1
-        for (int p0 = 0; p0 < ppw; p0 += 16) {
-            uint4 x[4];
-            uint8_t* b[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int pg = p0 + 4 * k + page, pe = pg < ppw ? pg : 0;
-                x[k] = lds_quad(lds + slot, pe, quad);
-                b[k] = reinterpret_cast<uint8_t*>(blobs[pe]);
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) stg16(b[k] + off, 0, x[k]);
+        for (int k = 0; k < 4; ++k) {
+            const int pg = kTaskPages * k + page;
+            blob[k] = reinterpret_cast<uint8_t*>(blobs[pg < pages ? pg : 0]) + 16 * quad;
         }
+        off = quad_word(page, quad) * 4u;
+        ng = page_groups(pages);
+    }
+    // The row in `slot` of every page to blob offset `dst`.
+    __device__ __forceinline__ void store(const uint32_t* slot, uint32_t dst) const {
+        uint4 x[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = lds_quad_at(slot + kTaskPages * 16 * k, off);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k < ng) stg16(blob[k] + dst, 0, x[k]);
     }
 };
 
@@ -730,9 +726,10 @@ __device__ void egress_store_rows(const EgressParams& p, int ppw, uint32_t* lds)
     auto store_scales = [&](int32_t u0, int32_t nu, uint32_t sblk) {
         const int32_t n = min(kScaleGroup, nu - u0), first = g0 + u0;
         wait_lanes_ge<kDiagEgressWait, kTmStorerWait>(&flags[kFlagEnc + fg * kStage + first % kStage], first + 1, wt);
-        const int32_t i = min(rs.row, n - 1);  // lanes past the last unit store its row again
-        rs.store((uint32_t)(kLdsStage + ((first + i) % kStage) * kRowWords),
-                 (uint32_t)kHeader + 64u * (sblk + (uint32_t)(u0 + i)) + 16u * (uint32_t)rs.quad);
+#pragma unroll 1
+        for (int32_t i = 0; i < n; ++i)
+            rs.store(lds + kLdsStage + ((first + i) % kStage) * kRowWords,
+                     (uint32_t)kHeader + 64u * (sblk + (uint32_t)(u0 + i)));
         // the release follows the slot reads
         if (lane < n) publish(&flags[kFlagStage + (first + lane) % kStage], (uint32_t)(first + lane) + 1u);
         made += n;
@@ -764,9 +761,9 @@ __device__ void egress_store_rows(const EgressParams& p, int ppw, uint32_t* lds)
                 pub = made;
             }
             wait_lanes_ge<kDiagEgressWait, kTmStorerWait>(f, want, wt);
-            int32_t ds = r % kRing + rs.row;
-            ds -= ds >= kRing ? kRing : 0;
-            rs.store((uint32_t)(ds * kRowWords), (uint32_t)kHeader + 64u * (uint32_t)r + rs.pofs);
+#pragma unroll 1
+            for (int32_t i = r; i < r + kTaskRows; ++i)
+                rs.store(lds + (i % kRing) * kRowWords, (uint32_t)kHeader + 64u * (uint32_t)i);
             publish(&flags[kFlagStored], (uint32_t)(r + kTaskRows));  // the release orders the slot reads before it
             const int32_t done = (cr + kTaskRows) / nblk;  // whole units stored
             if (quant && done - us >= 2 * kScaleGroup) {
