@@ -4,17 +4,20 @@ A CPU model of egress_fused_kernel and ingress_fused_kernel (workgroups of one
 to four page groups): producers / decoders take tasks in order, one ahead; the
 ring, its flags, the staging slots, their counts and flags are per page group;
 the storer passes four rows at a time and stores a scale group behind the code
-rows; the feeder puts the scale rows; the MAC wave takes rows that every page
-group has filled.  Random interleavings must neither deadlock nor read a slot
-that holds another row.  Sizes come from the kernel sources; planted mistakes
-show that the model sees the faults it is for.
+rows, encrypting it for some page groups of a full workgroup; the feeder puts
+the scale rows; the MAC wave takes rows that every page group has filled.
+Random interleavings must neither deadlock nor read a slot that holds another
+row.  Sizes come from the kernel sources; planted mistakes show that the model
+sees the faults it is for.
 """
+import re
+
 import pytest
 
-
-from test_handoff_model import CONFIGS, NBLK, Sched, _const, check, mac_groups, payload_rows, wait
+from test_handoff_model import CONFIGS, CSRC, NBLK, Sched, _const, check, mac_groups, payload_rows, wait
 
 ROWS = 4
+STORER_SKIPS_ITS_SHARE = False  # planted mistake: the storer stores a scale group without encrypting its share
 STORE_WHOLE_SECTION = False   # planted mistake: the storer stores scale groups only at a section's end
 FREE_ON_FIRST_TASK = False    # planted mistake: a unit's staging slot is freed by its first task
 ONE_GROUP_FLAG = False        # planted mistake: the MAC wave looks at page group 0's flags only
@@ -62,6 +65,12 @@ def code_items(secs, prow):
     return out
 
 
+def producer_scale_groups(ng, nblk):
+    """The kernel's rule of the same name: page groups whose scale rows the producers encrypt."""
+    m = re.search(r"return ng < 4 \? ng : 4 - min\(nblk / (\d+), 4\);", (CSRC / "ztcp_egress.hip").read_text())
+    return ng if ng < 4 else 4 - min(nblk // int(m.group(1)), 4)
+
+
 def egress(secs, n_prod, ng, seed):
     KR, KS, KG = (_const("ztcp_egress.hip", k) for k in ("kRing", "kStage", "kScaleGroup"))
     prow = payload_rows(secs)
@@ -71,6 +80,7 @@ def egress(secs, n_prod, ng, seed):
     stage = [[None] * KS for _ in range(ng)]            # unit whose scales a slot holds
     count = [[0] * KS for _ in range(ng)]
     enc = [[0] * KS for _ in range(ng)]
+    cipher = [set() for _ in range(ng)]                 # units whose staged scales are encrypted
     free = [0] * KS
     scale_stored = set()
 
@@ -96,13 +106,14 @@ def egress(secs, n_prod, ng, seed):
             for i in range(ROWS):
                 ring.flag[g][(m + i) % KR] = m + i + 1
             yield "ok"
-            if quant:
+            if quant and g < producer_scale_groups(ng, NBLK[it["kind"]]):
                 u0 = it["u"] - it["u"] % KG
                 n, g0 = min(KG, it["nu"] - u0), it["g"] - (it["u"] - u0)
                 count[g][g0 % KS] += 1
                 if count[g][g0 % KS] == n * (NBLK[it["kind"]] // ROWS):
                     count[g][g0 % KS] = 0
                     check(all(stage[g][(g0 + i) % KS] == g0 + i for i in range(n)), "encrypts another unit")
+                    cipher[g].update(range(g0, g0 + n))
                     yield "ok"
                     enc[g][g0 % KS] = g0 + 1
                 yield "ok"
@@ -112,24 +123,42 @@ def egress(secs, n_prod, ng, seed):
         made, pub, q = [], 0, 0
         r = 0
 
-        def scales(u0, nu):
-            nonlocal pub
-            n, g0 = min(KG, nu - u0), q + u0
-            yield from wait(lambda: all(enc[g][g0 % KS] >= g0 + 1 for g in range(ng)))
-            check(all(stage[g][(g0 + i) % KS] == g0 + i for g in range(ng) for i in range(n)), "stores another unit")
-            yield "ok"
-            for i in range(n):
-                free[(g0 + i) % KS] = g0 + i + 1
-                made.append(g0 + i)
-            if len(made) - pub >= 2 * KG:
-                scale_stored.update(made[pub:]); pub = len(made)
-            yield "ok"
-
         for kind, nu in secs:
-            us = 0
-            for cr in range(0, nu * NBLK[kind], ROWS):
+            nblk, quant, us = NBLK[kind], kind != "raw", 0
+            ngp = producer_scale_groups(ng, nblk)
+            eg, cr = ngp, 0
+            while True:
+                tail = cr >= nu * nblk
                 rows = range(r, r + ROWS)
                 ready = lambda: all(ring.flag[g][m % KR] >= m + 1 for g in range(ng) for m in rows)  # noqa: E731,B023
+                done = cr // nblk
+                while quant and us < nu and (tail or done - us >= KG):
+                    n, g0 = min(KG, nu - us), q + us
+                    due = tail or (done - us >= 2 * KG and not STORE_WHOLE_SECTION)
+                    if eg < ng and not STORER_SKIPS_ITS_SHARE:
+                        if not due and ready():
+                            break
+                        check(all(stage[eg][(g0 + i) % KS] == g0 + i for i in range(n)), "encrypts another unit")
+                        cipher[eg].update(range(g0, g0 + n))
+                        eg += 1
+                        yield "ok"
+                        continue
+                    if not due:
+                        break
+                    yield from wait(lambda: all(enc[g][g0 % KS] >= g0 + 1 for g in range(ngp)))  # noqa: B023
+                    for g in range(ng):
+                        check(all(stage[g][(g0 + i) % KS] == g0 + i for i in range(n)), "stores another unit")
+                        check(all(g0 + i in cipher[g] for i in range(n)), "stores scales in the clear")
+                    yield "ok"
+                    for i in range(n):
+                        free[(g0 + i) % KS] = g0 + i + 1
+                        made.append(g0 + i)
+                    if len(made) - pub >= 2 * KG:
+                        scale_stored.update(made[pub:]); pub = len(made)
+                    us, eg = us + KG, ngp
+                    yield "ok"
+                if tail:
+                    break
                 if pub < len(made) and not ready():
                     scale_stored.update(made[pub:]); pub = len(made)
                     yield "ok"
@@ -137,15 +166,10 @@ def egress(secs, n_prod, ng, seed):
                 check(all(ring.data[g][m % KR] == prow[m] for g in range(ng) for m in rows), "stores another row", r)
                 yield "ok"
                 r += ROWS
+                cr += ROWS
                 st["stored"] = r
                 yield "ok"
-                if kind != "raw" and (cr + ROWS) // NBLK[kind] - us >= 2 * KG and not STORE_WHOLE_SECTION:
-                    yield from scales(us, nu)
-                    us += KG
-            if kind != "raw":
-                while us < nu:
-                    yield from scales(us, nu)
-                    us += KG
+            if quant:
                 r += nu
                 st["stored"] = r
                 q += nu
@@ -279,6 +303,16 @@ def test_scale_groups_held_to_the_section_end_deadlock():
         assert not all(egress(CONFIGS["k8v4"], 11, 2, s) for s in range(2))
     finally:
         STORE_WHOLE_SECTION = False
+
+
+def test_model_catches_a_storer_that_skips_its_share():
+    global STORER_SKIPS_ITS_SHARE
+    STORER_SKIPS_ITS_SHARE = True
+    try:
+        with pytest.raises(AssertionError, match="in the clear"):
+            egress(CONFIGS["k8v4"], 11, 4, 0)
+    finally:
+        STORER_SKIPS_ITS_SHARE = False
 
 
 def test_model_catches_a_slot_freed_by_the_first_task():

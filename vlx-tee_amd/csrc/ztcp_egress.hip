@@ -18,7 +18,8 @@
 //     stages the scales in LDS, computes the keystream, XORs, and writes the
 //     ciphertext into a ring of row slots in LDS at its place in payload
 //     order.  The task that stages the last scales of four units (a scale
-//     group) encrypts them in their staging slots.
+//     group) encrypts them in their staging slots; in a workgroup of four page
+//     groups the storer does so for some of them.
 //     Four rows of 16 pages instead of one row of 64: a workgroup of a few
 //     pages leaves no lane idle (4,087 MLA pages, 16 a workgroup: 397 us a
 //     row at a time, 256 four rows at a time with the two-lane MAC wave;
@@ -258,14 +259,13 @@ __device__ __forceinline__ uint32_t quant_half_int4g32(const uint32_t (&w)[4][8]
 // their section, n <= kScaleGroup, the first one quantized unit g0) of one
 // page group in their staging slots: lane 16 r + c takes unit u0 + r of page
 // c (lanes past the last unit do the last one's again and write the same).
-// Run by the producer whose task staged the last scales of the group.
-__device__ __forceinline__ void encrypt_scales(const ProducerCtx& c, int group, int32_t n, int32_t g0, uint32_t block0) {
-    const EgressParams& p = *c.p;
-    const int pg = group * kTaskPages + (c.lane & 15);
-    const int32_t i = min(c.lane >> 4, n - 1);
+__device__ __forceinline__ void encrypt_scales(const EgressParams& p, uint32_t* lds, int lane, int group, int32_t n,
+                                               int32_t g0, uint32_t block0) {
+    const int pg = group * kTaskPages + (lane & 15);
+    const int32_t i = min(lane >> 4, n - 1);
     uint32_t ks[16];
-    table_block(p.key, c.lds + kLdsNonce + pg * kNonceWords, 1u + block0 + (uint32_t)i, ks);
-    uint32_t* stage = c.lds + kLdsStage + ((g0 + i) % kStage) * kRowWords;
+    table_block(p.key, lds + kLdsNonce + pg * kNonceWords, 1u + block0 + (uint32_t)i, ks);
+    uint32_t* stage = lds + kLdsStage + ((g0 + i) % kStage) * kRowWords;
     uint4 sw[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) sw[q] = lds_quad(stage, pg, q);
@@ -274,6 +274,20 @@ __device__ __forceinline__ void encrypt_scales(const ProducerCtx& c, int group, 
         lds_put_quad(stage, pg, q,
                      make_uint4(sw[q].x ^ ks[4 * q], sw[q].y ^ ks[4 * q + 1], sw[q].z ^ ks[4 * q + 2],
                                 sw[q].w ^ ks[4 * q + 3]));
+}
+
+// Of the page groups of a workgroup, those whose scale rows the producers
+// encrypt (the first ones; the storer encrypts the others').  A launch of
+// four page groups a workgroup is bound by the vector instructions of SIMDs
+// 1-3, and the storer's wave has time left on SIMD 1: it takes two keystream
+// blocks per four rows that it stores (half of the page groups of int4
+// sections, with a scale row per four code rows, all of them elsewhere).
+// With none of them 16,384 MLA pages take 451 us (int4) and 438 (int4 per
+// 32), with this share 447 and 430; with all of them, where the storer falls
+// behind, the int4 ones take 455.  Below four page groups the hash chain is
+// the bound and the producers have the time.
+__device__ __forceinline__ int producer_scale_groups(int ng, int32_t nblk) {
+    return ng < 4 ? ng : 4 - min(nblk / 2, 4);
 }
 
 // Publishes that scale rows [from, to) are in the blobs, for the feeder.
@@ -436,7 +450,7 @@ __device__ __forceinline__ void code_task(const ProducerCtx& c, const Row& row, 
         if (group == 0)
             for (int i = 0; i < kTaskRows; ++i) tm_trace(c.wt.trace, row.mrow + i, c.wt.t0);
     }
-    if (kind != kSecRaw) {
+    if (kind != kSecRaw && group < producer_scale_groups(c.ng, row.s.nblk)) {
         // the task that stages the last scales of its scale group (for this
         // page group) encrypts them; the storer stores them
         const int32_t u0 = row.u & ~(kScaleGroup - 1), n = min(kScaleGroup, row.s.n_units - u0);
@@ -448,7 +462,7 @@ __device__ __forceinline__ void code_task(const ProducerCtx& c, const Row& row, 
         old = __builtin_amdgcn_readfirstlane(old);
         if (old == (uint32_t)(n * (row.s.nblk / kTaskRows)) - 1u) {
             flags[kFlagCount + group * kStage + g0 % kStage] = 0u;
-            encrypt_scales(c, group, n, g0, row.s.s_off / 64u + (uint32_t)u0);
+            encrypt_scales(p, c.lds, c.lane, group, n, g0, row.s.s_off / 64u + (uint32_t)u0);
             publish_lds(&flags[kFlagEnc + group * kStage + g0 % kStage], (uint32_t)g0 + 1u);
         }
     }
@@ -671,7 +685,9 @@ __device__ void egress_scale_feed(const EgressParams& p, int ng, uint32_t* lds) 
 // a workgroup more.)  The scale rows of a scale group (kScaleGroup units)
 // are stored the same way from their staging slots, which that frees: one
 // scale group behind the code rows, so that the producer that encrypts them
-// has done so, and the last ones at the section's end.
+// has done so, and the last ones at the section's end.  The scale rows of the
+// page groups left to it (producer_scale_groups) this wave encrypts itself,
+// while it would wait for rows, or when the group is due.
 // The waits point backwards only: a scale group is waited for after all of
 // its code rows are stored, so each of its tasks is past its ring wait; the
 // producer of a unit waits for the slot of the unit kStage before it, which
@@ -723,40 +739,62 @@ __device__ void egress_store_rows(const EgressParams& p, int ppw, uint32_t* lds)
     int32_t r = 0, g0 = 0;      // payload row; quantized units before the section
     int32_t made = 0, pub = 0;  // scale rows stored / published as stored
     const int fg = min(lane >> 2 & 3, ng - 1);  // the page group and row this lane's flag stands for
-    auto store_scales = [&](int32_t u0, int32_t nu, uint32_t sblk) {
-        const int32_t n = min(kScaleGroup, nu - u0), first = g0 + u0;
-        wait_lanes_ge<kDiagEgressWait, kTmStorerWait>(&flags[kFlagEnc + fg * kStage + first % kStage], first + 1, wt);
+    // One copy of the code for all sections (a copy of the encryption each
+    // cost 16,384-page launches about 1 %): the section at hand is the first
+    // of three that move up.
+    int32_t kind = p.lay.sec[0].kind, kind1 = p.lay.sec[1].kind, kind2 = p.lay.sec[2].kind;
+    int32_t nu = p.lay.sec[0].n_units, nu1 = p.lay.sec[1].n_units, nu2 = p.lay.sec[2].n_units;
+    uint32_t sblk = p.lay.sec[0].s_off / 64u, sblk1 = p.lay.sec[1].s_off / 64u, sblk2 = p.lay.sec[2].s_off / 64u;
 #pragma unroll 1
-        for (int32_t i = 0; i < n; ++i)
-            rs.store(lds + kLdsStage + ((first + i) % kStage) * kRowWords,
-                     (uint32_t)kHeader + 64u * (sblk + (uint32_t)(u0 + i)));
-        // the release follows the slot reads
-        if (lane < n) publish(&flags[kFlagStage + (first + lane) % kStage], (uint32_t)(first + lane) + 1u);
-        made += n;
-        if (made - pub >= 2 * kScaleGroup) {
-            publish_scales(flags, pub, made);
-            pub = made;
-        }
-    };
-#pragma unroll
-    for (int si = 0; si < 3; ++si) {
-        if (si >= p.lay.n_sec) continue;
-        const int32_t kind = ZTCP_SEC_FIELD(p.lay, si, kind);
-        const int32_t nu = ZTCP_SEC_FIELD(p.lay, si, n_units);
+    for (int si = 0; si < p.lay.n_sec; ++si) {
         const int32_t nblk = code_rows_per_unit(kind);  // 4, 8 or 16
-        const uint32_t sblk = ZTCP_SEC_FIELD(p.lay, si, s_off) / 64u;
         const bool quant = kind != kSecRaw;
+        const int ngp = producer_scale_groups(ng, nblk);
         const int32_t ncode = nu * nblk;
         int32_t us = 0;  // units whose scale rows are stored
+        int eg = ngp;    // next page group of the scale group from unit us on that this wave encrypts
 #pragma unroll 1
-        for (int32_t cr = 0; cr < ncode; cr += kTaskRows, r += kTaskRows) {
+        for (int32_t cr = 0;; cr += kTaskRows, r += kTaskRows) {
+            const bool tail = cr >= ncode;  // no code rows left: the section's last scale groups
             int32_t slot = r % kRing + (lane & 3);
             slot -= slot >= kRing ? kRing : 0;
             const uint32_t* f = &flags[kFlagRing + fg * kRing + slot];
             const int32_t want = r + (lane & 3) + 1;
-            if (pub < made &&
-                __builtin_amdgcn_ballot_w64((int32_t)__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <
-                                            want) != 0ull) {
+            auto ready = [&]() {
+                return __builtin_amdgcn_ballot_w64(
+                           (int32_t)__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < want) == 0ull;
+            };
+            const int32_t done = cr / nblk;  // whole units stored
+#pragma unroll 1
+            while (quant && us < nu && (tail || done - us >= kScaleGroup)) {
+                const int32_t n = min(kScaleGroup, nu - us), first = g0 + us;
+                const bool due = tail || done - us >= 2 * kScaleGroup;
+                if (eg < ng) {  // this wave's share, while the next rows are not there yet or when the group is due
+                    if (!due && ready()) break;
+                    encrypt_scales(p, lds, lane, eg, n, first, sblk + (uint32_t)us);
+                    ++eg;
+                    continue;
+                }
+                if (!due) break;
+                if (ngp > 0)
+                    wait_lanes_ge<kDiagEgressWait, kTmStorerWait>(
+                        &flags[kFlagEnc + min(fg, ngp - 1) * kStage + first % kStage], first + 1, wt);
+#pragma unroll 1
+                for (int32_t i = 0; i < n; ++i)
+                    rs.store(lds + kLdsStage + ((first + i) % kStage) * kRowWords,
+                             (uint32_t)kHeader + 64u * (sblk + (uint32_t)(us + i)));
+                // the release follows the slot reads
+                if (lane < n) publish(&flags[kFlagStage + (first + lane) % kStage], (uint32_t)(first + lane) + 1u);
+                made += n;
+                if (made - pub >= 2 * kScaleGroup) {
+                    publish_scales(flags, pub, made);
+                    pub = made;
+                }
+                us += kScaleGroup;
+                eg = ngp;
+            }
+            if (tail) break;
+            if (pub < made && !ready()) {
                 publish_scales(flags, pub, made);
                 pub = made;
             }
@@ -765,19 +803,15 @@ __device__ void egress_store_rows(const EgressParams& p, int ppw, uint32_t* lds)
             for (int32_t i = r; i < r + kTaskRows; ++i)
                 rs.store(lds + (i % kRing) * kRowWords, (uint32_t)kHeader + 64u * (uint32_t)i);
             publish(&flags[kFlagStored], (uint32_t)(r + kTaskRows));  // the release orders the slot reads before it
-            const int32_t done = (cr + kTaskRows) / nblk;  // whole units stored
-            if (quant && done - us >= 2 * kScaleGroup) {
-                store_scales(us, nu, sblk);
-                us += kScaleGroup;
-            }
         }
         if (quant) {  // the section's scale rows reach the ring through the feeder
-#pragma unroll 1
-            for (; us < nu; us += kScaleGroup) store_scales(us, nu, sblk);
             r += nu;
             publish(&flags[kFlagStored], (uint32_t)r);
             g0 += nu;
         }
+        kind = kind1, kind1 = kind2;
+        nu = nu1, nu1 = nu2;
+        sblk = sblk1, sblk1 = sblk2;
     }
     publish_scales(flags, pub, made);
     if constexpr (kPhaseTimers) tm_max(wt.tm, kTmStorerEnd, phase_clock() - wt.t0);
