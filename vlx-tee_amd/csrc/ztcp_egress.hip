@@ -5,16 +5,16 @@
 // fused_encode_cold_pages_peak_into_cpu (cpp:1904-2004).
 //
 // Work decomposition (one workgroup = up to 64 pages, 16 waves, four per
-// SIMD, or 12 for the int4-per-32 and asym8 kinds):
+// SIMD):
 //   * A "row" is one 64-byte keystream block position of the payload, for all
 //     pages of the workgroup.  Every payload block is exactly one row: a code
 //     row (4 int8 / e4m3 / int4-per-32 groups, 8 int4 groups, 2 raw groups
 //     or 1 asym8 group) or a scale row (the 64 parameter bytes of one unit).
-//   * Eleven producer waves (on SIMDs 1-3; eight in the 12-wave kernels)
-//     take tasks in order from an LDS counter: four consecutive code rows of
-//     a unit for one group of 16 pages, lane = (row, page).  A task
-//     quantizes its groups (loaded a task ahead; the int4 rows four lanes
-//     per page, transposed between the wave's 16-lane rows afterwards),
+//   * Eleven producer waves (on SIMDs 1-3) take tasks in order from an LDS
+//     counter: four consecutive code rows of a unit for one group of 16
+//     pages, lane = (row, page).  A task quantizes its groups (loaded a task
+//     ahead; the int4 rows four lanes per page, transposed between the wave's
+//     16-lane rows afterwards),
 //     stages the scales in LDS, computes the keystream, XORs, and writes the
 //     ciphertext into a ring of row slots in LDS at its place in payload
 //     order.  The task that stages the last scales of four units (a scale
@@ -64,12 +64,11 @@ namespace {
 // 16 waves, four per SIMD, 128 VGPRs each: the MAC wave (0) and the
 // scale-row feeder (4) on SIMD 0 (waves 8 and 12 exit at once: producers
 // there slow the MAC chain down more than they add), the storer (1) and
-// eleven producers on the other three SIMDs.  The kernels of the int4-per-32
-// and asym8 kinds run 12 waves, three per SIMD (eight producers): their
-// quantizers need more than 128 VGPRs, and 168 keep them out of scratch
-// memory.
-template <int FAM>
-constexpr int egress_waves() { return FAM <= 1 ? 16 : 12; }  // family 2's quantizers need 168 VGPRs
+// eleven producers on the other three SIMDs.  (The kernels of the int4-per-32
+// and asym8 kinds ran 12 waves of 168 VGPRs, eight of them producers: 16,384
+// MLA pages of int4 per 32 took 437 us, with 16 waves 420; 24,000 pages of
+// K8V4_ASYM_G64 860 and 794.)
+constexpr int kEgressWaves = 16;
 constexpr int kRing = 24;             // payload rows between their makers and the MAC wave
 constexpr int kStage = 13;            // units whose scales are staged at once
 constexpr int kScaleGroup = 4;        // units whose scale rows are encrypted and stored together
@@ -125,7 +124,24 @@ __device__ __forceinline__ void load_half(const EgressParams& p, const EgressPag
 // page; lane 16 r + c has row r.
 // ---------------------------------------------------------------------------
 
+// This lane's number, and its row (lane / 16) and page (lane % 16) of a task.
+// The asym8 / int4-per-32 kernels (FAM 2) take them from the thread's number
+// where they are used: what the loads derive from them would otherwise be
+// kept over the task loop, in vector registers that those kernels do not have
+// at 16 waves.
+template <int FAM>
+__device__ __forceinline__ uint32_t lane_here() {
+    uint32_t t = threadIdx.x;
+    if constexpr (FAM == 2) asm volatile("" : "+v"(t));
+    return t & 63u;
+}
+template <int FAM>
+__device__ __forceinline__ uint32_t task_row() { return lane_here<FAM>() >> 4; }
+template <int FAM>
+__device__ __forceinline__ int task_page() { return (int)(lane_here<FAM>() & 15u); }
+
 // Hot loads of half h (chunks [4 h, 4 h + 4)) of this lane's own row.
+template <int FAM>
 __device__ __forceinline__ void load_task_half(const EgressParams& p, const uint8_t* src, const Row& row, int h,
                                                uint32_t (&w)[4][8]) {
     const int nch = chunks_per_row(row.s.kind);
@@ -136,7 +152,7 @@ __device__ __forceinline__ void load_task_half(const EgressParams& p, const uint
     // row's: at most gpv - 1 + 3 * 8, so past 28 chunks per vector it wraps
     // at most once, and below a 16-bit reciprocal is exact.  24-bit
     // multiplies where the operands allow: a 32-bit one takes four issues.
-    uint32_t g = G0 - vec0 * gpv + (threadIdx.x >> 4 & 3u) * (uint32_t)nch;
+    uint32_t g = G0 - vec0 * gpv + task_row<FAM>() * (uint32_t)nch;
     const uint32_t m16 = (row.s.gmul >> 16) + 1u;
     const uint32_t over = gpv > 28u ? (g >= gpv ? 1u : 0u) : (gpv == 1u ? g : __umul24(g, m16) >> 16);
     const uint32_t skip = (uint32_t)(p.head_dim - row.s.gpv * 16) * 2u;  // between vectors
@@ -162,6 +178,7 @@ __device__ __forceinline__ void load_task_half(const EgressParams& p, const uint
 // 4 (i / 4) + r of row i % 4 of page c, 64 contiguous bytes of 16 pages;
 // row_untranspose then gives every lane its own row's eight quads.  Needs the
 // half's four chunks contiguous (tq_row).
+template <int FAM>
 __device__ __forceinline__ void load_task_half_t(const EgressParams& p, const uint8_t* src, const Row& row, int h,
                                                  uint32_t (&w)[4][8]) {
     const int32_t per_row = chunks_per_row(row.s.kind) / 4;  // pieces of four chunks
@@ -169,7 +186,7 @@ __device__ __forceinline__ void load_task_half_t(const EgressParams& p, const ui
     const int32_t piece = (row.u * row.s.nblk + row.j) * per_row + h;
     const int32_t vec = (int32_t)div_gpv(row.s, (uint32_t)piece * 4u);
     int32_t gi = piece - vec * gp4;
-    const uint8_t* base = src + (uint32_t)row.s.col * 2u + (threadIdx.x >> 4 & 3u) * 16u;
+    const uint8_t* base = src + (uint32_t)row.s.col * 2u + task_row<FAM>() * 16u;
     // Offsets run on from the first row's instead of being made from (vec,
     // gi) each: the vectors then stay out of vector registers, and a half
     // takes 3 32-bit multiplies and 10 vector instructions less (16,384 k8v4
@@ -206,12 +223,12 @@ __device__ __forceinline__ void row_untranspose(uint32_t (&w)[4][8]) {
 struct ProducerCtx {
     const EgressParams* p;
     uint32_t* lds;
-    int lane;
     int ng;       // page groups of the workgroup
     Waiter wt;
     // Hot buffer (K or V) of this lane's page in page group `group`.
+    template <int FAM>
     __device__ __forceinline__ const uint8_t* hot(int group, int src) const {
-        const uint64_t* t = reinterpret_cast<const uint64_t*>(lds + kLdsHot) + 2 * (group * kTaskPages + (lane & 15));
+        const uint64_t* t = reinterpret_cast<const uint64_t*>(lds + kLdsHot) + 2 * (group * kTaskPages + task_page<FAM>());
         return reinterpret_cast<const uint8_t*>(t[src]);
     }
 };
@@ -341,8 +358,8 @@ __device__ __forceinline__ bool tq_row(const Row& row) {
 template <int FAM>
 __device__ __forceinline__ void load_half_any(const EgressParams& p, const uint8_t* src, const Row& row, int h,
                                               uint32_t (&w)[4][8]) {
-    if (tq_row<FAM>(row)) load_task_half_t(p, src, row, h, w);
-    else load_task_half(p, src, row, h, w);
+    if (tq_row<FAM>(row)) load_task_half_t<FAM>(p, src, row, h, w);
+    else load_task_half<FAM>(p, src, row, h, w);
 }
 
 // The first half of a task's chunks, once they have arrived: quantizes them
@@ -354,7 +371,7 @@ __device__ __forceinline__ void first_half(const ProducerCtx& c, const Row& row,
                                            uint32_t (&w)[4][8], uint32_t (&pt)[16], uint32_t (&sc)[4]) {
     if (tq_row<FAM>(row)) row_untranspose(w);
     quant_first<DT, FAM>(row.s.kind, w, pt, sc);
-    if (two_halves<FAM>(row.s.kind)) load_half_any<FAM>(*c.p, c.hot(group, row.s.src), row, 1, w);
+    if (two_halves<FAM>(row.s.kind)) load_half_any<FAM>(*c.p, c.template hot<FAM>(group, row.s.src), row, 1, w);
 }
 
 // One task.  pt / sc hold its rows' first half quantized (first_half, at
@@ -372,7 +389,7 @@ __device__ __forceinline__ void code_task(const ProducerCtx& c, const Row& row, 
     uint32_t* flags = c.lds + kLdsFlags;
     const uint32_t* used = &flags[kFlagMacUsed];
     const int32_t kind = row.s.kind;
-    const int r = c.lane >> 4, pg = group * kTaskPages + (c.lane & 15);
+    const int r = (int)task_row<FAM>(), pg = group * kTaskPages + task_page<FAM>();
     const uint32_t* tab = c.lds + kLdsNonce + pg * kNonceWords;
     const uint32_t ctr = 1u + (uint32_t)(row.block + r);
     ChaChaState st;
@@ -400,7 +417,7 @@ __device__ __forceinline__ void code_task(const ProducerCtx& c, const Row& row, 
     } else if (FAM == 2 && kind == kSecInt4G32) {
         s2 = quant_half_int4g32<DT>(w, pt + 8);
     }
-    if (nxt.valid) load_half_any<FAM>(p, c.hot(ngroup, nxt.s.src), nxt, 0, w);
+    if (nxt.valid) load_half_any<FAM>(p, c.template hot<FAM>(ngroup, nxt.s.src), nxt, 0, w);
     st.double_rounds<3>();
     pin_words(st.x);
     refresh_row_priority(used, row.mrow);
@@ -445,7 +462,7 @@ __device__ __forceinline__ void code_task(const ProducerCtx& c, const Row& row, 
     for (int q = 0; q < 4; ++q)
         lds_put_quad(dst, pg, q, make_uint4(ks[4 * q], ks[4 * q + 1], ks[4 * q + 2], ks[4 * q + 3]));
     // the MAC wave and the storer take them from here
-    if ((c.lane & 15) == 0) publish_lds(&flags[kFlagRing + group * kRing + slot], (uint32_t)(row.mrow + r) + 1u);
+    if (task_page<FAM>() == 0) publish_lds(&flags[kFlagRing + group * kRing + slot], (uint32_t)(row.mrow + r) + 1u);
     if constexpr (kPhaseTimers) {
         if (group == 0)
             for (int i = 0; i < kTaskRows; ++i) tm_trace(c.wt.trace, row.mrow + i, c.wt.t0);
@@ -456,13 +473,13 @@ __device__ __forceinline__ void code_task(const ProducerCtx& c, const Row& row, 
         const int32_t u0 = row.u & ~(kScaleGroup - 1), n = min(kScaleGroup, row.s.n_units - u0);
         const int32_t g0 = row.g - (row.u - u0);
         uint32_t old = 0;
-        if (c.lane == 0)
+        if (lane_here<FAM>() == 0u)
             old = __hip_atomic_fetch_add(&flags[kFlagCount + group * kStage + g0 % kStage], 1u, __ATOMIC_ACQ_REL,
                                          __HIP_MEMORY_SCOPE_WORKGROUP);
         old = __builtin_amdgcn_readfirstlane(old);
         if (old == (uint32_t)(n * (row.s.nblk / kTaskRows)) - 1u) {
             flags[kFlagCount + group * kStage + g0 % kStage] = 0u;
-            encrypt_scales(p, c.lds, c.lane, group, n, g0, row.s.s_off / 64u + (uint32_t)u0);
+            encrypt_scales(p, c.lds, (int)lane_here<FAM>(), group, n, g0, row.s.s_off / 64u + (uint32_t)u0);
             publish_lds(&flags[kFlagEnc + group * kStage + g0 % kStage], (uint32_t)g0 + 1u);
         }
     }
@@ -473,7 +490,6 @@ template <int DT, int FAM>
 __device__ void egress_produce(const EgressParams& p, int ppw, uint32_t* lds) {
     ProducerCtx c;
     c.p = &p;
-    c.lane = threadIdx.x & 63;
     c.lds = lds;
     c.ng = page_groups(ppw);
     c.wt = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, phase_clock());
@@ -494,7 +510,7 @@ __device__ void egress_produce(const EgressParams& p, int ppw, uint32_t* lds) {
     auto grab = [&]() -> int32_t {
         uint32_t t = 0;
         const uint32_t u = __hip_atomic_load(&flags[kFlagMacUsed], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (c.lane == 0)
+        if (lane_here<FAM>() == 0u)
             t = __hip_atomic_fetch_add(&flags[kFlagTask], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         used = (int32_t)__builtin_amdgcn_readfirstlane(u);
         return (int32_t)__builtin_amdgcn_readfirstlane(t);
@@ -505,7 +521,7 @@ __device__ void egress_produce(const EgressParams& p, int ppw, uint32_t* lds) {
     split_task(t, c.ng, quad, group);
     Row cur = row_info(p.lay, quad * kTaskRows);
     if (cur.valid) {
-        load_half_any<FAM>(p, c.hot(group, cur.s.src), cur, 0, w);
+        load_half_any<FAM>(p, c.template hot<FAM>(group, cur.s.src), cur, 0, w);
         first_half<DT, FAM>(c, cur, group, w, pt, sc);
         if constexpr (kPhaseTimers) tm_min(c.wt.tm, kTmProdLoaded, phase_clock() - c.wt.t0);
     }
@@ -817,13 +833,13 @@ __device__ void egress_store_rows(const EgressParams& p, int ppw, uint32_t* lds)
     if constexpr (kPhaseTimers) tm_max(wt.tm, kTmStorerEnd, phase_clock() - wt.t0);
 }
 
-// FAM 0: the reference's section kinds (int8, int4, raw); FAM 1: also e4m3
-// (16 waves, as FAM 0); FAM 2: also int4 per 32 and asym8, whose 32- and
-// 64-element groups need the most registers (12 waves, 168 VGPRs each).
+// FAM 0: the reference's section kinds (int8, int4, raw); FAM 1: also e4m3;
+// FAM 2: also int4 per 32 and asym8, whose 32- and 64-element groups need the
+// most registers (all 128).
 // Separate instantiations keep each kind's registers out of the kernels of
 // layouts that do not use it.
 template <int DT, int FAM>
-__global__ __launch_bounds__(64 * egress_waves<FAM>()) void egress_fused_kernel(EgressParams p) {
+__global__ __launch_bounds__(64 * kEgressWaves) void egress_fused_kernel(EgressParams p) {
     extern __shared__ __align__(16) uint32_t lds[];
     const int64_t page0 = (int64_t)blockIdx.x * p.ppw;
     const int ppw = (int)min((int64_t)p.ppw, p.batch - page0);
@@ -1162,7 +1178,7 @@ hipError_t launch_egress_fused(const EgressParams& p, int dtype, hipStream_t s) 
         return hipGetLastError();
     }
     const dim3 g((uint32_t)grid),
-        b((uint32_t)(64 * (fam == 0 ? egress_waves<0>() : (fam == 1 ? egress_waves<1>() : egress_waves<2>()))));
+        b((uint32_t)(64 * kEgressWaves));
     if (dtype == kHotBf16) {
         if (fam == 2) hipLaunchKernelGGL((egress_fused_kernel<kHotBf16, 2>), g, b, lds, s, p);
         else if (fam == 1) hipLaunchKernelGGL((egress_fused_kernel<kHotBf16, 1>), g, b, lds, s, p);

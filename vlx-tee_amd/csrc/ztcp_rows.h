@@ -212,9 +212,13 @@ __device__ __forceinline__ void expire(const Waiter& w) {
         if (w.call_diag) {
             // egress calls carry a tag (the host reads the slot back by tag);
             // ingress calls or in their kernel's bit
-            if constexpr (DIAG == kDiagEgressWait)
-                __hip_atomic_store(w.call_diag, w.call_tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            else atomicOr(w.call_diag, DIAG);
+            if constexpr (DIAG == kDiagEgressWait) {
+                uint32_t tag = w.call_tag;
+                asm volatile("" : "+s"(tag));  // moved to a vector register only here, not ahead of the task loop
+                __hip_atomic_store(w.call_diag, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            } else {
+                atomicOr(w.call_diag, DIAG);
+            }
         }
     }
     __hip_atomic_store(w.expired, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
