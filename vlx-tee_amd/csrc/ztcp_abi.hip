@@ -31,7 +31,7 @@ constexpr int kCallSlots = 64;
 struct DeviceCtx {
     DeviceState* state = nullptr;      // sticky diagnostics (ztcp_device_diag)
     CallState* calls = nullptr;        // [kCallSlots], device
-    CallState* host_calls = nullptr;   // [kCallSlots], pinned: where kernels leave a call's verdict for the host
+    CallState* host_calls = nullptr;   // [kCallSlots], pinned: where kernels leave a synchronous call's verdict
     hipEvent_t done[kCallSlots] = {};
     bool busy[kCallSlots] = {};        // taken by a call
     bool pending[kCallSlots] = {};     // released by an asynchronous call: free once done[k] completes
@@ -65,11 +65,13 @@ int device_ctx(DeviceCtx** out) {
                   hipMalloc(&c->calls, sizeof(CallState) * kCallSlots) == hipSuccess &&
                   hipHostMalloc(&c->host_calls, sizeof(CallState) * kCallSlots, hipHostMallocDefault) == hipSuccess &&
                   hipDeviceGetAttribute(&c->cu_count, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess;
-        if (ok) std::memset(c->host_calls, 0, sizeof(CallState) * kCallSlots);  // no egress tag
+        if (ok) std::memset(c->host_calls, 0, sizeof(CallState) * kCallSlots);
         // A slot's event only tells the host that the device is done with the
-        // slot's CallState, which only later device work touches: a device-scope
-        // release suffices, and spares each asynchronous call the system-scope
-        // fence (an L2 writeback and invalidate on every XCD).
+        // slot: its CallState, which only later device work touches, and its
+        // host_calls entry, which kernels write with system-scope stores (done
+        // when the kernel is) and every synchronous call sets anew.  A
+        // device-scope release suffices, and spares each asynchronous call the
+        // system-scope fence (an L2 writeback and invalidate on every XCD).
         for (int i = 0; ok && i < kCallSlots; ++i)
             ok = hipEventCreateWithFlags(&c->done[i], hipEventDisableTiming | hipEventReleaseToDevice) == hipSuccess;
         if (!ok) return ZTCP_EHIP;  // the partial context is left unused (one per device, process lifetime)
@@ -283,30 +285,41 @@ int egress_common(const void* k, const void* v, const int64_t* tok, uint8_t* blo
         if (e == hipSuccess && !async && hipStreamSynchronize(stream) != hipSuccess) return ZTCP_EHIP;
         return e == hipSuccess ? ZTCP_OK : ZTCP_EHIP;
     }
+    // An asynchronous call has no verdict of its own (an expired wait zeroes
+    // the workgroup's headers and sets the sticky diagnostic), so it takes no
+    // slot: kernels that run after the call, a captured graph's replays among
+    // them, never write a word that another call reads.
+    if (async) {
+        p.sink = wait_sink(ctx, nullptr);
+        p.timers = timer_record(0, (batch + p.ppw - 1) / p.ppw);
+        return launch_egress_fused(p, g->hot_dtype, stream) == hipSuccess ? ZTCP_OK : ZTCP_EHIP;
+    }
     // The fused kernel reports an expired bounded wait into this call's slot,
-    // raising its diag word to the call's tag (no reset kernel needed).
+    // setting its diag word to the call's tag (no reset kernel needed).
     int slot = 0;
     rc = acquire_call(ctx, &slot);
     if (rc) return rc;
+    volatile uint32_t* word = &ctx->host_calls[slot].diag;
+    *word = 0u;
     uint32_t tag;
     {
         std::lock_guard<std::mutex> lock(g_mu);
         tag = ctx->egress_tag = ctx->egress_tag == 0xFFFFFFFFu ? 16u : ctx->egress_tag + 1u;
     }
-    // The word is in pinned host memory: only an expiry writes it, and a
-    // synchronous call reads it once the stream is done, without a copy
-    // (one page of 114,736 bytes: 932 us with the copy, 910 without).
+    // The word is in pinned host memory: only an expiry writes it, and the
+    // call reads it once the stream is done, without a copy (one page of
+    // 114,736 bytes: 932 us with the copy, 910 without).
     p.sink = wait_sink(ctx, ctx->host_calls + slot);
     p.sink.call_tag = tag;
     p.timers = timer_record(0, (batch + p.ppw - 1) / p.ppw);
     hipError_t e = launch_egress_fused(p, g->hot_dtype, stream);
-    if (e == hipSuccess && !async) e = hipStreamSynchronize(stream);
-    const bool expired = e == hipSuccess && !async && *(volatile uint32_t*)&ctx->host_calls[slot].diag == tag;
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    const bool expired = e == hipSuccess && *word == tag;
     if (expired) {  // fail closed: every blob of the call is zeroed before the call returns
         e = launch_egress_zero_blobs(p, stream);
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
     }
-    const int rel = release_call(ctx, slot, stream, async || e != hipSuccess);
+    const int rel = release_call(ctx, slot, stream, e != hipSuccess);
     if (e != hipSuccess) return ZTCP_EHIP;
     if (rel) return rel;
     return expired ? ZTCP_EDEVICE : ZTCP_OK;
