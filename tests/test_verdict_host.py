@@ -2,8 +2,9 @@
 
 The host side of the C ABI (ztcp_abi.hip) is linked with a stand-in for the HIP
 runtime and the launchers, whose launches and synchronisations all succeed
-and do only what the test asks for.  An asynchronous egress must not give its
-kernels a word that a later call reads.
+and do only what the test asks for.  A synchronous ingress must then not
+report success unless its verdict was written; an asynchronous egress must
+not give its kernels a word that a later call reads.
 """
 import ctypes as C
 import re
@@ -143,6 +144,22 @@ def _constants():
 
 
 K = _constants()
+
+
+@pytest.mark.parametrize("fn", ["ztcp_ingress_peak_into", "ztcp_ingress_peak_into_noalloc"])
+@pytest.mark.parametrize("per_page", [False, True])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_an_unwritten_verdict_is_no_success(abi, fn, per_page, aligned):
+    geo = GEO if aligned else Geo(7, 3, 80, 16, 0, 0)
+    flags = K["ZTCP_PER_PAGE"] if per_page else 0
+    abi.set_mode(1, 0)
+    for _ in range(70):  # every slot once: a passing verdict left in each
+        assert _ingress(abi, geo, flags, fn=fn) == 0
+    abi.set_mode(2, 0)
+    assert _ingress(abi, geo, flags, fn=fn) == 2
+    abi.set_mode(0, 0)
+    for _ in range(70):
+        assert _ingress(abi, geo, flags, fn=fn) == K["ZTCP_EHIP"]
 
 
 def test_asynchronous_egress_leaves_no_word_behind(abi):

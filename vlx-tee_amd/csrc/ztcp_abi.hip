@@ -406,17 +406,26 @@ int ingress_prepare(const uint8_t* blobs, int64_t blob_bytes, const int64_t* tok
     return ZTCP_OK;
 }
 
+// The verdict of a synchronous call until the device has written it: an error,
+// whatever the launches and the synchronisation said.
+constexpr CallState kUnwritten{0ull, 0xFFFFFFFFu, 0u};
+
 // Enqueues an ingress call whose CallState is `call`: reset, kernels,
 // finalize, and for a synchronous call the verdict's read-back into
 // `result`.  `status` is the per-page status array of the generic path when
 // the caller gave none (nullptr: a stream-ordered allocation of its own).
-// `result`: pinned memory that a kernel writes (`pinned`), or any host memory.
+// `result`: pinned memory that a kernel writes (`pinned`), or any host memory;
+// it is set to the failing kUnwritten first.
 hipError_t ingress_enqueue(IngressCall& c, CallState* call, int32_t* status, const WaitSink& sink,
                            CallState* result, bool pinned, hipStream_t stream) {
     IngressParams& p = c.p;
     p.call = call;
     p.sink = sink;
     p.host_call = pinned && !c.async ? result : nullptr;
+    if (!c.async) {
+        *(volatile uint64_t*)&result->fail = kUnwritten.fail;
+        *(volatile uint32_t*)&result->diag = kUnwritten.diag;
+    }
     if (p.page_status) status = p.page_status;
     bool own_status = false;
     hipError_t e = launch_reset_call(call, stream);
@@ -439,6 +448,7 @@ hipError_t ingress_enqueue(IngressCall& c, CallState* call, int32_t* status, con
 }
 
 int verdict(const CallState& r) {
+    if (r.diag == kUnwritten.diag) return ZTCP_EHIP;
     if (r.diag) return ZTCP_EDEVICE;
     return r.fail == ~0ull ? ZTCP_OK : (int)(r.fail & 0xFFu);
 }
@@ -621,7 +631,7 @@ int ztcp_ingress_peak_into_noalloc(const uint8_t* cold_blobs, int64_t blob_bytes
     CallState* call = reinterpret_cast<CallState*>(d->scratch);
     DeviceState* sticky = reinterpret_cast<DeviceState*>(d->scratch + sizeof(CallState));
     int32_t* status = reinterpret_cast<int32_t*>(d->scratch + kScratchStatusOff);
-    CallState result{~0ull, 0u, 0u};  // pageable: the read-back allocates nothing
+    CallState result = kUnwritten;  // pageable: the read-back allocates nothing
     const WaitSink sink{&sticky->diag, &call->diag, g_spin_limit.load(std::memory_order_relaxed)};
     const hipError_t e = ingress_enqueue(c, call, status, sink, &result, false, (hipStream_t)stream);
     if (e != hipSuccess) return ZTCP_EHIP;
