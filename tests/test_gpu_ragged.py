@@ -1,10 +1,10 @@
 """Pages that are not cut into whole 64-byte units, in the kernels that keep
 their payloads in LDS (ztcp_ragged.hip), and on both sides of the payload
-size past which the layout-agnostic kernels take over.
+sizes and batches past which the layout-agnostic kernels take over.
 
 Every form that path accepts: each section kind, payloads padded to any
 length, blobs and hot pages at odd addresses and strides (descriptors), one
-page per workgroup and several, mixed header flags.  Blobs must equal the
+page per workgroup and several.  Blobs must equal the
 oracle's byte for byte, decoded pages bit for bit, and a flipped bit must give
 the oracle's verdict for its page alone.
 """
@@ -149,3 +149,46 @@ def test_payloads_around_the_lds_limits(hip, O, T):
                                    expected_model_hash=MOD, expected_layer_id=LAYER, **KEYS)
     assert np.array_equal(bits(ko.cpu()).ravel(), np.asarray(ok).ravel())
     assert np.array_equal(bits(vo.cpu()).ravel(), np.asarray(ov).ravel())
+
+
+# last and first batch on each side of the rule (rounds of the pages that fit a
+# CU's LDS at once): egress of 84,240-byte payloads (one fits, 10 rounds), ingress
+# of 75,600 (one, 4 rounds), 32,400 (two, 6) and 23,760 bytes (three, 10)
+@pytest.mark.parametrize("way,T,fit,rounds", [("egress", 39, 1, 10), ("ingress", 35, 1, 4), ("ingress", 15, 2, 6),
+                                              ("ingress", 11, 3, 10)])
+def test_batches_around_the_rule(hip, O, way, T, fit, rounds):
+    H, D, R, preset, rm = 5, 192, 32, 3, 0
+    dev = torch.device("cuda")
+    k, v, _ = _pages(T, 1, T, H, D, R, False, "bf16")
+    exp = O.payload_bytes(preset, rm, T * H, D, R, True)
+    line = torch.cuda.get_device_properties(0).multi_processor_count * fit * rounds
+    for B in (line, line + 1):
+        th = np.arange(B, dtype=np.int64) + 5
+        kd, vd = (t.to(dev).expand(B, -1, -1, -1).contiguous() for t in (k, v))
+        blobs = torch.full((B, 48 + exp), 0xA5, dtype=torch.uint8, device=dev)
+        hip.fused_encode_cold_pages_peak_into(kd, vd, torch.from_numpy(th), blobs, preset, rm, R, exp, TEN, MOD, LAYER,
+                                              HG, BASE, **KEYS)
+        for b in (0, B // 2, B - 1):
+            want = O.egress_batch(bits(k), bits(v), th[b:b + 1], dtype=O.BF16, preset=preset, rope_mode=rm, rope_dim=R,
+                                  expected_payload_bytes=exp, tenant_id_hash=TEN, model_id_hash=MOD, layer_id=LAYER,
+                                  head_group_id=HG, base_sequence_nonce=BASE + b, **KEYS)
+            assert np.array_equal(blobs[b].cpu().numpy(), want[0]), (B, b)
+        if way == "egress":
+            continue
+        _, _, ok, ov = O.ingress_batch(want, th[B - 1:], num_tokens=T, num_heads=H, head_dim=D, rope_dim=R,
+                                       is_mla_single_buffer=False, dtype=O.BF16, expected_tenant_hash=TEN,
+                                       expected_model_hash=MOD, expected_layer_id=LAYER, **KEYS)
+        blobs[B // 3, 40] ^= 1
+        kd.fill_(3.0), vd.fill_(3.0)
+        st = torch.full((B,), -9, dtype=torch.int32, device=dev)
+        with pytest.raises(RuntimeError):
+            hip.fused_decode_cold_pages_peak_into(blobs, torch.from_numpy(th), kd, vd, R, False, TEN, MOD, LAYER,
+                                                  page_status=st, per_page=True, **KEYS)
+        want_st = torch.zeros(B, dtype=torch.int32, device=dev)
+        want_st[B // 3] = 3
+        assert torch.equal(st, want_st)
+        for got, o in ((kd, ok), (vd, ov)):
+            page = torch.from_numpy(np.asarray(o).ravel().view(np.int16).reshape(T, H, D).copy()).to(dev)
+            good = torch.ones(B, dtype=torch.bool, device=dev)
+            good[B // 3] = False
+            assert (got.view(torch.int16)[good] == page).all() and (got[B // 3] == 0).all(), B

@@ -5,7 +5,8 @@
 // ZTCP_EOVERLAP instead of raising.  Each call picks the fused kernels
 // (ztcp_egress.hip / ztcp_ingress.hip) when the page layout is cut into whole
 // 64-byte keystream blocks and every pointer is 16-byte aligned, otherwise
-// the generic kernels (ztcp_generic.hip).
+// the ragged kernels (ztcp_ragged.hip) or, where those do not pay, the
+// layout-agnostic ones (ztcp_generic.hip).
 #include <atomic>
 #include <cstring>
 #include <mutex>
@@ -211,6 +212,13 @@ int pages_per_group(int64_t batch, int cu_count) {
     return (int)ppw;
 }
 
+// What depends on the device's CU count in a call's parameters.
+template <class P>
+void set_cus(P& p, int cu_count) {
+    p.ppw = pages_per_group(p.batch, cu_count);
+    p.cu_count = cu_count > 0 ? cu_count : 1;
+}
+
 int egress_common(const void* k, const void* v, const int64_t* tok, uint8_t* blobs,
                   const ztcp_page_desc* descs, int64_t batch, const ztcp_geometry* g,
                   int64_t preset, int64_t rope_mode, int64_t expected_payload, const ztcp_aad* aad,
@@ -274,7 +282,7 @@ int egress_common(const void* k, const void* v, const int64_t* tok, uint8_t* blo
              ((uint64_t)aad->head_group_id << 48);
     p.nonce2 = ((uint32_t)aad->layer_id << 16) | (uint32_t)aad->head_group_id;  // cpp:108-109
     p.base_seq = base_seq;
-    p.ppw = pages_per_group(batch, ctx->cu_count);
+    set_cus(p, ctx->cu_count);
 
     const bool fast = lay.aligned && expected_payload == (int64_t)lay.required && blob_bytes % 16 == 0 &&
                       (descs || (aligned16(k) && aligned16(v) && aligned16(blobs)));
@@ -397,7 +405,7 @@ int ingress_prepare(const uint8_t* blobs, int64_t blob_bytes, const int64_t* tok
     p.exp_model = model;
     p.exp_layer = layer;
     p.per_page = (flags & ZTCP_PER_PAGE) ? 1 : 0;
-    p.ppw = pages_per_group(batch, cu_count);
+    set_cus(p, cu_count);
     p.n_units = (int32_t)(vecs * (g->head_dim / 16) * (mla ? 1 : 2));  // generic path: groups per page
     out->dtype = g->hot_dtype;
     out->async = (flags & ZTCP_ASYNC) != 0;
@@ -464,7 +472,7 @@ int ingress_common(const uint8_t* blobs, int64_t blob_bytes, const int64_t* tok,
     if (rc) return rc;
     rc = device_ctx(&ctx);
     if (rc) return rc;
-    c.p.ppw = pages_per_group(batch, ctx->cu_count);
+    set_cus(c.p, ctx->cu_count);
     int slot = 0;
     rc = acquire_call(ctx, &slot);
     if (rc) return rc;
@@ -627,7 +635,7 @@ int ztcp_ingress_peak_into_noalloc(const uint8_t* cold_blobs, int64_t blob_bytes
     NoAllocDevice* d = nullptr;
     rc = noalloc_device(&d);
     if (rc) return rc;
-    c.p.ppw = pages_per_group(batch, d->cu_count);
+    set_cus(c.p, d->cu_count);
     CallState* call = reinterpret_cast<CallState*>(d->scratch);
     DeviceState* sticky = reinterpret_cast<DeviceState*>(d->scratch + sizeof(CallState));
     int32_t* status = reinterpret_cast<int32_t*>(d->scratch + kScratchStatusOff);

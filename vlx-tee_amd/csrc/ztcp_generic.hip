@@ -15,8 +15,9 @@
 //            failing pages are zeroed (per page, or all-or-nothing).
 // Byte-granular loads and stores keep every access in bounds for any
 // alignment.  This path is correct for every geometry the reference accepts.
-// Pages whose payload fits the LDS take the kernels of ztcp_ragged.hip
-// instead (for ingress two copies of it), so these run for larger ones.
+// Pages whose payload fits the LDS (for ingress two copies of it) take the
+// kernels of ztcp_ragged.hip instead, except large batches of which few pages
+// fit at once (ragged_pages), so these run for larger pages and those.
 #include "ztcp_params.h"
 
 namespace ztcp {

@@ -67,6 +67,7 @@ struct EgressParams {
     uint32_t nonce2;               // (layer_id << 16) | head_group_id
     uint64_t base_seq;
     int32_t ppw;                   // pages per workgroup
+    int32_t cu_count;              // of the device, at least 1
     WaitSink sink;
     unsigned long long* timers;    // phase-timer records, one per workgroup (timer builds; else nullptr)
 };
@@ -92,6 +93,7 @@ struct IngressParams {
     uint32_t exp_layer;
     int32_t per_page;              // zero failing pages in-kernel
     int32_t ppw;
+    int32_t cu_count;              // of the device, at least 1
     CallState* call;               // this call's failure word and diagnostics
     CallState* host_call;          // pinned host copy of it, written by the call's last kernel; may be null
     WaitSink sink;
@@ -189,7 +191,7 @@ __device__ __forceinline__ GroupCursor group_cursor(int32_t G0, int32_t gpv, int
 hipError_t launch_egress_fused(const EgressParams& p, int dtype, hipStream_t s);
 hipError_t launch_ingress_fused(const IngressParams& p, int dtype, hipStream_t s);
 hipError_t launch_egress_generic(const EgressParams& p, int dtype, hipStream_t s);
-// False when a page does not fit the LDS (nothing was launched).
+// False when the batch is not for these kernels (ragged_pages; nothing was launched).
 bool launch_egress_ragged(const EgressParams& p, int dtype, hipStream_t s);
 bool launch_ingress_ragged(const IngressParams& p, int dtype, int32_t* status, hipStream_t s);
 hipError_t launch_egress_zero_blobs(const EgressParams& p, hipStream_t s);

@@ -14,30 +14,27 @@
 //            the others dequantize the groups of the second.
 // The steps are separated by workgroup barriers, so there are no bounded
 // waits.  What lasts is the SipHash chain of a page, two lanes per page
-// (SipPair): a workgroup holds one page until every SIMD of the chip has one
-// (1,024 workgroups), then more; its hashing wave is another one of its four
-// with every 256 workgroups, so that those of one CU land on different
+// (SipPair): a workgroup holds one page until every SIMD of the chip has one,
+// then more (ragged_pages); its hashing wave is another one of its four with
+// every workgroup per CU, so that those of one CU land on different
 // SIMDs.  Against the layout-agnostic kernels (ztcp_generic.hip: one thread
 // per page and byte loads for the hash, byte arrays in scratch memory for the
 // blocks): 333 pages of 10,708 bytes egress 925 -> 115 us, 1,200 pages of
 // 2,988 bytes ingress 238 -> 104 us.  Those remain for pages that do not fit
-// the LDS and as the definition of the path.
+// the LDS, for batches of many rounds of large pages, and as the definition
+// of the path.
 #include "ztcp_params.h"
+#include "ztcp_ragged.h"
 
 namespace ztcp {
 
 namespace {
 
 constexpr int kRgThreads = 256;
-constexpr int kRgMaxPages = 32;                 // two lanes of the hashing wave per page
 constexpr int kRgZero = 0;                      // [16] zero words: the message of the hashing wave's A lanes
 constexpr int kRgPages = 16;                    // egress: the payloads; ingress: the layouts first
 constexpr int kRgLayoutWords = (int)((sizeof(Layout) / 4 + 4) & ~3);  // Layout, then its index (or -1)
-constexpr size_t kRgLds = 160 * 1024;
-
-// LDS words of one page's payload: 64-byte blocks and a pad of 16 bytes, so
-// that the hashing lanes' rows start at different banks.
-__host__ __device__ inline uint32_t page_words(uint32_t payload) { return (payload + 63u) / 64u * 16u + 4u; }
+static_assert(kRgPages * 4 == (int)kRaggedFixed, "LDS beside the pages");
 
 // 16 bytes at any address (the hardware's unaligned access; never outside the
 // 16 bytes).
@@ -145,14 +142,14 @@ __device__ __forceinline__ void hash_page(SipPair& s, const uint64_t (&hdr)[4], 
 }
 
 // The wave of the workgroup that hashes.
-__device__ __forceinline__ int hash_wave() { return (int)(blockIdx.x >> 8) & 3; }
+__device__ __forceinline__ int hash_wave(int cu_count) { return (int)(blockIdx.x / (uint32_t)cu_count) & 3; }
 
 template <int DT>
 __global__ __launch_bounds__(kRgThreads) void egress_ragged_kernel(EgressParams p) {
     extern __shared__ __align__(16) uint32_t lds[];
     const int64_t page0 = (int64_t)blockIdx.x * p.ppw;
     const int np = (int)min((int64_t)p.ppw, p.batch - page0);
-    const uint32_t stride = page_words(p.payload), nblk = (p.payload + 63u) / 64u;
+    const uint32_t stride = ragged_page_words(p.payload), nblk = (p.payload + 63u) / 64u;
     if (threadIdx.x < 16) lds[kRgZero + threadIdx.x] = 0u;
     // the bytes after the last section (padding, the last block's rest) are zero
     for (int i = 0; i < np; ++i) {
@@ -199,7 +196,7 @@ __global__ __launch_bounds__(kRgThreads) void egress_ragged_kernel(EgressParams 
         }
     }
     __syncthreads();
-    if ((int)(threadIdx.x >> 6) != hash_wave()) return;
+    if ((int)(threadIdx.x >> 6) != hash_wave(p.cu_count)) return;
     __builtin_amdgcn_s_setprio(3);
     const int pl = (int)(threadIdx.x & 63) >> 1;
     const bool b = SipPair::lane_b();
@@ -281,7 +278,7 @@ __global__ __launch_bounds__(kRgThreads) void ingress_ragged_kernel(IngressParam
     extern __shared__ __align__(16) uint32_t lds[];
     const int64_t page0 = (int64_t)blockIdx.x * p.ppw;
     const int np = (int)min((int64_t)p.ppw, p.batch - page0);
-    const uint32_t stride = page_words(p.payload), nblk = (p.payload + 63u) / 64u;
+    const uint32_t stride = ragged_page_words(p.payload), nblk = (p.payload + 63u) / 64u;
     uint32_t* cts = lds + kRgPages + p.ppw * kRgLayoutWords;  // ciphertexts, then plaintexts
     uint32_t* pts = cts + p.ppw * stride;
     if (threadIdx.x < 16) lds[kRgZero + threadIdx.x] = 0u;
@@ -323,7 +320,7 @@ __global__ __launch_bounds__(kRgThreads) void ingress_ragged_kernel(IngressParam
         }
     }
     __syncthreads();
-    const int wave = (int)(threadIdx.x >> 6), hw = hash_wave();
+    const int wave = (int)(threadIdx.x >> 6), hw = hash_wave(p.cu_count);
     if (wave != hw) {  // the other three waves dequantize
         const int t0 = (wave - (wave > hw ? 1 : 0)) * 64 + (int)(threadIdx.x & 63);
         for (int i = 0; i < np; ++i) {
@@ -366,25 +363,14 @@ __global__ __launch_bounds__(kRgThreads) void ingress_ragged_kernel(IngressParam
     if (st != 0) atomicMin(&p.call->fail, ((unsigned long long)page << 8) | (unsigned long long)st);
 }
 
-// Pages per workgroup for `bytes` of LDS per page, 0 when one does not fit
-// (or the batch is beyond what one grid of them holds).
-int ragged_pages(int64_t batch, size_t bytes) {
-    const size_t room = kRgLds - (size_t)kRgPages * 4;
-    if (bytes > room || batch > ((int64_t)1 << 30)) return 0;
-    int64_t n = (batch + 1023) / 1024;
-    if (n > kRgMaxPages) n = kRgMaxPages;
-    if ((size_t)n * bytes > room) n = (int64_t)(room / bytes);
-    return n < 1 ? 1 : (int)n;
-}
-
 }  // namespace
 
-// False when a page does not fit the LDS (the caller then uses the
-// layout-agnostic kernels).
+// False when the batch is not for these kernels (ragged_pages): the caller
+// then uses the layout-agnostic ones.
 bool launch_egress_ragged(const EgressParams& p0, int dtype, hipStream_t s) {
     EgressParams p = p0;
-    const size_t bytes = (size_t)page_words(p.payload) * 4;
-    p.ppw = ragged_pages(p.batch, bytes);
+    const size_t bytes = ragged_page_bytes(p.payload, false, 0);
+    p.ppw = ragged_pages(p.batch, bytes, false, p.cu_count);
     if (p.ppw == 0) return false;
     const dim3 g((uint32_t)((p.batch + p.ppw - 1) / p.ppw)), b(kRgThreads);
     const size_t lds = (size_t)kRgPages * 4 + (size_t)p.ppw * bytes;
@@ -395,8 +381,8 @@ bool launch_egress_ragged(const EgressParams& p0, int dtype, hipStream_t s) {
 
 bool launch_ingress_ragged(const IngressParams& p0, int dtype, int32_t* status, hipStream_t s) {
     IngressParams p = p0;
-    const size_t bytes = (size_t)kRgLayoutWords * 4 + 2 * (size_t)page_words(p.payload) * 4;
-    p.ppw = ragged_pages(p.batch, bytes);
+    const size_t bytes = ragged_page_bytes(p.payload, true, kRgLayoutWords);
+    p.ppw = ragged_pages(p.batch, bytes, true, p.cu_count);
     if (p.ppw == 0) return false;
     const dim3 g((uint32_t)((p.batch + p.ppw - 1) / p.ppw)), b(kRgThreads);
     const size_t lds = (size_t)kRgPages * 4 + (size_t)p.ppw * bytes;
