@@ -4,7 +4,8 @@ sizes and batches past which the layout-agnostic kernels take over.
 
 Every form that path accepts: each section kind, payloads padded to any
 length, blobs and hot pages at odd addresses and strides (descriptors), one
-page per workgroup and several.  Blobs must equal the
+page per workgroup and several, pages of mixed and of invalid header flags in
+one workgroup.  Blobs must equal the
 oracle's byte for byte, decoded pages bit for bit, and a flipped bit must give
 the oracle's verdict for its page alone.
 """
@@ -192,3 +193,38 @@ def test_batches_around_the_rule(hip, O, way, T, fit, rounds):
             good = torch.ones(B, dtype=torch.bool, device=dev)
             good[B // 3] = False
             assert (got.view(torch.int16)[good] == page).all() and (got[B // 3] == 0).all(), B
+
+
+@pytest.mark.parametrize("per_page", [True, False])
+def test_mixed_and_invalid_flags_in_one_workgroup(hip, O, per_page):
+    """Pages of several presets and RoPE modes, padded to one blob size, beside
+    pages of invalid flags, two and three to a workgroup: each by its own header."""
+    T, H, D, R, per = 7, 3, 80, 16, 700
+    modes = [(1, 0), (2, 1), (3, 2)]
+    exp = max(O.payload_bytes(p, m, T * H, D, R, True) for p, m in modes) + 5
+    parts, ths = [], []
+    for i, (preset, rm) in enumerate(modes):
+        k, v, th = _pages(i, per, T, H, D, R, False, "fp16")
+        parts.append(O.egress_batch(bits(k), bits(v), th, dtype=O.FP16, preset=preset, rope_mode=rm, rope_dim=R,
+                                    expected_payload_bytes=exp, tenant_id_hash=TEN, model_id_hash=MOD, layer_id=LAYER,
+                                    head_group_id=HG, base_sequence_nonce=BASE + i * per, **KEYS))
+        ths.append(th)
+    order = np.random.default_rng(0).permutation(3 * per)
+    blobs, th = np.concatenate(parts)[order], np.concatenate(ths)[order]
+    blobs[5, 3] = 0x07    # preset 7: no layout
+    blobs[901, 3] = 0x31  # RoPE mode 3: an extension layout, not asked for here
+    dev = torch.device("cuda")
+    ko = torch.full((3 * per, T, H, D), 7.0, dtype=torch.float16, device=dev)
+    vo = torch.full_like(ko, 7.0)
+    st = torch.full((3 * per,), -9, dtype=torch.int32, device=dev)
+    with pytest.raises(RuntimeError):
+        hip.fused_decode_cold_pages_peak_into(torch.from_numpy(blobs).to(dev), torch.from_numpy(th), ko, vo, R, False, TEN,
+                                              MOD, LAYER, page_status=st, per_page=per_page, **KEYS)
+    _, ost, ok, ov = O.ingress_batch(blobs, th, num_tokens=T, num_heads=H, head_dim=D, rope_dim=R,
+                                     is_mla_single_buffer=False, dtype=O.FP16, expected_tenant_hash=TEN,
+                                     expected_model_hash=MOD, expected_layer_id=LAYER, all_or_nothing=not per_page, **KEYS)
+    ost = np.asarray(ost)
+    assert (ost != 0).sum() == 2 and np.array_equal(st.cpu().numpy(), ost)
+    for got, o in ((ko, ok), (vo, ov)):
+        assert np.array_equal(bits(got.cpu()).ravel(), np.asarray(o).ravel())
+        assert per_page or not got.any()

@@ -4,8 +4,9 @@ The row-pipeline kernels keep every live value in registers: a value the
 register allocator puts in scratch memory is reloaded with a wait for every
 load the wave has in flight, which stalls the producers' and decoders' row
 pipelines.  Their workgroups of 16 waves (four per SIMD) leave each wave 128
-of the SIMD's 512 VGPRs.  This compiles the device code of the two fused
-sources with the library's flags and checks, for every kernel, what the compiler's metadata reports: no
+of the SIMD's 512 VGPRs.  The ragged kernels have four waves a workgroup, and
+several workgroups share a CU.  This compiles the device code of those sources
+with the library's flags and checks, for every kernel, what the compiler's metadata reports: no
 scratch (private segment 0, no VGPR spills) and a VGPR count that fits the
 kernel's waves.
 """
@@ -33,6 +34,7 @@ BUDGET = {
     "ingress_fused_kernelILi0ELi0E": 128, "ingress_fused_kernelILi1ELi0E": 128,
     "ingress_fused_kernelILi0ELi1E": 128, "ingress_fused_kernelILi1ELi1E": 128,
     "egress_small_kernel": 512, "ingress_small_kernel": 512,
+    "egress_ragged_kernel": 128, "ingress_ragged_kernel": 128,
 }
 
 
@@ -61,8 +63,8 @@ def metadata(tmp_path_factory):
         subprocess.run(cmd, check=True, capture_output=True)
         return _kernels(out.read_text())
 
-    with ThreadPoolExecutor(2) as pool:
-        parts = list(pool.map(compile_one, ["ztcp_egress", "ztcp_ingress"]))
+    with ThreadPoolExecutor(3) as pool:
+        parts = list(pool.map(compile_one, ["ztcp_egress", "ztcp_ingress", "ztcp_ragged"]))
     return {k: v for p in parts for k, v in p.items()}
 
 
