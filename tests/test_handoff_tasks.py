@@ -14,13 +14,17 @@ import re
 
 import pytest
 
-from test_handoff_model import CONFIGS, CSRC, NBLK, Sched, _const, check, mac_groups, payload_rows, wait
+import test_handoff_model as M
+from test_handoff_model import CONFIGS, CSRC, NBLK, Bounded, Sched, _const, check, mac_groups, payload_rows, wait
 
 ROWS = 4
 STORER_SKIPS_ITS_SHARE = False  # planted mistake: the storer stores a scale group without encrypting its share
 STORE_WHOLE_SECTION = False   # planted mistake: the storer stores scale groups only at a section's end
 FREE_ON_FIRST_TASK = False    # planted mistake: a unit's staging slot is freed by its first task
 ONE_GROUP_FLAG = False        # planted mistake: the MAC wave looks at page group 0's flags only
+IGNORE_STORER = False         # planted mistake: a ring slot is reused once the MAC wave alone has passed it
+LAZY_PUBLISH = False          # planted mistake: the storer publishes stored scale rows only when it is done
+WHOLE_GROUPS_ONLY = False     # planted mistake: a section's last scale group is stored only if it is whole
 
 
 class AllGroups:
@@ -84,6 +88,9 @@ def egress(secs, n_prod, ng, seed):
     free = [0] * KS
     scale_stored = set()
 
+    def passed():
+        return st["used"] if IGNORE_STORER else min(st["used"], st["stored"])
+
     def producer():
         t = st["task"]; st["task"] += 1
         yield "ok"
@@ -99,7 +106,7 @@ def egress(secs, n_prod, ng, seed):
                 stage[g][u % KS] = u
                 yield "ok"
             m = it["m"]
-            yield from wait(lambda: min(st["used"], st["stored"]) >= m + ROWS - KR)
+            yield from wait(lambda: passed() >= m + ROWS - KR)
             for i in range(ROWS):
                 ring.put(g, m + i, prow[m + i])
             yield "ok"
@@ -134,6 +141,9 @@ def egress(secs, n_prod, ng, seed):
                 done = cr // nblk
                 while quant and us < nu and (tail or done - us >= KG):
                     n, g0 = min(KG, nu - us), q + us
+                    if WHOLE_GROUPS_ONLY and n < KG:
+                        us = nu
+                        break
                     due = tail or (done - us >= 2 * KG and not STORE_WHOLE_SECTION)
                     if eg < ng and not STORER_SKIPS_ITS_SHARE:
                         if not due and ready():
@@ -153,18 +163,19 @@ def egress(secs, n_prod, ng, seed):
                     for i in range(n):
                         free[(g0 + i) % KS] = g0 + i + 1
                         made.append(g0 + i)
-                    if len(made) - pub >= 2 * KG:
+                    if len(made) - pub >= 2 * KG and not LAZY_PUBLISH:
                         scale_stored.update(made[pub:]); pub = len(made)
                     us, eg = us + KG, ngp
                     yield "ok"
                 if tail:
                     break
-                if pub < len(made) and not ready():
+                if pub < len(made) and not ready() and not LAZY_PUBLISH:
                     scale_stored.update(made[pub:]); pub = len(made)
                     yield "ok"
                 yield from wait(ready)
-                check(all(ring.data[g][m % KR] == prow[m] for g in range(ng) for m in rows), "stores another row", r)
-                yield "ok"
+                for m in rows:  # one row after the other
+                    check(all(ring.data[g][m % KR] == prow[m] for g in range(ng)), "stores another row", m)
+                    yield "ok"
                 r += ROWS
                 cr += ROWS
                 st["stored"] = r
@@ -185,7 +196,7 @@ def egress(secs, n_prod, ng, seed):
             if i + 1 < len(rows) and rows[i + 1][0] == m + 1:
                 gn = rows[i + 1][1]
                 yield from wait(lambda: gn in scale_stored)
-            yield from wait(lambda: min(st["used"], st["stored"]) >= m - KR + 1)
+            yield from wait(lambda: passed() >= m - KR + 1)
             for p in range(ng):
                 ring.put(p, m, prow[m])
             yield "ok"
@@ -364,3 +375,100 @@ def test_section_item_order(qpu):
         assert [section_item(i, nsg) for i in range(nu * qpu + nsg)] == section_items(nu, qpu, L)
 
 
+
+
+def _planted(name, run):
+    """run() with the module's planted mistake `name` on."""
+    globals()[name] = True
+    try:
+        return run()
+    finally:
+        globals()[name] = False
+
+
+@pytest.mark.parametrize("name,cfgs", [("LAZY_PUBLISH", ["k8v4"]), ("WHOLE_GROUPS_ONLY", ["tiny", "one_unit_sections"])])
+@pytest.mark.parametrize("ng", [1, 4])
+def test_scale_rows_published_or_stored_too_late_deadlock(name, cfgs, ng):
+    """The feeder, through it the MAC wave and through the ring the producers
+    wait for scale rows that the storer has not published or never stores."""
+    for cfg in cfgs:
+        assert not all(_planted(name, lambda: egress(CONFIGS[cfg], 11, ng, s)) for s in range(3)), cfg  # noqa: B023
+
+
+def test_model_catches_a_slot_reused_before_the_storer_read_it():
+    with pytest.raises(AssertionError, match="stores another row|stores another unit"):
+        for s in range(20):
+            _planted("IGNORE_STORER", lambda: egress(CONFIGS["fp8only"], 11, 1, s))  # noqa: B023
+
+
+def test_model_catches_a_group_read_on_its_first_flag_only():
+    M.MAC_GROUP_OFF = True
+    try:
+        with pytest.raises(AssertionError):
+            for s in range(20):
+                egress(CONFIGS["k8v4"], 11, 1, s)
+    finally:
+        M.MAC_GROUP_OFF = False
+
+
+def _with_stage(n, run):
+    """run() with kStage = n instead of the kernels' (fewer slots than the schedule needs)."""
+    global _const
+    real = _const
+    try:
+        _const = lambda f, name: n if name == "kStage" else real(f, name)  # noqa: E731
+        return run()
+    finally:
+        _const = real
+
+
+@pytest.mark.parametrize("ng", [1, 4])
+def test_a_staging_ring_smaller_than_the_schedule_deadlocks(ng):
+    """Scale groups of four units cannot be staged in fewer than two groups'
+    slots (ingress), nor kept by the storer a group behind (egress)."""
+    assert not _with_stage(3, lambda: ingress(CONFIGS["k8v4"], 12, ng, 0))
+    assert not _with_stage(4, lambda: egress(CONFIGS["k8v4"], 11, ng, 0))
+
+
+def _run_bounded(limit, short_circuit, model):
+    M.BOUND = Bounded(limit, short_circuit)
+    try:
+        done = model()
+        return done, M.BOUND
+    finally:
+        M.BOUND = None
+
+
+@pytest.mark.parametrize("cfg", ["k8v4", "k8v4asym_e4rope"])
+@pytest.mark.parametrize("ng", [1, 4])
+def test_bounded_waits_never_expire_in_a_healthy_workgroup(cfg, ng):
+    for model in (lambda: egress(CONFIGS[cfg], 11, ng, 0), lambda: ingress(CONFIGS[cfg], 12, ng, 0)):
+        done, b = _run_bounded(10**6, True, model)
+        assert done and not b.expired
+
+
+@pytest.mark.parametrize("ng", [1, 4])
+def test_one_expired_wait_ends_every_later_wait_of_the_workgroup(ng):
+    """A planted deadlock (the storer holding back its stored scale rows) with
+    the kernels' bounded waits: the first wait to run out its bound marks the
+    workgroup, every other wait returns at its next poll, and the workgroup
+    finishes after at most one expiry per wave.  Without that rule each later
+    wait spins out its own bound again, so the time to failure grows with the
+    number of waits left (hundreds of bounds per wave in the kernel)."""
+    n_prod, limit = 11, 400
+    waves = n_prod + 3  # producers, storer, feeder, MAC wave
+    for seed in range(2):
+        model = lambda: _planted("LAZY_PUBLISH", lambda: egress(CONFIGS["k8v4"], n_prod, ng, seed))  # noqa: E731,B023
+        done, b = _run_bounded(limit, True, model)
+        assert done and b.expired
+        assert 1 <= b.expiries <= waves
+        assert b.polls <= waves * limit
+        done, old = _run_bounded(limit, False, model)
+        assert done and old.expiries > 2 * waves
+        assert old.polls > 2 * waves * limit
+
+
+def test_one_expired_wait_ends_a_broken_ingress_workgroup():
+    for seed in range(2):
+        done, b = _run_bounded(400, True, lambda: _with_stage(3, lambda: ingress(CONFIGS["k8v4"], 12, 1, seed)))  # noqa: B023
+        assert done and b.expired and 1 <= b.expiries <= 14
