@@ -2,10 +2,11 @@
 // egress and ingress kernels.
 //
 // A row is one 64-byte keystream block position of the payload, for all pages
-// of a workgroup (lane = page).  Row slots in LDS hold 16 words per page; the
-// 16-byte quads of a page are XOR-swizzled so that both lane-per-page access
-// and the transposed four-lanes-per-page access used for coalesced global
-// stores are free of bank conflicts.
+// of a workgroup; workers take four rows of 16 pages at a time, lane = (row,
+// page).  Row slots in LDS hold 16 words per page; the 16-byte quads of a page
+// are XOR-swizzled so that both lane-per-page access and the transposed
+// four-lanes-per-page access used for coalesced global stores are free of
+// bank conflicts.
 #pragma once
 
 #include "ztcp_params.h"
@@ -83,7 +84,7 @@ enum TimerSlot : int {
     kTmStorerEnd = 29,     // egress storer: done
     kTmFeedEnd = 30,       // feeder: done
     kTmProdWaves = 31,     // producer / decoder waves that ran
-    kTmRows = 32,          // rows made by producers / decoders
+    kTmRows = 32,          // tasks (four rows of 16 pages) made by producers / decoders
     kTmProdSetup = 33,     // earliest producer / decoder done with its page setup (descriptor, nonce cache)
     kTmProdLoaded = 34,    // earliest producer / decoder holding its first row's data (egress: quantized)
     // written to the record by thread 0 directly
