@@ -224,7 +224,7 @@ struct ProducerCtx {
     const EgressParams* p;
     uint32_t* lds;
     int ng;       // page groups of the workgroup
-    Waiter wt;
+    LateTagWaiter wt;
     // Hot buffer (K or V) of this lane's page in page group `group`.
     template <int FAM>
     __device__ __forceinline__ const uint8_t* hot(int group, int src) const {
@@ -492,7 +492,7 @@ __device__ void egress_produce(const EgressParams& p, int ppw, uint32_t* lds) {
     c.p = &p;
     c.lds = lds;
     c.ng = page_groups(ppw);
-    c.wt = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, phase_clock());
+    static_cast<Waiter&>(c.wt) = make_waiter(p.sink, lds + kLdsFlags + kFlagExpired, lds + kLdsTimers, phase_clock());
     c.wt.trace = trace_of(p.timers);
     const int32_t total = total_code_rows(p.lay) / kTaskRows * c.ng;
     // The kernel argument loads above complete here, before the loop: a load

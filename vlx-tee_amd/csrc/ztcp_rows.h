@@ -197,6 +197,15 @@ struct Waiter {
     uint32_t* tm;          // LDS phase-timer counters (timer builds)
     uint64_t t0;           // clock at which the wave left the first barrier (timer builds)
     uint32_t* trace;       // workgroup 0's row trace (timer builds), else nullptr
+    static constexpr bool kLateTag = false;
+};
+// A waiter whose call_tag goes to a vector register only where a wait expires:
+// the compiler otherwise moves that copy ahead of the egress producers' task
+// loop, which has no register to spare.  (Elsewhere it is left to the
+// compiler: in the one-page egress kernel the change of registers alone made
+// the hash chain 0.7 % slower, 909 -> 915 us.)
+struct LateTagWaiter : Waiter {
+    static constexpr bool kLateTag = true;
 };
 
 __device__ __forceinline__ Waiter make_waiter(const WaitSink& s, uint32_t* expired_lds, uint32_t* tm = nullptr,
@@ -206,8 +215,8 @@ __device__ __forceinline__ Waiter make_waiter(const WaitSink& s, uint32_t* expir
 
 // Records an expired wait: the device's and the call's diagnostics, and the
 // workgroup's LDS word.
-template <uint32_t DIAG>
-__device__ __forceinline__ void expire(const Waiter& w) {
+template <uint32_t DIAG, class W>
+__device__ __forceinline__ void expire(const W& w) {
     if ((threadIdx.x & 63) == 0) {
         atomicOr(w.dev_diag, DIAG);
         if (w.call_diag) {
@@ -215,7 +224,7 @@ __device__ __forceinline__ void expire(const Waiter& w) {
             // ingress calls or in their kernel's bit
             if constexpr (DIAG == kDiagEgressWait) {
                 uint32_t tag = w.call_tag;
-                asm volatile("" : "+s"(tag));  // moved to a vector register only here, not ahead of the task loop
+                if constexpr (W::kLateTag) asm volatile("" : "+s"(tag));
                 __hip_atomic_store(w.call_diag, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             } else {
                 atomicOr(w.call_diag, DIAG);
@@ -234,8 +243,8 @@ __device__ __forceinline__ void expire(const Waiter& w) {
 // next poll instead of spinning out its own bound, so a broken workgroup
 // ends about one bound after its first expiry.  TSLOT >= 0: timer builds add
 // the clocks spent here to that phase-timer slot.
-template <uint32_t DIAG, int TSLOT = -1>
-__device__ __forceinline__ void wait_ge(const uint32_t* flag, int32_t want, const Waiter& w) {
+template <uint32_t DIAG, int TSLOT = -1, class W>
+__device__ __forceinline__ void wait_ge(const uint32_t* flag, int32_t want, const W& w) {
     if ((int32_t)__hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= want) return;
     [[maybe_unused]] const uint64_t t_in = (kPhaseTimers && TSLOT >= 0) ? phase_clock() : 0;
     for (uint32_t spin = 0;; ++spin) {
@@ -252,8 +261,8 @@ __device__ __forceinline__ void wait_ge(const uint32_t* flag, int32_t want, cons
 
 // Waits until *f0 and *f1 are both >= want: the two counters are loaded
 // together, so a wait that is already satisfied costs one LDS latency.
-template <uint32_t DIAG, int TSLOT>
-__device__ __forceinline__ void wait_both_ge(const uint32_t* f0, const uint32_t* f1, int32_t want, const Waiter& w) {
+template <uint32_t DIAG, int TSLOT, class W>
+__device__ __forceinline__ void wait_both_ge(const uint32_t* f0, const uint32_t* f1, int32_t want, const W& w) {
     const uint32_t a = __hip_atomic_load(f0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     const uint32_t b = __hip_atomic_load(f1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     if ((int32_t)a >= want && (int32_t)b >= want) {
