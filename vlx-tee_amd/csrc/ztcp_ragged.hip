@@ -16,7 +16,7 @@
 // waits.  What lasts is the SipHash chain of a page, two lanes per page
 // (SipPair): a workgroup holds one page until every SIMD of the chip has one,
 // then more (ragged_pages); its hashing wave is another one of its four with
-// every workgroup per CU, so that those of one CU land on different
+// every workgroup per CU or so, and those of one CU land on different
 // SIMDs.  Against the layout-agnostic kernels (ztcp_generic.hip: one thread
 // per page and byte loads for the hash, byte arrays in scratch memory for the
 // blocks): 333 pages of 10,708 bytes egress 925 -> 115 us, 1,200 pages of
@@ -141,8 +141,12 @@ __device__ __forceinline__ void hash_page(SipPair& s, const uint64_t (&hdr)[4], 
     s.finish(last, lo, hi);
 }
 
-// The wave of the workgroup that hashes.
-__device__ __forceinline__ int hash_wave(int cu_count) { return (int)(blockIdx.x / (uint32_t)cu_count) & 3; }
+// The wave of the workgroup that hashes: another one with every 2^k
+// workgroups, 2^k <= CUs (a division by the CU count costs 1 % of a launch of
+// 333 pages).
+__device__ __forceinline__ int hash_wave(int cu_count) {
+    return (int)(blockIdx.x >> (31 - __builtin_clz((uint32_t)cu_count))) & 3;
+}
 
 template <int DT>
 __global__ __launch_bounds__(kRgThreads) void egress_ragged_kernel(EgressParams p) {
