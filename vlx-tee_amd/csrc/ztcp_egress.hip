@@ -734,8 +734,13 @@ struct RowStores {
     // The row in `slot` of every page to blob offset `dst`.
     __device__ __forceinline__ void store(const uint32_t* slot, uint32_t dst) const {
         uint4 x[4];
+        if (ng == 1) {  // no reads of pages that are not there: they take LDS time from the hash chain's
+            stg16(blob[0] + dst, 0, lds_quad_at(slot, off));
+            return;
+        }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) x[k] = lds_quad_at(slot + kTaskPages * 16 * k, off);
+        for (int k = 0; k < 4; ++k)
+            if (k < 2 || ng > 2) x[k] = lds_quad_at(slot + kTaskPages * 16 * k, off);
 #pragma unroll
         for (int k = 0; k < 4; ++k)
             if (k < ng) stg16(blob[k] + dst, 0, x[k]);
@@ -869,6 +874,10 @@ __global__ __launch_bounds__(64 * kEgressWaves) void egress_fused_kernel(EgressP
         egress_scale_feed(p, page_groups(ppw), lds);
     } else if ((wave & 3) == 0) {
         // the rest of the MAC wave's SIMD stays idle
+    } else if (FAM == 2 && wave > 12 && p.ppw <= kPairPages) {
+        // up to 32 pages the hash chain is the bound, and eight producers
+        // keep ahead of it with less LDS traffic in its way (8,192 pages of
+        // K8V4_ASYM_G64: 274 us with eleven, 270 with eight)
     } else if (wave == 1) {
         egress_store_rows(p, ppw, lds);
     } else {
